@@ -12,31 +12,39 @@
 // maps them through Moro's inverse normal, evolves the forward curve
 //   f(s, l) = f(s-1, l+1) + mu[l] dt + sqrt(dt) sum_k sigma_k[l] Z_k(s)
 // for every step, discounts along the short rate f(s, 0) and prices the swap
-// on the curve f(m, .) at the swaption's start m.  The payoff reads only the
-// short rates before m and the curve at m, so the kernel follows each forward
-// chain d (f(0,d) -> f(1,d-1) -> ...) through steps 1..min(d, m) only, with
-// the reference's additions in the reference's order, and takes the swap
-// curve's exponentials only up to the swap's last cash flow (past it the
-// reference multiplies its discount factors by zero cash flows; a guard sends
-// any path where those factors could be non-finite through the full
-// computation).  The prices are the reference's up to the device exp/log
-// (last-bit differences) and the order of the final sums.  With the reference's parameters (11 steps, maturity 1
-// year on a 5-20 year horizon) m is 1 or 2 of the 10 steps.
+// on the curve f(m, .) at the swaption's start m.
+//
+// Every exponent of that payoff is linear in the path's draws: the payoff
+// reads the short rates before m and the curve at m, the model is Gaussian,
+// and a discount factor is the exponential of a sum of rates.  So a path of
+// k_sw_paths is
+//   max(sum_c pay_c 2^(C_c + sum_j G_cj Z_j) - 1, 0) 2^(C_0 + sum_j G_0j Z_j)
+// over the m F draws Z_j before the start and the swap's cash flows c (the
+// reference multiplies the discount factors between them by zero), with C and
+// G formed once per swaption on the host: one FMA per draw and cash flow and
+// one exponential per cash flow, where the recursion takes them per curve
+// point and step.  It holds wherever the reference's running products neither
+// overflow nor underflow (pack_linear bounds them) and every draw is finite
+// (a counter that is a multiple of 2^31-1 draws u = 0, whose normal is
+// infinite); blocks of paths where it may not hold are left to
+// k_sw_paths_steps, which follows the reference statement by statement.  The
+// prices are the reference's up to rounding: measured against the oracle's
+// restatement, 1e-15 relative.
 //
 // Generator: the reference's RanUnif (PARSEC 3.0 RanUnif.cpp, not in the
 // reference tree) is the Park-Miller minimal standard generator applied to
-// 1513517 c mod (2^31-1); both products are reduced here with the Mersenne
-// identity 2^31 = 1 (mod 2^31-1) in 64-bit integers, which gives the same
-// residues as its Schrage factorisation.
+// 1513517 c mod (2^31-1).  Both products together are A c mod (2^31-1) with
+// A = 16807 * 1513517, the same residues as its Schrage factorisation, so the
+// residue of the next counter is one 32-bit addition away.
 //
-// Kernels (the caller's stream): k_sw_paths, one path at a time per work-item,
-// kSwPer paths each, Moro's tail evaluated for a whole wave's draws at once
-// (draws_compact), each block's sums of payoff and payoff^2 folded in a fixed
-// order into one partial; k_sw_final, one block per swaption, adds its
-// partials in a fixed order and forms the mean and standard error as the
-// reference does.  Results are bit-reproducible for given inputs.  The
-// arithmetic is FP64 (the reference's FTYPE); this file is compiled without
-// FMA contraction so every product and sum rounds as the reference's do.
+// Kernels (the caller's stream): k_sw_paths, 4 to 16 paths per work-item, and,
+// where it left blocks out, k_sw_paths_steps, each block's sums of payoff and
+// payoff^2 folded in a fixed order into one partial; k_sw_final, one block per
+// swaption, adds its partials in a fixed order and forms the mean and standard
+// error as the reference does.  Results are bit-reproducible for given inputs.
+// The arithmetic is FP64 (the reference's FTYPE); this file is compiled
+// without FMA contraction, so the step-by-step kernel rounds every product and
+// sum as the reference does and the other one's FMAs are the ones written.
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -52,25 +60,30 @@ namespace bs {
 namespace {
 
 constexpr int kSwThreads = 256;
-constexpr int kSwPer = 4;                 // paths per work-item
+constexpr int kSwRows = 4;                // fewest paths per work-item
 constexpr int kSwMaxSteps = 64;           // n_steps
 constexpr int kSwMaxFactors = 8;          // n_factors
 constexpr int kSwMaxDraws = 64;           // start index x n_factors
-constexpr int kSwCompactDraws = 12;       // register forms up to this many draws compact Moro's tail
 constexpr int64_t kSwCounterLimit = int64_t(1) << 42;
 constexpr uint64_t kM31 = 2147483647u;
 
-// One swaption as the kernel reads it.  pool + off holds f0[n] (the forward
+// How a launch's blocks cover the paths: block b takes swaption b / bps, its
+// paths [(b % bps) kSwThreads rows, + kSwThreads rows), `rows` of them per
+// work-item, kSwThreads apart.
+struct SwGrid {
+    int64_t paths;
+    int32_t bps, rows;
+};
+
+// One swaption as the step-by-step kernel reads it.  pool + off holds f0[n] (the forward
 // curve at t = 0), mudt[n-1] (total drift x dt), sigma[F][n-1] and pay[L]
 // (the swap's cash flows per unit notional).
 struct SwHead {
     int64_t seed;        // counter of path 0's first draw
     double dt, sdt, dts; // HJM step, its square root, the swap curve's step
     int32_t n, m, L, off;
-    int32_t last;        // index of the swap's last cash flow (pay[l] = 0 past it)
-    int32_t pad;
 };
-static_assert(sizeof(SwHead) == 56, "SwHead layout");
+static_assert(sizeof(SwHead) == 48, "SwHead layout");
 
 __device__ __forceinline__ uint64_t mod_m31(uint64_t x) {   // x < 2^63
     x = (x & kM31) + (x >> 31);
@@ -115,91 +128,32 @@ __device__ __forceinline__ double moro_inv(double u) {
 
 // The normal draws of path p: z[s][k] = Z_k(s + 1) for s < m.
 template <int F, int MAXM>
-__device__ __forceinline__ void draws_direct(const SwHead& h, int64_t p, double (&z)[MAXM][F]) {
+__device__ __forceinline__ void draws(const SwHead& h, int64_t p, double (&z)[MAXM][F]) {
     const int64_t c0 = h.seed + p * (int64_t)((h.n - 1) * F);
-#pragma unroll
-    for (int s = 0; s < MAXM; ++s) {
-        if (s >= h.m) break;
+    for (int s = 0; s < h.m; ++s) {
 #pragma unroll
         for (int k = 0; k < F; ++k) z[s][k] = moro_inv(ran_unif(c0 + s * F + k));
     }
 }
 
-// The same draws, with Moro's tail (16% of draws, but taken by nearly every
-// wave at every draw when each lane branches on its own) compacted: the lanes
-// write the uniforms that need it to their wave's LDS list (ballot + mbcnt),
-// every lane then evaluates the tail for list entries lane, lane + 64, ...,
-// and each owner reads its results back.  The same operations on the same
-// values as draws_direct.  Every thread of the block must call it (it
-// synchronises the block); wl is this wave's MAXM F 64 doubles.
+// Discounted payoff of a path from its draws z, the reference's arithmetic
+// statement by statement: each forward chain d (f(0,d) -> f(1,d-1) -> ...)
+// takes the steps 1..min(d, m) that the payoff reads, with the reference's
+// additions in the reference's order.
 template <int F, int MAXM>
-__device__ __forceinline__ void draws_compact(const SwHead& h, int64_t p, double (&z)[MAXM][F],
-                                              double* wl) {
-    const int64_t c0 = h.seed + p * (int64_t)((h.n - 1) * F);
-    const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-    int pos[MAXM][F];
-    bool tail[MAXM][F];
-    int count = 0;   // tail entries of this wave so far (uniform)
-#pragma unroll
-    for (int s = 0; s < MAXM; ++s) {
-        const bool live = s < h.m;   // uniform
-#pragma unroll
-        for (int k = 0; k < F; ++k) {
-            const double u = live ? ran_unif(c0 + s * F + k) : 0.25;
-            const double x = u - 0.5;
-            const bool t = !(fabs(x) < 0.42);
-            z[s][k] = moro_central(x);
-            const uint64_t b = __ballot(t);
-            pos[s][k] = count + (int)__builtin_amdgcn_mbcnt_hi(
-                                    (uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
-            tail[s][k] = t;
-            if (t) wl[pos[s][k]] = u;
-            count += __popcll(b);
-        }
-    }
-    __syncthreads();
-    for (int r = 0; r < count; r += 64) {
-        const int i = r + lane;
-        if (i < count) wl[i] = moro_tail(wl[i]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int s = 0; s < MAXM; ++s)
-#pragma unroll
-        for (int k = 0; k < F; ++k)
-            if (tail[s][k]) z[s][k] = wl[pos[s][k]];
-    __syncthreads();   // the list is rewritten for the next path
-}
-
-// Discounted payoff of a path from its draws z.  F factors; the swaption
-// starts at step m <= MAXM.
-//
-// kAll = true is the reference's arithmetic in full.  kAll = false skips the
-// swap-curve exponentials past the last cash flow: those discount factors
-// only ever multiply pay[l] = 0, so the terms they make are +0 and leave the
-// fixed leg unchanged -- provided every one of them is finite.  That holds
-// when the rates past the last cash flow are finite, the discount factor at
-// the last cash flow is at most 1e300 and the positive exponents past it sum
-// to at most 1 (the factors then stay below 1e300 e); *exact reports it, and
-// the caller recomputes the path with kAll = true when it does not hold.
-template <int F, int MAXM, bool kAll>
 __device__ __forceinline__ double path_payoff(const SwHead& h, const double* __restrict__ q,
-                                              const double (&z)[MAXM][F], bool* exact) {
+                                              const double (&z)[MAXM][F]) {
     const int n = h.n, m = h.m, L = h.L, w = n - 1;
-    const int last = kAll ? L : h.last;
     const double* f0 = q;
     const double* mudt = q + n;
     const double* sigma = q + n + w;
     const double* pay = q + n + w + F * w;
-    double df = 1.0, sdf = 1.0, leg = 0.0, grow = 0.0;
-    bool finite = true;
+    double df = 1.0, sdf = 1.0, leg = 0.0;
     const int dend = min(n, m + L);
     for (int d = 0; d < dend; ++d) {
         double x = f0[d];
         const int steps = min(d, m);
-#pragma unroll
-        for (int s = 1; s <= MAXM; ++s) {
-            if (s > steps) break;
+        for (int s = 1; s <= steps; ++s) {
             const int l = d - s;
             double shock = 0.0;
 #pragma unroll
@@ -210,63 +164,384 @@ __device__ __forceinline__ double path_payoff(const SwHead& h, const double* __r
             df *= exp(-x * h.dt);
         } else {
             const int l = d - m;
-            if (l <= last) leg += pay[l] * sdf;
-            if (l < L - 1) {
-                const double y = -x * h.dts;
-                if (l < last) {
-                    sdf *= exp(y);
-                } else {
-                    finite = finite && fabs(y) <= 1e300;   // false for inf and NaN
-                    grow += y > 0 ? y : 0;
-                }
-            }
+            leg += pay[l] * sdf;
+            if (l < L - 1) sdf *= exp(-x * h.dts);
         }
     }
     // curve points past the simulated horizon are zero rates: factor exp(-0) = 1
-    for (int l = n - m; l < L; ++l)
-        if (l <= last) leg += pay[l] * sdf;
-    *exact = kAll || (finite && grow <= 1.0 && sdf <= 1e300);
+    for (int l = n - m; l < L; ++l) leg += pay[l] * sdf;
     const double payoff = leg - 1.0 > 0 ? leg - 1.0 : 0;
     return payoff * df;
 }
 
-// Block b covers swaption b / bps, paths [(b % bps) kSwThreads kSwPer, +kSwThreads kSwPer).
-// The compacted forms hold the draws, their list slots and the payoff state at
-// once; up to 6 draws per path, asking for 6 waves per SIMD keeps them within
-// 80 VGPRs without spilling (the reference's shape: 79).
-template <int F, int MAXM>
-__global__ __launch_bounds__(kSwThreads)
-__attribute__((amdgpu_waves_per_eu(MAXM * F <= 6 ? 6 : 1))) void k_sw_paths(const SwHead* __restrict__ heads,
-                                                         const double* __restrict__ pool, int bps,
-                                                         int64_t paths,
-                                                         double* __restrict__ partial) {
-    const int sw = (int)(blockIdx.x / (unsigned)bps);
-    const int64_t chunk = blockIdx.x % (unsigned)bps;
-    const SwHead h = heads[sw];
-    const double* q = pool + h.off;
-    constexpr bool kCompact = MAXM * F <= kSwCompactDraws;
-    __shared__ double lds_tail[kCompact ? kSwThreads / 64 : 1][kCompact ? MAXM * F * 64 : 1];
-    double sum = 0.0, sumsq = 0.0;
-#pragma unroll 1
-    for (int j = 0; j < kSwPer; ++j) {
-        const int64_t p = (chunk * kSwPer + j) * kSwThreads + threadIdx.x;
-        const bool valid = p < paths;
-        double z[MAXM][F];
-        if constexpr (kCompact) {
-            // every work-item takes part (the draws synchronise the block);
-            // past the last path it draws for the last one and discards them
-            draws_compact<F, MAXM>(h, valid ? p : paths - 1, z, lds_tail[threadIdx.x / 64]);
-        } else {
-            if (valid) draws_direct<F, MAXM>(h, p, z);
-        }
-        if (valid) {
-            bool exact;
-            double v = path_payoff<F, MAXM, false>(h, q, z, &exact);
-            if (!exact) v = path_payoff<F, MAXM, true>(h, q, z, &exact);
-            sum += v;
-            sumsq += v * v;
+// ---- the linear form --------------------------------------------------------------
+// One swaption as k_sw_paths reads it; pool + off holds, for W = the width of
+// its form (lin_width: at least `flows`, padded with zeros), C[W], pay[W],
+// G[draws][W] and Gdf[draws].  Exponents are in base 2.
+struct SwLin {
+    int64_t seed;        // counter of path 0's first draw
+    double c_df;         // C of the discount to the swaption's start
+    uint32_t per_path;   // counters a path takes, (n-1) F
+    uint32_t x_path;     // A per_path mod M: residue step to the next path
+    uint32_t x_row;      // A kSwThreads per_path mod M: to a work-item's next path
+    int32_t draws;       // m F, those the payoff reads
+    int32_t df_draws;    // (m-1) F, those the discount to the start reads
+    int32_t flows;       // cash flows
+    int32_t off;
+    int32_t linear;      // 0: every block is left to k_sw_paths_steps
+};
+static_assert(sizeof(SwLin) == 48, "SwLin layout");
+
+constexpr uint32_t kGenA = (uint32_t)(uint64_t(16807) * 1513517u % kM31);
+constexpr uint32_t gen_step(uint64_t counters) {
+    return (uint32_t)(counters % kM31 * kGenA % kM31);
+}
+
+// a + b mod M for residues a, b < M = 2^31-1.
+__device__ __forceinline__ uint32_t add_m31(uint32_t a, uint32_t b) {
+    const uint32_t t = a + b;
+    return min(t, t - (uint32_t)kM31);   // t < M: t - M wraps past it
+}
+
+// Residues whose uniform |u - 0.5| >= 0.42 takes Moro's tail: x <= kTailLo or
+// x >= kTailHi, u rounded as in ran_unif.
+constexpr bool in_tail(uint32_t x) {
+    const double d = (double)x * 4.656612875e-10 - 0.5;
+    return !((d < 0 ? -d : d) < 0.42);
+}
+constexpr uint32_t tail_edge(bool upper) {
+    uint32_t a = upper ? (uint32_t)kM31 / 2 : 0, b = upper ? (uint32_t)kM31 - 1 : (uint32_t)kM31 / 2;
+    while (b - a > 1) {   // upper: b is in the tail and a is not; lower: a is and b is not
+        const uint32_t c = a + (b - a) / 2;
+        if (in_tail(c) == upper) b = c;
+        else a = c;
+    }
+    return upper ? b : a;
+}
+constexpr uint32_t kTailLo = tail_edge(false), kTailHi = tail_edge(true);
+static_assert(in_tail(kTailLo) && !in_tail(kTailLo + 1) && in_tail(kTailHi) &&
+                  !in_tail(kTailHi - 1) && in_tail(0) && in_tail((uint32_t)kM31 - 1),
+              "tail residues");
+
+// a / b for b in [0.007, 4]: with e = 1 - b y the error of v_rcp_f64's y (at
+// most 2^-24.3 there, measured), a y (1 + e + e^2), within an ulp of a / b.
+__device__ __forceinline__ double div_near1(double a, double b) {
+    const double y = __builtin_amdgcn_rcp(b);
+    const double e = __builtin_fma(-b, y, 1.0);
+    const double q = a * y;
+    return __builtin_fma(q, __builtin_fma(e, e, e), q);
+}
+
+// log(x) of a positive normal x: x = 2^e m, m in [sqrt(1/2), sqrt(2)) (the
+// exponent field counted from the high word of sqrt(1/2)), s = (m - 1) / (m + 1),
+// log m = 2 atanh(s) with (2 atanh(s) / s - 2) / s^2 interpolated at Chebyshev
+// nodes in s^2 (degree 6, relative error 5e-18).
+__device__ __forceinline__ double log_pos(double x) {
+    constexpr uint32_t kRootHalf = 0x3fe6a09eu;
+    const uint32_t b = (uint32_t)__double2hiint(x) - kRootHalf;
+    const int e = (int)b >> 20;
+    const double m = __hiloint2double((int)((b & 0xfffffu) + kRootHalf), __double2loint(x));
+    const double f = m - 1.0;
+    const double s = div_near1(f, m + 1.0);
+    const double z = s * s;
+    double p = 0.14616449685043406;
+    p = __builtin_fma(p, z, 0.15331721600556042);
+    p = __builtin_fma(p, z, 0.18182889125261723);
+    p = __builtin_fma(p, z, 0.2222221113479508);
+    p = __builtin_fma(p, z, 0.28571428625975487);
+    p = __builtin_fma(p, z, 0.39999999999899505);
+    p = __builtin_fma(p, z, 0.666666666666667);
+    const double h = 0.5 * (f * f);
+    const double lm = f + __builtin_fma(s, __builtin_fma(z, p, h), -h);
+    const double ed = (double)e;
+    // ln 2 in two parts, the first with 32 significant bits
+    return __builtin_fma(ed, 0.6931471803691238, __builtin_fma(ed, 1.9082149292705877e-10, lm));
+}
+
+// 2^x for |x| < 1000: (2^f - 1) / f interpolated at Chebyshev nodes over
+// |f| <= 1/2 (degree 10, relative error of 2^f 2e-17 with rounded
+// coefficients).
+__device__ __forceinline__ double exp2_mid(double x) {
+    const double k = __builtin_rint(x);
+    const double f = x - k;
+    double p = 4.4549605981865186e-10;
+    p = __builtin_fma(p, f, 7.072585949269223e-09);
+    p = __builtin_fma(p, f, 1.0178062445845774e-07);
+    p = __builtin_fma(p, f, 1.321544258792169e-06);
+    p = __builtin_fma(p, f, 1.525273382983612e-05);
+    p = __builtin_fma(p, f, 0.0001540353044173605);
+    p = __builtin_fma(p, f, 0.0013333558146416936);
+    p = __builtin_fma(p, f, 0.009618129107606888);
+    p = __builtin_fma(p, f, 0.0555041086648216);
+    p = __builtin_fma(p, f, 0.24022650695910097);
+    p = __builtin_fma(p, f, 0.6931471805599453);
+    p = __builtin_fma(p, f, 1.0);
+    return __builtin_amdgcn_ldexp(p, (int)k);
+}
+
+// A constant held in a vector register from here on.  An FP64 instruction reads
+// one scalar operand at most and there are not enough scalar registers for
+// every constant of k_sw_paths, so the compiler otherwise builds the central
+// branch's constants anew for every draw, 6 of its 23 instructions.
+__device__ __forceinline__ double pinned(double c) {
+    asm("" : "+v"(c));
+    return c;
+}
+
+// Moro's two branches (moro_central, moro_tail) with FMAs.
+struct MoroCentral {
+    double scale = pinned(4.656612875e-10);
+    double a1 = pinned(-25.44106049637), a2 = pinned(41.39119773534),
+           a3 = pinned(-18.61500062529), a4 = pinned(2.50662823884);
+    double b1 = pinned(3.13082909833), b2 = pinned(-21.06224101826),
+           b3 = pinned(23.08336743743), b4 = pinned(-8.47351093090);
+    // The normal of residue x's uniform, for the residues outside the tail.
+    __device__ __forceinline__ double operator()(uint32_t residue) const {
+        const double x = __builtin_fma((double)residue, scale, -0.5);
+        const double r = x * x;
+        double num = __builtin_fma(r, a1, a2);
+        num = __builtin_fma(r, num, a3);
+        num = __builtin_fma(r, num, a4);
+        double den = __builtin_fma(r, b1, b2);
+        den = __builtin_fma(r, den, b3);
+        den = __builtin_fma(r, den, b4);
+        den = __builtin_fma(r, den, 1.0);   // 0.11 <= den <= 1 for |x| <= 0.42
+        return div_near1(x * num, den);
+    }
+};
+
+// The normal of a nonzero residue in the tail: log(-log(min(u, 1 - u))).
+__device__ __forceinline__ double moro_tail_fma(uint32_t residue) {
+    const bool upper = residue > (uint32_t)kM31 / 2;
+    const double w = __builtin_fma((double)residue, upper ? -4.656612875e-10 : 4.656612875e-10,
+                                   upper ? 1.0 : 0.0);
+    const double t = log_pos(-log_pos(w));
+    double v = __builtin_fma(t, 0.0000003960315187, 0.0000002888167364);
+    v = __builtin_fma(t, v, 0.0000321767881768);
+    v = __builtin_fma(t, v, 0.0003951896511919);
+    v = __builtin_fma(t, v, 0.0038405729373609);
+    v = __builtin_fma(t, v, 0.0276438810333863);
+    v = __builtin_fma(t, v, 0.1607979714918209);
+    v = __builtin_fma(t, v, 0.9761690190917186);
+    v = __builtin_fma(t, v, 0.3374754822726147);
+    return upper ? v : -v;
+}
+
+// Whether the linear form takes the paths of block `chunk` of a swaption: it is
+// bounded and no counter of the block draws u = 0.
+__device__ __forceinline__ bool block_linear(const SwLin& h, const SwGrid& grid, int64_t chunk) {
+    const uint64_t span = (uint64_t)(kSwThreads * grid.rows) * h.per_path;
+    const uint64_t r = mod_m31((uint64_t)h.seed + (uint64_t)chunk * span);
+    return h.linear && r != 0 && r + span <= kM31;
+}
+
+// Keeps the compiler from moving the lanes' accesses to their wave's LDS list
+// across this point; the hardware performs a wave's LDS accesses in order.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The h.draws <= DB draws of PP paths, added into the paths' exponents.  FULL:
+// h.draws = DB.  xs holds each path's residue at its first draw.
+//
+// Moro's tail (16% of draws, but taken by nearly every wave at every draw when
+// each lane branches on its own) is compacted over the batch: the lanes write
+// the residues that need it to their wave's LDS list (ballot and mbcnt give
+// the places), all lanes evaluate the list, and each owner reads its results
+// back.  PP DB = 12 draws make 123 list entries a batch on average, so the
+// last of its rounds of 64 wastes little.
+template <int W, int PP, int DB, bool FULL>
+__device__ __forceinline__ void linear_batch(const SwLin& h, const double* __restrict__ G,
+                                             const double* __restrict__ gdf,
+                                             const uint32_t (&xs)[PP], char* lds, uint32_t wl,
+                                             const MoroCentral& central,
+                                             double (&acc)[PP][W], double (&dfe)[PP]) {
+    const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    double z[PP][DB];
+    bool tail[PP][DB];
+    uint32_t at[PP][DB];   // a tail draw's list entry (its offset in lds)
+    int count = 0;       // the wave's list so far (uniform)
+#pragma unroll
+    for (int j = 0; j < DB; ++j) {
+        if (FULL || j < h.draws) {
+#pragma unroll
+            for (int p = 0; p < PP; ++p) {
+                const uint32_t x = add_m31(xs[p], gen_step(j));
+                z[p][j] = central(x);
+                tail[p][j] = x - (kTailLo + 1) >= kTailHi - (kTailLo + 1);
+                const uint64_t b = __ballot(tail[p][j]);
+                at[p][j] = (wl + 8 * (uint32_t)count) +
+                           8 * __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
+                if (tail[p][j]) *reinterpret_cast<uint32_t*>(lds + at[p][j]) = x;
+                count += __popcll(b);
+            }
         }
     }
+    wave_lds_order();
+    for (int r = 0; r < count; r += 64) {
+        const int i = r + lane;
+        if (i < count) {
+            const uint32_t e = wl + 8 * (uint32_t)i;
+            *reinterpret_cast<double*>(lds + e) = moro_tail_fma(
+                *reinterpret_cast<const uint32_t*>(lds + e));
+        }
+    }
+    wave_lds_order();
+#pragma unroll
+    for (int j = 0; j < DB; ++j) {
+        if (FULL || j < h.draws) {
+            const double* __restrict__ g = G + j * W;
+#pragma unroll
+            for (int p = 0; p < PP; ++p)
+                if (tail[p][j]) z[p][j] = *reinterpret_cast<const double*>(lds + at[p][j]);
+#pragma unroll
+            for (int c = 0; c < W; ++c)
+#pragma unroll
+                for (int p = 0; p < PP; ++p)
+                    acc[p][c] = __builtin_fma(g[c], z[p][j], acc[p][c]);
+            if (j < h.df_draws) {
+#pragma unroll
+                for (int p = 0; p < PP; ++p)
+                    dfe[p] = __builtin_fma(gdf[j], z[p][j], dfe[p]);
+            }
+        }
+    }
+    wave_lds_order();   // the list is rewritten by the next batch
+}
+
+// The paths of a work-item, PP at a time.
+template <int W, int PP, int DB>
+__device__ __forceinline__ void linear_paths(const SwLin& h, const double* __restrict__ q,
+                                             uint32_t xb, int64_t p0, const SwGrid& grid,
+                                             char* lds, uint32_t wl,
+                                             double* sum, double* sumsq) {
+    const double* __restrict__ pay = q + W;
+    const double* __restrict__ G = q + 2 * W;
+    const double* __restrict__ gdf = G + h.draws * W;
+    const double df0 = exp2_mid(h.c_df);
+    const MoroCentral central;
+#pragma unroll 1
+    for (int row = 0; row < grid.rows; row += PP) {
+        double acc[PP][W], dfe[PP];
+        uint32_t xs[PP];
+#pragma unroll
+        for (int p = 0; p < PP; ++p) {
+#pragma unroll
+            for (int c = 0; c < W; ++c) acc[p][c] = q[c];
+            dfe[p] = h.c_df;
+            xs[p] = xb;
+            xb = add_m31(xb, h.x_row);
+        }
+        if (h.draws == DB)
+            linear_batch<W, PP, DB, true>(h, G, gdf, xs, lds, wl, central, acc, dfe);
+        else
+            linear_batch<W, PP, DB, false>(h, G, gdf, xs, lds, wl, central, acc, dfe);
+        double leg[PP];
+#pragma unroll
+        for (int p = 0; p < PP; ++p) leg[p] = -1.0;
+#pragma unroll
+        for (int c = 0; c < W; ++c)
+#pragma unroll
+            for (int p = 0; p < PP; ++p)
+                leg[p] = __builtin_fma(pay[c], exp2_mid(acc[p][c]), leg[p]);
+        double df[PP];
+#pragma unroll
+        for (int p = 0; p < PP; ++p) df[p] = df0;
+        if (h.df_draws > 0) {
+#pragma unroll
+            for (int p = 0; p < PP; ++p) df[p] = exp2_mid(dfe[p]);
+        }
+#pragma unroll
+        for (int p = 0; p < PP; ++p) {
+            double v = (leg[p] > 0 ? leg[p] : 0) * df[p];
+            v = p0 + (row + p) * kSwThreads < grid.paths ? v : 0.0;
+            *sum += v;
+            *sumsq = __builtin_fma(v, v, *sumsq);
+        }
+    }
+}
+
+// The paths of a work-item one at a time, for many draws or cash flows: only
+// the W exponents stay in registers.  The draws of a batch live in LDS, slot
+// j 64 + lane: a central draw's normal, or a tail draw's residue until the
+// compacted evaluation (as in linear_batch, over a list of slots) replaces it.
+constexpr int kWideDraws = 12;   // draws in a batch
+constexpr uint32_t kWideBytes = kWideDraws * 64 * (8 + 2);   // a wave's slots and list
+
+template <int W>
+__device__ __forceinline__ void linear_wide(const SwLin& h, const double* __restrict__ q,
+                                            uint32_t xb, int64_t p0, const SwGrid& grid,
+                                            char* lds, double* sum, double* sumsq) {
+    const double* __restrict__ pay = q + W;
+    const double* __restrict__ G = q + 2 * W;
+    const double* __restrict__ gdf = G + h.draws * W;
+    const double df0 = exp2_mid(h.c_df);
+    const MoroCentral central;
+    const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    char* slots = lds + wave * kWideBytes;
+    uint16_t* list = reinterpret_cast<uint16_t*>(slots + kWideDraws * 64 * 8);
+    char* mine = slots + lane * 8;
+#pragma unroll 1
+    for (int row = 0; row < grid.rows; ++row) {
+        double acc[W], dfe = h.c_df;
+#pragma unroll
+        for (int c = 0; c < W; ++c) acc[c] = q[c];
+        uint32_t x = xb;
+        xb = add_m31(xb, h.x_row);
+#pragma unroll 1
+        for (int j0 = 0; j0 < h.draws; j0 += kWideDraws) {
+            const int nj = min(kWideDraws, h.draws - j0);
+            int count = 0;
+#pragma unroll 2
+            for (int j = 0; j < nj; ++j) {
+                const bool tail = x - (kTailLo + 1) >= kTailHi - (kTailLo + 1);
+                const uint64_t b = __ballot(tail);
+                *reinterpret_cast<double*>(mine + j * 512) = central(x);
+                if (tail) {
+                    const uint32_t at = __builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
+                    *reinterpret_cast<uint32_t*>(mine + j * 512) = x;
+                    list[count + at] = (uint16_t)(j * 512 + lane * 8);
+                }
+                count += __popcll(b);
+                x = add_m31(x, gen_step(1));
+            }
+            wave_lds_order();
+            for (int r = 0; r < count; r += 64) {
+                if (r + lane < count) {
+                    char* slot = slots + list[r + lane];
+                    *reinterpret_cast<double*>(slot) = moro_tail_fma(
+                        *reinterpret_cast<const uint32_t*>(slot));
+                }
+            }
+            wave_lds_order();
+            const double* __restrict__ g = G + j0 * W;
+#pragma unroll 2
+            for (int j = 0; j < nj; ++j, g += W) {
+                const double z = *reinterpret_cast<const double*>(mine + j * 512);
+#pragma unroll
+                for (int c = 0; c < W; ++c) acc[c] = __builtin_fma(g[c], z, acc[c]);
+                if (j0 + j < h.df_draws) dfe = __builtin_fma(gdf[j0 + j], z, dfe);
+            }
+            wave_lds_order();   // the slots are rewritten by the next batch
+        }
+        double leg = -1.0;
+#pragma unroll
+        for (int c = 0; c < W; ++c)
+            if (c < h.flows) leg = __builtin_fma(pay[c], exp2_mid(acc[c]), leg);
+        double v = (leg > 0 ? leg : 0) * (h.df_draws > 0 ? exp2_mid(dfe) : df0);
+        v = p0 + row * kSwThreads < grid.paths ? v : 0.0;
+        *sum += v;
+        *sumsq = __builtin_fma(v, v, *sumsq);
+    }
+}
+
+// A block's sums of payoff and payoff^2, in a fixed order.
+__device__ __forceinline__ void block_partial(double sum, double sumsq, double* partial) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
         sum += __shfl_xor(sum, o, 64);
@@ -288,6 +563,111 @@ __attribute__((amdgpu_waves_per_eu(MAXM * F <= 6 ? 6 : 1))) void k_sw_paths(cons
         partial[2 * (int64_t)blockIdx.x] = a;
         partial[2 * (int64_t)blockIdx.x + 1] = b;
     }
+}
+
+constexpr int kSwBatch = 12;   // draws of a work-item in one batch of the narrow form
+
+// Widths of the linear form's accumulators: the smallest that holds the cash
+// flows.  A launch's kernel holds the forms up to the widest of its swaptions
+// and each block takes its swaption's own.
+constexpr int kLinWidths[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+constexpr int lin_width(int flows) {
+    for (int w : kLinWidths)
+        if (flows <= w) return w;
+    return 0;
+}
+
+// Few draws and cash flows (the reference driver's swaptions have 3 or 6 and 1
+// to 3): several paths at a time in registers.  Otherwise the wide form.
+template <int W>
+__device__ __forceinline__ void linear_form(const SwLin& h, const double* __restrict__ q,
+                                            uint32_t xb, int64_t p0, const SwGrid& grid,
+                                            char* lds, double* sum, double* sumsq) {
+    if constexpr (W <= 4) {
+        const uint32_t wl = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / 64) *
+                            (kSwBatch * 64 * 8);
+        if (h.draws <= 3) return linear_paths<W, 4, 3>(h, q, xb, p0, grid, lds, wl, sum, sumsq);
+        if (h.draws <= 6) return linear_paths<W, 2, 6>(h, q, xb, p0, grid, lds, wl, sum, sumsq);
+    }
+    linear_wide<W>(h, q, xb, p0, grid, lds, sum, sumsq);
+}
+
+// Bound by FP64 issue (parameters and partial sums are all it reads and
+// writes): PARSEC's native run, 128 swaptions x 1M trials with 3 or 6 draws and
+// 1 to 3 cash flows, takes 0.80 ms at 200 VALU instructions per path, and
+// took 3.31 ms at 928 in the form that followed the forward-rate chains (a
+// 64-bit generator, 6 draws for every swaption, an exponential per curve
+// point); 32 swaptions x 50,000 trials with 4-40 draws 0.09 ms and 0.76 ms.
+// With 3 or 5 waves per SIMD in place of 4 the times are the same.
+template <int MAXW>
+__global__ __launch_bounds__(kSwThreads)
+__attribute__((amdgpu_waves_per_eu(MAXW <= 8 ? 4 : MAXW <= 32 ? 3 : 2))) void k_sw_paths(
+    const SwLin* __restrict__ heads, const double* __restrict__ pool, SwGrid grid,
+    double* __restrict__ partial) {
+    __shared__ __align__(8) char lds[kSwThreads / 64 * kWideBytes];
+    static_assert(kSwThreads * kSwBatch * 8 <= sizeof lds, "the narrow form's lists");
+    const int sw = (int)(blockIdx.x / (unsigned)grid.bps);
+    const int64_t chunk = blockIdx.x % (unsigned)grid.bps;
+    const SwLin h = heads[sw];
+    if (!block_linear(h, grid, chunk)) return;
+    const double* q = pool + h.off;
+    const int64_t first = chunk * (kSwThreads * grid.rows);
+    // residue of this work-item's first draw: the block's (uniform) and the
+    // work-item's path, A (seed + (first + t) per_path)
+    const uint64_t xu = mod_m31(mod_m31((uint64_t)h.seed + (uint64_t)first * h.per_path) * kGenA);
+    const uint32_t xb = add_m31((uint32_t)xu, (uint32_t)mod_m31((uint64_t)h.x_path * threadIdx.x));
+    const int64_t p0 = first + threadIdx.x;
+    double sum = 0.0, sumsq = 0.0;
+    const int W = h.flows;
+    if (W <= 1) linear_form<1>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+    if (W == 2) linear_form<2>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+    if constexpr (MAXW >= 4) {
+        if (W == 3) linear_form<3>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W == 4) linear_form<4>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+    }
+    if constexpr (MAXW >= 8) {
+        if (W > 4 && W <= 6) linear_form<6>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W > 6 && W <= 8) linear_form<8>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+    }
+    if constexpr (MAXW >= 16) {
+        if (W > 8 && W <= 12) linear_form<12>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W > 12 && W <= 16) linear_form<16>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+    }
+    if constexpr (MAXW >= 32) {
+        if (W > 16 && W <= 24) linear_form<24>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W > 24 && W <= 32) linear_form<32>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+    }
+    if constexpr (MAXW >= 64) {
+        if (W > 32 && W <= 48) linear_form<48>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W > 48) linear_form<64>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+    }
+    block_partial(sum, sumsq, partial);
+}
+
+// The blocks that k_sw_paths left out, one path at a time per work-item (the
+// draws live in scratch).
+template <int F, int MAXM>
+__global__ __launch_bounds__(kSwThreads) void k_sw_paths_steps(
+    const SwLin* __restrict__ lin, const SwHead* __restrict__ heads,
+    const double* __restrict__ pool, SwGrid grid, double* __restrict__ partial) {
+    const int sw = (int)(blockIdx.x / (unsigned)grid.bps);
+    const int64_t chunk = blockIdx.x % (unsigned)grid.bps;
+    if (block_linear(lin[sw], grid, chunk)) return;
+    const SwHead h = heads[sw];
+    const double* q = pool + h.off;
+    double sum = 0.0, sumsq = 0.0;
+#pragma unroll 1
+    for (int j = 0; j < grid.rows; ++j) {
+        const int64_t p = (chunk * grid.rows + j) * kSwThreads + threadIdx.x;
+        if (p < grid.paths) {
+            double z[MAXM][F];
+            draws<F, MAXM>(h, p, z);
+            const double v = path_payoff<F, MAXM>(h, q, z);
+            sum += v;
+            sumsq += v * v;
+        }
+    }
+    block_partial(sum, sumsq, partial);
 }
 
 // Block i adds swaption i's bps partials (work-item t takes t, t + 256, ...
@@ -321,37 +701,34 @@ __global__ __launch_bounds__(kSwThreads) void k_sw_final(const double* __restric
     }
 }
 
-template <int F, int MAXM>
-void launch_paths(unsigned blocks, hipStream_t st, const SwHead* heads, const double* pool,
-                  int bps, int64_t paths, double* partial) {
-    hipLaunchKernelGGL((k_sw_paths<F, MAXM>), dim3(blocks), dim3(kSwThreads), 0, st, heads, pool,
-                       bps, paths, partial);
+using LaunchLin = void (*)(unsigned, hipStream_t, const SwLin*, const double*, const SwGrid&,
+                           double*);
+template <int MAXW>
+void launch_linear(unsigned blocks, hipStream_t st, const SwLin* heads, const double* pool,
+                   const SwGrid& grid, double* partial) {
+    hipLaunchKernelGGL((k_sw_paths<MAXW>), dim3(blocks), dim3(kSwThreads), 0, st, heads, pool,
+                       grid, partial);
+}
+LaunchLin linear_kernel(int flows) {
+    return flows <= 2    ? launch_linear<2>
+           : flows <= 4  ? launch_linear<4>
+           : flows <= 8  ? launch_linear<8>
+           : flows <= 16 ? launch_linear<16>
+           : flows <= 32 ? launch_linear<32>
+                         : launch_linear<64>;
 }
 
 template <int F>
-void launch_f(int mmax, unsigned blocks, hipStream_t st, const SwHead* heads, const double* pool,
-              int bps, int64_t paths, double* partial) {
-    if (mmax <= 2)
-        launch_paths<F, 2>(blocks, st, heads, pool, bps, paths, partial);
-    else if (mmax <= 4)
-        launch_paths<F, 4>(blocks, st, heads, pool, bps, paths, partial);
-    else if constexpr (F <= 4) {
-        // starts at steps 5-8: draws in registers (86-118 VGPRs), 2.1-2.5x the
-        // speed of the generic form, whose draws live in scratch
-        if (mmax <= 8)
-            launch_paths<F, 8>(blocks, st, heads, pool, bps, paths, partial);
-        else
-            launch_paths<F, kSwMaxDraws / F>(blocks, st, heads, pool, bps, paths, partial);
-    } else {
-        launch_paths<F, kSwMaxDraws / F>(blocks, st, heads, pool, bps, paths, partial);
-    }
+void launch_steps(unsigned blocks, hipStream_t st, const SwLin* lin, const SwHead* heads,
+                  const double* pool, const SwGrid& grid, double* partial) {
+    hipLaunchKernelGGL((k_sw_paths_steps<F, kSwMaxDraws / F>), dim3(blocks), dim3(kSwThreads), 0,
+                       st, lin, heads, pool, grid, partial);
 }
-
-using LaunchF = void (*)(int, unsigned, hipStream_t, const SwHead*, const double*, int, int64_t,
-                         double*);
-constexpr LaunchF kLaunchByFactors[kSwMaxFactors] = {launch_f<1>, launch_f<2>, launch_f<3>,
-                                                     launch_f<4>, launch_f<5>, launch_f<6>,
-                                                     launch_f<7>, launch_f<8>};
+using LaunchSteps = void (*)(unsigned, hipStream_t, const SwLin*, const SwHead*, const double*,
+                             const SwGrid&, double*);
+constexpr LaunchSteps kStepsByFactors[kSwMaxFactors] = {
+    launch_steps<1>, launch_steps<2>, launch_steps<3>, launch_steps<4>,
+    launch_steps<5>, launch_steps<6>, launch_steps<7>, launch_steps<8>};
 
 bool finite_all(const bs_swaption_t& s) {
     return std::isfinite(s.strike) && std::isfinite(s.compounding) && std::isfinite(s.maturity) &&
@@ -364,11 +741,14 @@ int round_index(double x) {
     return (y > -1e9 && y < 1e9) ? (int)y : INT32_MIN;
 }
 
-// Validates swaption i and appends its head and data (the per-swaption set-up
-// of HJM_Swaption_Blocking.cpp:48-150 and HJM.cpp's forward curve and drifts,
-// in host FP64 without contraction, as the reference computes them).
-int pack_swaption(const bs_swaption_t& s, int64_t i, int64_t seed, SwHead* h,
-                  std::vector<double>* pool) {
+// Index sizes of a swaption (HJM_Swaption_Blocking.cpp:48-70).
+struct SwShape {
+    double dt;
+    int m, L, freq, points;
+};
+
+// Validates swaption i.
+int shape_of(const bs_swaption_t& s, int64_t i, SwShape* x) {
     const int n = s.n_steps, F = s.n_factors;
     char msg[160];
     auto bad = [&](const char* why) {
@@ -388,6 +768,17 @@ int pack_swaption(const bs_swaption_t& s, int64_t i, int64_t seed, SwHead* h,
     if (m < 0 || m >= n) return bad("maturity outside the simulated horizon");
     if (L < 1 || points < 0 || points > L - 1) return bad("swap tenor outside the horizon");
     if (m * F > kSwMaxDraws) return bad("start step x n_factors exceeds 64");
+    *x = {dt, m, L, freq, points};
+    return BS_OK;
+}
+
+// Appends a swaption's head and data (the per-swaption set-up of
+// HJM_Swaption_Blocking.cpp:48-150 and HJM.cpp's forward curve and drifts, in
+// host FP64 without contraction, as the reference computes them).
+void pack_swaption(const bs_swaption_t& s, const SwShape& x, int64_t seed, SwHead* h,
+                   std::vector<double>* pool) {
+    const int n = s.n_steps, F = s.n_factors, m = x.m, L = x.L, freq = x.freq, points = x.points;
+    const double dt = x.dt;
     const double strike_cont = s.compounding == 0
                                    ? s.strike
                                    : (1 / s.compounding) * log(1 + s.strike * s.compounding);
@@ -400,8 +791,6 @@ int pack_swaption(const bs_swaption_t& s, int64_t i, int64_t seed, SwHead* h,
     h->m = m;
     h->L = L;
     h->off = (int32_t)pool->size();
-    h->last = points;
-    h->pad = 0;
     const size_t base = pool->size();
     pool->resize(base + n + w + (size_t)F * w + L, 0.0);
     double* f0 = pool->data() + base;
@@ -435,7 +824,92 @@ int pack_swaption(const bs_swaption_t& s, int64_t i, int64_t seed, SwHead* h,
     for (int l = freq; l <= points; l += freq)
         pay[l] = l != points ? exp(strike_cont * s.payment_interval) - 1
                              : exp(strike_cont * s.payment_interval);
-    return BS_OK;
+}
+
+// Appends the linear form of the swaption that pack_swaption packed at h:
+// every exponent of its payoff, in base 2, as a constant and one coefficient
+// per draw.
+// It holds if the running products of discount factors that the reference
+// forms stay far from overflow and underflow: with every finite draw below 7
+// in size (Moro at u = 4.66e-10 is 6.2), the rates times their times sum to at
+// most 400 in base 2 over the whole curve, so every product is within 2^+-400.
+// (Their terms are then finite too, and the factors past the last cash flow,
+// which the reference multiplies by zero, contribute +0.)
+void pack_linear(const SwHead& h, int F, int freq, int points, SwLin* x,
+                 std::vector<double>* pool) {
+    const int n = h.n, m = h.m, w = n - 1, D = m * F;
+    x->seed = h.seed;
+    x->per_path = (uint32_t)(w * F);
+    x->x_path = gen_step(x->per_path);
+    x->x_row = gen_step((uint64_t)kSwThreads * x->per_path);
+    x->draws = D;
+    x->df_draws = m > 0 ? (m - 1) * F : 0;
+    x->flows = points / freq;
+    const int W = lin_width(x->flows);
+    pool->resize((pool->size() + 7) & ~(size_t)7);   // scalar loads of whole lines
+    x->off = (int32_t)pool->size();
+    const size_t base = pool->size(), old = (size_t)h.off;
+    pool->resize(base + 2 * W + (size_t)D * W + D, 0.0);
+    const double* f0 = pool->data() + old;
+    const double* mudt = f0 + n;
+    const double* sig = mudt + w;
+    const double* cash = sig + (size_t)F * w;
+    double* C = pool->data() + base;
+    double* pay = C + W;
+    double* G = pay + W;
+    double* gdf = G + (size_t)D * W;
+    constexpr long double kLog2eL = 1.442695040888963407359924681001892137L;
+    // sqrt(dt) sigma log2 e per rate step and factor, and their sizes
+    double g[kSwMaxSteps * kSwMaxFactors], size_of[kSwMaxSteps];
+    for (int l = 0; l < w; ++l) {
+        size_of[l] = 0.0;
+        for (int k = 0; k < F; ++k) {
+            g[l * F + k] = (double)(h.sdt * kLog2eL * sig[(size_t)k * w + l]);
+            size_of[l] += std::fabs(g[l * F + k]);
+        }
+    }
+    long double base_sum = 0.0L;   // the running exponent: its constant,
+    double sum[kSwMaxDraws] = {};  // and per draw, both before the factor -t
+    double size = 0.0;             // bound on the sum of |rate| x time, in base 2
+    int c = 0;
+    for (int d = 0; d < n; ++d) {
+        if (d == m) {   // the discount to the start is complete
+            x->c_df = (double)(-h.dt * base_sum);
+            for (int j = 0; j < D; ++j) gdf[j] = -h.dt * sum[j];
+            base_sum = 0.0L;
+            std::fill(sum, sum + D, 0.0);
+        }
+        const int steps = std::min(d, m);
+        long double rate = f0[d];
+        double shocks = 0.0;
+        for (int s = 1; s <= steps; ++s) {
+            const int l = d - s;
+            rate += mudt[l];
+            shocks += size_of[l];
+            for (int k = 0; k < F; ++k) sum[(s - 1) * F + k] += g[l * F + k];
+        }
+        base_sum += kLog2eL * rate;
+        size += (d < m ? h.dt : h.dts) * (1.4427 * std::fabs((double)rate) + 7.0 * shocks);
+        const int l = d - m + 1;   // the swap curve's point whose discount this completes
+        if (d >= m && l <= points && l % freq == 0) {
+            C[c] = (double)(-h.dts * base_sum);
+            pay[c] = cash[l];
+            for (int j = 0; j < D; ++j) G[(size_t)j * W + c] = -h.dts * sum[j];
+            ++c;
+        }
+    }
+    for (; c < x->flows; ++c) {   // cash flows past the simulated curve: zero rates there
+        C[c] = (double)(-h.dts * base_sum);
+        pay[c] = cash[(c + 1) * freq];
+        for (int j = 0; j < D; ++j) G[(size_t)j * W + c] = -h.dts * sum[j];
+    }
+    x->linear = size <= 400.0 ? 1 : 0;   // false for NaN
+}
+
+// Whether counters [c, c + count) hold a multiple of 2^31-1.
+bool draws_zero(int64_t c, int64_t count) {
+    const int64_t m = (int64_t)kM31;
+    return c % m == 0 || c / m != (c + count - 1) / m;
 }
 
 // The per-call buffers (parameters, partial sums, results) come from one
@@ -469,6 +943,79 @@ hipError_t pool_of(int dev, hipMemPool_t* out) {
     return hipSuccess;
 }
 
+// Swaptions of one launch.
+struct SwBatch {
+    std::vector<SwLin> lins;
+    std::vector<SwHead> heads;
+    std::vector<double> pool;
+    std::vector<int32_t> index;   // places in the caller's array
+    int flows = 0;
+    bool steps = false;           // some block needs the step-by-step kernel
+
+    // paths: those the swaption's blocks cover.
+    void add(const bs_swaption_t& s, const SwShape& x, int64_t seed, int32_t i, int64_t paths) {
+        heads.emplace_back();
+        lins.emplace_back();
+        index.push_back(i);
+        pack_swaption(s, x, seed, &heads.back(), &pool);
+        pack_linear(heads.back(), s.n_factors, x.freq, x.points, &lins.back(), &pool);
+        flows = std::max(flows, lins.back().flows);
+        steps = steps || !lins.back().linear ||
+                draws_zero(seed, paths * lins.back().per_path);
+    }
+};
+
+int price_batch(const SwBatch& b, int F, const SwGrid& grid, int64_t trials, double* price,
+                double* std_error, hipStream_t st) {
+    const size_t n = b.lins.size();
+    const unsigned blocks = (unsigned)(grid.bps * (int64_t)n);
+    // one device allocation: heads of both kernels | pool | partials | results
+    auto up = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
+    const size_t lb = up(n * sizeof(SwLin)), hb = lb + up(n * sizeof(SwHead));
+    const size_t pb = up(b.pool.size() * sizeof(double));
+    const size_t qb = up((size_t)blocks * 2 * sizeof(double));
+    const size_t ob = n * 2 * sizeof(double);
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return hip_error(e, "hipGetDevice");
+    hipMemPool_t mem = nullptr;
+    e = pool_of(dev, &mem);
+    if (e != hipSuccess) return hip_error(e, "hipMemPoolCreate");
+    char* base = nullptr;
+    e = hipMallocFromPoolAsync(reinterpret_cast<void**>(&base), hb + pb + qb + ob, mem, st);
+    if (e != hipSuccess) return hip_error(e, "hipMallocFromPoolAsync");
+    SwLin* dl = reinterpret_cast<SwLin*>(base);
+    SwHead* dh = reinterpret_cast<SwHead*>(base + lb);
+    double* dp = reinterpret_cast<double*>(base + hb);
+    double* dq = reinterpret_cast<double*>(base + hb + pb);
+    double* dout = reinterpret_cast<double*>(base + hb + pb + qb);
+    std::vector<double> out(n * 2);
+    // heads and pool leave the host as one copy, laid out as on the device
+    std::vector<char> staged(hb + b.pool.size() * sizeof(double));
+    memcpy(staged.data(), b.lins.data(), n * sizeof(SwLin));
+    memcpy(staged.data() + lb, b.heads.data(), n * sizeof(SwHead));
+    memcpy(staged.data() + hb, b.pool.data(), b.pool.size() * sizeof(double));
+    e = hipMemcpyAsync(base, staged.data(), staged.size(), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) {
+        linear_kernel(b.flows)(blocks, st, dl, dp, grid, dq);
+        if (b.steps) kStepsByFactors[F - 1](blocks, st, dl, dh, dp, grid, dq);
+        hipLaunchKernelGGL(k_sw_final, dim3((unsigned)n), dim3(kSwThreads), 0, st, dq, grid.bps,
+                           trials, dout);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(out.data(), dout, ob, hipMemcpyDeviceToHost, st);
+    const hipError_t ef = hipFreeAsync(base, st);
+    const hipError_t es = hipStreamSynchronize(st);
+    if (e != hipSuccess) return hip_error(e, "bs_swaptions_host_f64");
+    if (ef != hipSuccess) return hip_error(ef, "hipFreeAsync");
+    if (es != hipSuccess) return hip_error(es, "hipStreamSynchronize");
+    for (size_t k = 0; k < n; ++k) {
+        price[b.index[k]] = out[2 * k];
+        std_error[b.index[k]] = out[2 * k + 1];
+    }
+    return BS_OK;
+}
+
 }  // namespace
 }  // namespace bs
 
@@ -489,69 +1036,49 @@ extern "C" int bs_swaptions_host_f64(const bs_swaption_t* sw, int64_t n, int64_t
             return set_error(BS_ERR_INVALID, "seed must be in [0, 2^42)");
         const int F = sw[0].n_factors;
         const int64_t paths = (trials + block_size - 1) / block_size * block_size;
-        std::vector<SwHead> heads((size_t)n);
-        std::vector<double> pool;
-        int mmax = 0;
+        std::vector<SwShape> shapes((size_t)n);
         for (int64_t i = 0; i < n; ++i) {
             if (sw[i].n_factors != F)
                 return set_error(BS_ERR_INVALID, "every swaption must have the same n_factors");
-            int rc = pack_swaption(sw[i], i, seed + i, &heads[(size_t)i], &pool);
+            const int rc = shape_of(sw[i], i, &shapes[(size_t)i]);
             if (rc) return rc;
             const int64_t draws = (int64_t)(sw[i].n_steps - 1) * F;
             if (paths > (kSwCounterLimit - (seed + i)) / draws)
                 return set_error(BS_ERR_INVALID, "seed + paths x draws exceeds 2^42");
-            mmax = std::max(mmax, heads[(size_t)i].m);
         }
-        if (pool.size() > (size_t)INT32_MAX) return set_error(BS_ERR_INVALID, "too many swaptions");
-        const int64_t per_block = (int64_t)kSwThreads * kSwPer;
-        const int64_t bps64 = (paths + per_block - 1) / per_block;
         // one launch of at most 2^32 work-items: 2^24 blocks of 1024 paths
-        if (bps64 * n > (int64_t(1) << 24))
+        const int64_t bps_most = (paths + kSwThreads * kSwRows - 1) / (kSwThreads * kSwRows);
+        if (bps_most * n > (int64_t(1) << 24))
             return set_error(BS_ERR_INVALID,
                              "more than 2^24 blocks of 1024 paths (2^34 paths) in one call");
-        const int bps = (int)bps64;
-        const unsigned blocks = (unsigned)(bps64 * n);
-        const hipStream_t st = static_cast<hipStream_t>(stream);
-        // one device allocation: heads | pool | partials | results
-        const size_t hb = ((size_t)n * sizeof(SwHead) + 255) & ~(size_t)255;
-        const size_t pb = (pool.size() * sizeof(double) + 255) & ~(size_t)255;
-        const size_t qb = (size_t)blocks * 2 * sizeof(double);
-        const size_t ob = (size_t)n * 2 * sizeof(double);
-        int dev = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e != hipSuccess) return hip_error(e, "hipGetDevice");
-        hipMemPool_t mem = nullptr;
-        e = pool_of(dev, &mem);
-        if (e != hipSuccess) return hip_error(e, "hipMemPoolCreate");
-        char* base = nullptr;
-        e = hipMallocFromPoolAsync(reinterpret_cast<void**>(&base), hb + pb + qb + ob, mem, st);
-        if (e != hipSuccess) return hip_error(e, "hipMallocFromPoolAsync");
-        SwHead* dh = reinterpret_cast<SwHead*>(base);
-        double* dp = reinterpret_cast<double*>(base + hb);
-        double* dq = reinterpret_cast<double*>(base + hb + pb);
-        double* dout = reinterpret_cast<double*>(base + hb + pb + qb);
-        std::vector<double> out((size_t)n * 2);
-        // heads and pool leave the host as one copy, laid out as on the device
-        std::vector<char> staged(hb + pool.size() * sizeof(double));
-        memcpy(staged.data(), heads.data(), (size_t)n * sizeof(SwHead));
-        memcpy(staged.data() + hb, pool.data(), pool.size() * sizeof(double));
-        e = hipMemcpyAsync(base, staged.data(), staged.size(), hipMemcpyHostToDevice, st);
-        if (e == hipSuccess) {
-            kLaunchByFactors[F - 1](mmax, blocks, st, dh, dp, bps, paths, dq);
-            hipLaunchKernelGGL(k_sw_final, dim3((unsigned)n), dim3(kSwThreads), 0, st, dq, bps,
-                               trials, dout);
-            e = hipGetLastError();
-        }
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(out.data(), dout, ob, hipMemcpyDeviceToHost, st);
-        const hipError_t ef = hipFreeAsync(base, st);
-        const hipError_t es = hipStreamSynchronize(st);
-        if (e != hipSuccess) return hip_error(e, "bs_swaptions_host_f64");
-        if (ef != hipSuccess) return hip_error(ef, "hipFreeAsync");
-        if (es != hipSuccess) return hip_error(es, "hipStreamSynchronize");
-        for (int64_t i = 0; i < n; ++i) {
-            price[i] = out[(size_t)(2 * i)];
-            std_error[i] = out[(size_t)(2 * i + 1)];
+        // Paths per work-item: enough of them to spread the 100 or so
+        // instructions of its set-up while several rounds of blocks are left
+        // (1024 are resident at once).  128 swaptions x 1M trials take 931 us
+        // with 4 rows, 844 with 8, 812 with 16 and 805 with 32; 32 swaptions x
+        // 50,000 trials (starts at steps 1-10, 4 factors) 171, 190, 282 and 468.
+        const int rows = bps_most * n >= 65536 ? 16 : bps_most * n >= 16384 ? 8 : kSwRows;
+        const int64_t bps = (paths + kSwThreads * rows - 1) / (kSwThreads * rows);
+        // the swaptions whose paths cost most first, so that the launch ends on
+        // its cheapest blocks
+        std::vector<int32_t> order((size_t)n);
+        for (int64_t i = 0; i < n; ++i) order[(size_t)i] = (int32_t)i;
+        auto cost = [&](int32_t i) {
+            const SwShape& x = shapes[(size_t)i];
+            const int W = lin_width(x.points / x.freq);
+            return x.m * F * (45 + W) + 20 * W;
+        };
+        std::stable_sort(order.begin(), order.end(),
+                         [&](int32_t a, int32_t b) { return cost(a) > cost(b); });
+        // parameters of more than 2^24 doubles go in several launches
+        for (size_t first = 0; first < (size_t)n;) {
+            SwBatch batch;
+            for (; first < (size_t)n && batch.pool.size() < (size_t(1) << 24); ++first) {
+                const int32_t i = order[first];
+                batch.add(sw[i], shapes[(size_t)i], seed + i, i, bps * kSwThreads * rows);
+            }
+            const int rc = price_batch(batch, F, {paths, (int32_t)bps, rows}, trials, price,
+                                       std_error, static_cast<hipStream_t>(stream));
+            if (rc) return rc;
         }
         return BS_OK;
     });

@@ -170,3 +170,53 @@ def test_counters_near_the_limit(gpu):
     from p3arsec_amd import capi
     with pytest.raises(capi.BSError):
         W.price([s], trials, 2 ** 42 - 1008 * 30 + 1)
+
+
+@pytest.mark.parametrize("n,F,start,points,every", [
+    # draws (start x F) and cash flows (points / every) at the edges of the
+    # register form (3, 6 draws; 1-4 flows) and of the wide form's batches of
+    # 12 draws and its widths up to 64 flows
+    (11, 1, 1, 1, 1), (11, 2, 1, 2, 1), (11, 1, 3, 3, 1), (11, 4, 1, 4, 1), (11, 5, 1, 2, 2),
+    (11, 3, 2, 4, 2), (11, 7, 1, 3, 1), (20, 4, 3, 5, 1), (20, 6, 2, 6, 1), (20, 1, 13, 6, 1),
+    (30, 8, 3, 7, 1), (30, 5, 5, 8, 1), (40, 7, 7, 9, 1), (40, 2, 12, 12, 1), (40, 8, 8, 13, 1),
+    (40, 3, 1, 16, 1), (40, 1, 4, 17, 1), (64, 2, 6, 24, 1), (64, 2, 32, 25, 1), (64, 3, 8, 32, 1),
+    (64, 1, 2, 33, 1), (64, 1, 7, 48, 1), (64, 1, 13, 49, 1), (64, 1, 1, 62, 1), (64, 4, 1, 62, 3),
+])
+def test_draw_and_cash_flow_edges(gpu, n, F, start, points, every):
+    """The bar is the file's: about 64 roundings of exponents below 4 in size
+    move a payoff by at most 64 x 4 x 2^-53 = 3e-14 relative to the bonds."""
+    years = 0.25 * n
+    s = sw(n=n, F=F, years=years, maturity=start * 0.25, tenor=points * 0.25,
+           interval=every * 0.25, strike=0.13)
+    for trials in (1, 255, 5000):
+        got = W.price([s], trials, 97 * n + F, 1)
+        check((got[0][0], got[1][0]), S.price_blocking(s, 97 * n + F, trials, 1), (n, F, trials))
+
+
+@pytest.mark.parametrize("count,trials", [(128, 131_073), (128, 524_289)])
+def test_more_paths_per_work_item(gpu, count, trials):
+    sws, base = W.parsec_portfolio(count)
+    p, e = W.price(sws, trials, base)
+    for i in (0, count - 1):
+        check((p[i], e[i]), S.price_chain(sws[i], base + i, trials), i)
+
+
+def test_blocks_with_a_zero_draw(gpu):
+    """One block of five holds the counter that draws u = 0, in a draw the
+    payoff does not read (finite prices) or reads (the reference's NaN or inf);
+    its paths take the step-by-step kernel, the others the linear one."""
+    m31 = 2147483647
+    for s in W.parsec_portfolio(3)[0]:
+        for offset in (25, 1):
+            seed = m31 - 30 * 2500 - offset
+            got = W.price([s], 5000, seed)
+            check((got[0][0], got[1][0]), S.price_blocking(s, seed, 5000), offset)
+
+
+def test_rates_past_the_linear_bound(gpu):
+    """A horizon of 2000 years: exponents past the bound that keeps the
+    reference's products from underflow, next to an ordinary swaption."""
+    wide = sw(years=2000.0, maturity=182.0, tenor=364.0, interval=182.0, strike=0.02)
+    p, e = W.price([wide, sw(strike=0.13)], 3000, 31)
+    for i, s in enumerate((wide, sw(strike=0.13))):
+        check((p[i], e[i]), S.price_blocking(s, 31 + i, 3000), i)
