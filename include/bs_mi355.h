@@ -114,15 +114,14 @@ int bs_price_i32type_f32(const float *s, const float *k, const float *r, const f
                          const float *t, const int32_t *otype, float *price, int64_t n,
                          bs_stream_t stream);
 /* The reference's NUM_RUNS loop (BS:315-348, the FastFlow map's passes;
- * BS:607-658, bs_thread's): prices the book `passes` times on `stream`, each
- * pass starting after the previous one ends, with the same output as calling
- * bs_price_f32 (otype_bytes = 1, uint8 types) or bs_price_i32type_f32
- * (otype_bytes = 4, int32 types) `passes` times.  For books of up to 2^25
- * options the passes are one hipGraph of `passes` kernel nodes, captured on
- * the first call for these arrays, n, passes and device, and replayed after
- * that (the library keeps the 16 most recently used): small books are bound
- * by launch cost, and larger ones lose less to the cache maintenance between
- * separately launched passes.  Larger books launch pass by pass. */
+ * BS:607-658, bs_thread's): prices the book `passes` times on `stream`, with
+ * the same output as calling bs_price_f32 (otype_bytes = 1, uint8 types) or
+ * bs_price_i32type_f32 (otype_bytes = 4, int32 types) `passes` times.  Every
+ * pass loads, prices and stores every option, and the passes of each option
+ * are in order; one launch carries them option by option, with no barrier over
+ * the book between passes (small books are bound by kernel boundaries).  Where
+ * price overlaps an input, each pass is a launch of its own, so that it reads
+ * what the pass before it wrote. */
 int bs_price_passes_f32(const float *s, const float *k, const float *r, const float *v,
                         const float *t, const void *otype, int otype_bytes, float *price,
                         int64_t n, int passes, bs_stream_t stream);

@@ -9,7 +9,6 @@
 #include <algorithm>
 #include <mutex>
 #include <string>
-#include <vector>
 
 #include "bs_internal.hpp"
 
@@ -119,98 +118,12 @@ float* scalar_slot() {
 
 }  // namespace
 
-// ---- repeated passes ---------------------------------------------------------------
 namespace {
 
-// Books up to this size replay their passes from one graph.  Small books are
-// bound by launch cost (a pass takes a few microseconds, about what the host
-// spends per launch); larger ones gain because consecutive kernel nodes of a
-// graph skip part of the cache maintenance that separate launches do between
-// passes that reread the same book (measured per pass: 4096 options 4.6 ->
-// 1.9 us, 10M 43.2 -> 39.4 us, 32M 124.0 -> 122.9 us).  Past this size the
-// gain no longer repays a first call's capture.
-constexpr int64_t kPassGraphMaxOptions = int64_t(1) << 25;
-constexpr size_t kPassGraphs = 16;
-constexpr int kPassDevices = 64;
-
-// A graph is valid for the arrays, sizes and device it was captured with, and
-// for the launch settings that shaped its kernels.
-struct PassKey {
-    const void* ptr[7];
-    int64_t n;
-    int passes, type_bytes, device;
-    int64_t launch[6];   // max_blocks, vector_width, nontemporal, pipeline, block_threads,
-                         // lds_per_wave
-    bool operator==(const PassKey& o) const {
-        return memcmp(ptr, o.ptr, sizeof(ptr)) == 0 && n == o.n && passes == o.passes &&
-               type_bytes == o.type_bytes && device == o.device &&
-               memcmp(launch, o.launch, sizeof(launch)) == 0;
-    }
-};
-
-struct PassGraph {
-    PassKey key;
-    hipGraphExec_t exec;
-    hipEvent_t done;   // recorded after each replay: eviction waits for it
-};
-
-struct PassGraphCache {
-    std::mutex mu;
-    std::vector<PassGraph> lru;                     // most recently used first
-    hipStream_t capture[kPassDevices] = {};
-};
-
-PassGraphCache& pass_cache() {
-    static PassGraphCache* c = new PassGraphCache();   // lives until the process ends
-    return *c;
-}
-
-hipError_t launch_pass(const SoaIn<float>& in, const void* type, int type_bytes, float* out,
-                       int64_t n, hipStream_t st) {
-    return type_bytes == 1
-               ? launch_price_f32(in, static_cast<const uint8_t*>(type), out, n, st)
-               : launch_price_i32type_f32(in, static_cast<const int32_t*>(type), out, n, st);
-}
-
-// The cached graph for key, captured now if absent (the cache's lock held).
-PassGraph* pass_graph(PassGraphCache& c, const PassKey& key, const SoaIn<float>& in,
-                      const void* type, float* out, hipError_t* e) {
-    for (size_t i = 0; i < c.lru.size(); ++i)
-        if (c.lru[i].key == key) {
-            std::rotate(c.lru.begin(), c.lru.begin() + (std::ptrdiff_t)i,
-                        c.lru.begin() + (std::ptrdiff_t)i + 1);
-            return &c.lru.front();
-        }
-    hipStream_t& cs = c.capture[key.device];
-    if (!cs && (*e = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking)) != hipSuccess) {
-        cs = nullptr;
-        return nullptr;
-    }
-    if ((*e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal)) != hipSuccess)
-        return nullptr;
-    hipError_t le = hipSuccess;
-    for (int p = 0; p < key.passes && le == hipSuccess; ++p)
-        le = launch_pass(in, type, key.type_bytes, out, key.n, cs);
-    hipGraph_t graph = nullptr;
-    const hipError_t ce = hipStreamEndCapture(cs, &graph);
-    *e = le != hipSuccess ? le : ce;
-    PassGraph g{key, nullptr, nullptr};
-    if (*e == hipSuccess) *e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
-    if (graph) (void)hipGraphDestroy(graph);
-    if (*e == hipSuccess) *e = hipEventCreateWithFlags(&g.done, hipEventDisableTiming);
-    if (*e != hipSuccess) {
-        if (g.exec) (void)hipGraphExecDestroy(g.exec);
-        return nullptr;
-    }
-    if (c.lru.size() == kPassGraphs) {
-        PassGraph& old = c.lru.back();
-        (void)hipEventSynchronize(old.done);
-        (void)hipEventDestroy(old.done);
-        (void)hipGraphExecDestroy(old.exec);
-        c.lru.pop_back();
-    }
-    c.lru.insert(c.lru.begin(), g);
-    return &c.lru.front();
+// Whether [a, a + na) and [b, b + nb) share a byte.
+bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + nb && y < x + na;
 }
 
 }  // namespace
@@ -455,24 +368,22 @@ int bs_price_passes_f32(const float* s, const float* k, const float* r, const fl
             return rc;
         const SoaIn<float> in{s, k, r, v, t};
         const hipStream_t st = as_stream(stream);
-        int dev = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e != hipSuccess) return hip_error(e, "hipGetDevice");
-        if (n <= kPassGraphMaxOptions && passes > 1 && dev < kPassDevices) {
-            const Config& cf = config();
-            const PassKey key{{s, k, r, v, t, otype, price}, n, passes, otype_bytes, dev,
-                              {cf.max_blocks, cf.vector_width, cf.nontemporal, cf.pipeline,
-                               cf.block_threads, cf.lds_per_wave}};
-            PassGraphCache& c = pass_cache();
-            std::lock_guard<std::mutex> lk(c.mu);
-            PassGraph* g = pass_graph(c, key, in, otype, price, &e);
-            if (!g) return hip_error(e, "bs_price_passes_f32: graph capture");
-            e = hipGraphLaunch(g->exec, st);
-            if (e == hipSuccess) e = hipEventRecord(g->done, st);
-            return done(e, "bs_price_passes_f32");
+        const size_t fb = (size_t)n * 4;
+        bool apart = !overlap(price, fb, otype, (size_t)n * otype_bytes);
+        for (const float* a : {s, k, r, v, t}) apart = apart && !overlap(price, fb, a, fb);
+        hipError_t e = hipSuccess;
+        // One launch holds at most 2^33 priced options (about 25 ms).  A pass
+        // that may read what the one before it wrote is a launch of its own.
+        const int64_t most = apart ? std::max<int64_t>(1, (int64_t(1) << 33) / n) : 1;
+        for (int64_t left = passes; left > 0 && e == hipSuccess; left -= most) {
+            const int now = (int)std::min(left, most);
+            if (now > 1)
+                e = launch_price_passes_f32(in, otype, otype_bytes, price, n, now, st);
+            else if (otype_bytes == 1)
+                e = launch_price_f32(in, static_cast<const uint8_t*>(otype), price, n, st);
+            else
+                e = launch_price_i32type_f32(in, static_cast<const int32_t*>(otype), price, n, st);
         }
-        for (int p = 0; p < passes && e == hipSuccess; ++p)
-            e = launch_pass(in, otype, otype_bytes, price, n, st);
         return done(e, "bs_price_passes_f32");
     });
 }

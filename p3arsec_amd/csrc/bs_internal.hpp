@@ -72,6 +72,9 @@ hipError_t launch_price_f32(SoaIn<float> in, const uint8_t* type, float* out, in
                             hipStream_t st);
 hipError_t launch_price_i32type_f32(SoaIn<float> in, const int32_t* type, float* out,
                                     int64_t n, hipStream_t st);
+// `passes` passes in one launch; out must overlap no input.
+hipError_t launch_price_passes_f32(SoaIn<float> in, const void* type, int type_bytes, float* out,
+                                   int64_t n, int passes, hipStream_t st);
 hipError_t launch_price_fast_f32(SoaIn<float> in, const uint8_t* type, float* out,
                                      int64_t n, hipStream_t st);
 hipError_t launch_price_f64(SoaIn<double> in, const uint8_t* type, double* out,

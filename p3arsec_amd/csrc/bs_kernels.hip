@@ -175,6 +175,86 @@ bool soa_aligned(const SoaIn<T>& in, uintptr_t a) {
            aligned(in.t, a);
 }
 
+// ---- repeated passes ------------------------------------------------------------
+// `passes` passes over a book in one launch: a work-item owns its options and
+// prices them pass after pass, every pass loading its inputs, pricing and
+// storing.  Passes of one option are in order; no pass reads another's output
+// (the caller has checked that price overlaps no input), so options need not
+// wait for one another, and a book is read from HBM once: later passes find
+// their inputs in the caches.  TOGETHER passes are in flight at once: their
+// loads go out before their arithmetic, whose chains are then independent.
+// The compiler may not carry a value from one pass to the next: each load is
+// behind a compiler fence.
+//
+// Bound by VALU issue, or by one wave's latency where a book leaves each SIMD
+// one wave or none.  100 passes, against a graph of 100 kernel nodes (1.9 us
+// each at least, the kernel boundary): 4096 options 27.4 us and 187 us, 65536
+// 29.3 and 201, 200,000 77 and 237, 1M 266 and 482; 10 passes of 10M 280 and
+// 403 us.  One pass at a time instead of four takes 35.4 us at 4096 options and
+// 39.9 at 65536; from 2 waves per SIMD on (2^17 options) it is as fast, and
+// with fewer registers faster past that (1M: 266 us against 288).
+constexpr int64_t kTogetherMaxOptions = int64_t(1) << 17;
+
+template <class TY>
+struct PassIn {
+    float s, k, r, v, t;
+    TY ty;
+};
+
+template <class TY, class Ix>
+__device__ __forceinline__ PassIn<TY> load_pass(const SoaIn<float>& in, const TY* type, Ix i) {
+    asm volatile("" ::: "memory");
+    return {*at(in.s, i), *at(in.k, i), *at(in.r, i), *at(in.v, i), *at(in.t, i), *at(type, i)};
+}
+
+template <class TY, int TOGETHER, class Ix>
+__global__ __launch_bounds__(kThreads) void k_passes(SoaIn<float> in, const TY* type, float* out,
+                                                     int64_t n, int passes) {
+    const Ix stride = (Ix)gridDim.x * blockDim.x;
+    for (Ix i = (Ix)blockIdx.x * blockDim.x + threadIdx.x; i < (Ix)n; i += stride) {
+        int p = 0;
+        for (; p + TOGETHER <= passes; p += TOGETHER) {
+            PassIn<TY> x[TOGETHER];
+            float price[TOGETHER];
+#pragma unroll
+            for (int j = 0; j < TOGETHER; ++j) x[j] = load_pass(in, type, i);
+#pragma unroll
+            for (int j = 0; j < TOGETHER; ++j)
+                price[j] = bs_price<Ref32>(x[j].s, x[j].k, x[j].r, x[j].v, x[j].t, x[j].ty != 0);
+#pragma unroll
+            for (int j = 0; j < TOGETHER; ++j) {
+                *at(out, i) = price[j];
+                asm volatile("" ::: "memory");
+            }
+        }
+        if constexpr (TOGETHER > 1) {
+            for (; p < passes; ++p) {
+                const PassIn<TY> x = load_pass(in, type, i);
+                *at(out, i) = bs_price<Ref32>(x.s, x.k, x.r, x.v, x.t, x.ty != 0);
+            }
+        }
+    }
+}
+
+template <class TY>
+hipError_t launch_passes_t(SoaIn<float> in, const TY* type, float* out, int64_t n, int passes,
+                           hipStream_t st) {
+    const int64_t cap = config().max_blocks.load(std::memory_order_relaxed);
+    const int bt = config().block_threads.load(std::memory_order_relaxed);
+    const int nt = bt > 0 ? bt : 64;
+    const dim3 grid(grid_for(n, cap, nt));
+    if (n <= kTogetherMaxOptions)
+        hipLaunchKernelGGL((k_passes<TY, 4, uint32_t>), grid, dim3(nt), 0, st, in, type, out, n,
+                           passes);
+    else if (n < (int64_t(1) << 30))
+        hipLaunchKernelGGL((k_passes<TY, 1, uint32_t>), grid, dim3(nt), 0, st, in, type, out, n,
+                           passes);
+    else
+        hipLaunchKernelGGL((k_passes<TY, 1, int64_t>), grid, dim3(nt), 0, st, in, type, out, n,
+                           passes);
+    return hipGetLastError();
+}
+
 // ---- AoS -> SoA repack ------------------------------------------------------
 // OptionData (blackscholes.c:89-100): 9 dwords per record; dword 6 holds the
 // OptionType char in its low byte.  A block stages 256 records (2304 dwords,
@@ -268,6 +348,13 @@ hipError_t launch_price_i32type_f32(SoaIn<float> in, const int32_t* type, float*
                                     int64_t n, hipStream_t st) {
     return launch_stream<PriceI32F32>(PriceI32Args{in, type, out}, n, 2,
                                       price_align(in, type, out, 4), st);
+}
+
+hipError_t launch_price_passes_f32(SoaIn<float> in, const void* type, int type_bytes, float* out,
+                                   int64_t n, int passes, hipStream_t st) {
+    return type_bytes == 1
+               ? launch_passes_t(in, static_cast<const uint8_t*>(type), out, n, passes, st)
+               : launch_passes_t(in, static_cast<const int32_t*>(type), out, n, passes, st);
 }
 
 hipError_t launch_price_f64(SoaIn<double> in, const uint8_t* type, double* out, int64_t n,

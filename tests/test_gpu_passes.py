@@ -9,6 +9,8 @@ MI355X, through the C ABI.
   result for the inputs it saw (the graph holds pointers, not contents).
 * More distinct calls than the cache holds (16), then the first ones again.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -113,5 +115,68 @@ def test_argument_errors(gpu):
     assert L.bs_price_passes_f32(*p[:5], p[5], 2, out.ptr, 16, 3, None) == -1    # type width
     assert L.bs_price_passes_f32(*p[:5], p[5], 1, out.ptr, -1, 3, None) == -1    # n < 0
     assert L.bs_price_passes_f32(*p[:5], p[5], 1, out.ptr, 0, 3, None) == 0      # nothing to do
+    db.free()
+    out.free()
+
+
+@pytest.mark.parametrize("n,passes", [(63, 3), (65, 4), (1000, 5), (1 << 17, 9), ((1 << 17) + 1, 9),
+                                      (300_001, 2)])
+@pytest.mark.parametrize("type_dtype", [np.uint8, np.int32])
+def test_one_launch_of_several_passes(gpu, n, passes, type_dtype):
+    """Passes in fours and what is left of them, on both sides of the size from
+    which one is in flight at a time: the bits of a single pass."""
+    book = books.make_book(n, books.SEED_BASE + 114 + n % 83)
+    db = gpu.DeviceBook(book, type_dtype=type_dtype)
+    want = eager(gpu, db, n)
+    out = gpu.alloc_out(n)
+    passes_call(gpu, db, out, n, passes)
+    gpu.call("bs_stream_sync", None)
+    assert np.array_equal(out.download(np.float32, n).view(np.uint32), want.view(np.uint32))
+    db.free()
+    out.free()
+
+
+def test_price_over_an_input(gpu):
+    """price = the spot array: pass 2 prices the output of pass 1, as separate
+    calls do."""
+    n, passes = 5000, 3
+    book = books.make_book(n, books.SEED_BASE + 115)
+    db, ref = gpu.DeviceBook(book), gpu.DeviceBook(book)
+    p = ref.ptrs()
+    for _ in range(passes):
+        gpu.call("bs_price_f32", *p, p[0], n, None)
+    q = db.ptrs()
+    gpu.call("bs_price_passes_f32", *q, 1, q[0], n, passes, None)
+    gpu.call("bs_stream_sync", None)
+    got, want = (b.bufs[0].download(np.uint32, n) for b in (db, ref))
+    assert np.array_equal(got, want)
+    db.free()
+    ref.free()
+
+
+def test_inside_a_callers_graph(gpu):
+    """The one launch is an ordinary kernel node of a caller's capture."""
+    from test_gpu_capture import CAPTURE_THREAD_LOCAL, hip
+    H, L, n = hip(), gpu.load(), 4096
+    book = books.make_book(n, books.SEED_BASE + 116)
+    db = gpu.DeviceBook(book)
+    out = gpu.alloc_out(n)
+    want = eager(gpu, db, n)
+    st = gpu.Stream()
+    graph, gexec = ctypes.c_void_p(), ctypes.c_void_p()
+    assert H.hipStreamBeginCapture(st.handle, CAPTURE_THREAD_LOCAL) == 0
+    p = db.ptrs()
+    rc = L.bs_price_passes_f32(*p, 1, out.ptr, n, 100, st.handle)
+    assert H.hipStreamEndCapture(st.handle, ctypes.byref(graph)) == 0 and rc == 0
+    assert H.hipGraphInstantiate(ctypes.byref(gexec), graph, None, None, 0) == 0
+    for rep in range(4):
+        gpu.call("bs_memset", out.ptr, 0, n * 4, st.handle)
+        assert H.hipGraphLaunch(gexec, st.handle) == 0
+        gpu.call("bs_stream_sync", st.handle)
+        assert np.array_equal(out.download(np.float32, n).view(np.uint32), want.view(np.uint32)), rep
+        eager(gpu, db, n)
+    H.hipGraphExecDestroy(gexec)
+    H.hipGraphDestroy(graph)
+    st.destroy()
     db.free()
     out.free()
