@@ -20,10 +20,10 @@
  *     the null stream).  Functions named *_host take host pointers and are
  *     synchronous.  Pointers are validated (hipPointerGetAttributes) unless
  *     bs_config_set(BS_CFG_CHECK_POINTERS, 0).
- *   - Arrays aligned for two elements per load (8 bytes for float arrays,
- *     16 for double, 2 for uint8 types, 8 for int32 types) take the vector
- *     path; anything else the one-option-per-work-item path.  Results are
- *     identical either way.
+ *   - Arrays may start at any element.  Those that start at the same element
+ *     of their 128-byte lines (a slice [i, i + n) of a book into the same
+ *     slice of its output) run at the speed of aligned ones; arrays out of
+ *     step with one another 10-15% slower.  Results are identical either way.
  *   - Arithmetic: FP32 entry points follow the reference's float statements
  *     and its order of operations: correctly rounded division, reciprocal
  *     and square root, the double literals applied with one rounding, exp

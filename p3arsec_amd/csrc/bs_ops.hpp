@@ -2,7 +2,8 @@
 // batch map (bs_kernels.hip) and the serving loop's fused kernels
 // (bs_serve.hip), so both compute every option with the same code.
 //
-// Each op: Group (registers of one VW-option group), load<NT>(g),
+// Each op: AL (every vector store's address is a multiple of its size; loads
+// take any), Group (registers of one VW-option group), load<NT>(g),
 // finish<NT>(g, x) (compute + store; g is the group index, int64_t or, for
 // arrays under 4 GiB, uint32_t), scalar(i) for options outside whole groups,
 // kElemBytes (the widest array element, for the 4 GiB test), kLdsPerWave
@@ -40,20 +41,33 @@ using vec = T __attribute__((ext_vector_type(N)));
 template <int VW>
 using tword = typename std::conditional<VW == 4, uint32_t, uint16_t>::type;
 
+// Loads of any alignment: the same instructions as aligned ones (gfx950's vector
+// memory takes any byte address), at the cost of the lines a wave's span then
+// straddles.  Unaligned streams load through the caches (ops' NT && AL), which
+// then hold a straddled line for the wave beside it: 5M options 23.6 us, with
+// non-temporal loads 25.6.
 template <bool NT, class T>
 __device__ __forceinline__ T ld(const T* p) {
-    if constexpr (NT) return __builtin_nontemporal_load(p);
-    else return *p;
+    typedef T U __attribute__((aligned(1)));
+    const U* q = reinterpret_cast<const U*>(p);
+    if constexpr (NT) return __builtin_nontemporal_load(q);
+    else return *q;
 }
 // Streaming stores.  An 8-byte value goes out as a relaxed agent-scope atomic
 // store: the same global_store_dwordx2, with the memory model's agent-scope
 // cache policy (sc1), which on MI355X streams the outputs faster than the
 // non-temporal hint (10M options: price map on one stream 38.9 -> 37.9 us,
 // Greeks 67.9 -> 67.1 us).  Other sizes keep the non-temporal store (the FP64
-// map's 16-byte stores split in two ran 4 us slower).
-template <bool NT, class T>
+// map's 16-byte stores split in two ran 4 us slower), and so do addresses that
+// are not a multiple of the size (AL false).
+template <bool NT, bool AL, class T>
 __device__ __forceinline__ void st(T* p, T v) {
-    if constexpr (NT && sizeof(T) == 8) {
+    typedef T U __attribute__((aligned(1)));
+    if constexpr (!AL) {
+        U* q = reinterpret_cast<U*>(p);
+        if constexpr (NT) __builtin_nontemporal_store(v, q);
+        else *q = v;
+    } else if constexpr (NT && sizeof(T) == 8) {
         __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v),
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else if constexpr (NT) {
@@ -82,7 +96,7 @@ __device__ __forceinline__ bool put_of(uint32_t word, int j) {
     return ((word >> (8 * j)) & 0xffu) != 0u;
 }
 
-template <class Math, int VW>
+template <class Math, int VW, bool AL = true>
 struct PriceF32 {
     static constexpr int kVW = VW;
     static constexpr int kElemBytes = 4;   // widest array element
@@ -104,12 +118,12 @@ struct PriceF32 {
     template <bool NT, class Ix = int64_t>
     __device__ __forceinline__ Group load(Ix g) const {
         Group x;
-        x.s = ld<NT>(at(reinterpret_cast<const F*>(in.s), g));
-        x.k = ld<NT>(at(reinterpret_cast<const F*>(in.k), g));
-        x.r = ld<NT>(at(reinterpret_cast<const F*>(in.r), g));
-        x.v = ld<NT>(at(reinterpret_cast<const F*>(in.v), g));
-        x.t = ld<NT>(at(reinterpret_cast<const F*>(in.t), g));
-        x.ty = ld<NT>(at(reinterpret_cast<const tword<VW>*>(type), g));
+        x.s = ld<NT && AL>(at(reinterpret_cast<const F*>(in.s), g));
+        x.k = ld<NT && AL>(at(reinterpret_cast<const F*>(in.k), g));
+        x.r = ld<NT && AL>(at(reinterpret_cast<const F*>(in.r), g));
+        x.v = ld<NT && AL>(at(reinterpret_cast<const F*>(in.v), g));
+        x.t = ld<NT && AL>(at(reinterpret_cast<const F*>(in.t), g));
+        x.ty = ld<NT && AL>(at(reinterpret_cast<const tword<VW>*>(type), g));
         return x;
     }
     template <bool NT, class Ix = int64_t>
@@ -118,14 +132,14 @@ struct PriceF32 {
 #pragma unroll
         for (int j = 0; j < VW; ++j)
             p[j] = bs_price<Math>(x.s[j], x.k[j], x.r[j], x.v[j], x.t[j], put_of(x.ty, j));
-        st<NT>(at(reinterpret_cast<F*>(out), g), p);
+        st<NT, AL>(at(reinterpret_cast<F*>(out), g), p);
     }
     __device__ __forceinline__ void scalar(int64_t i) const {
         out[i] = bs_price<Math>(in.s[i], in.k[i], in.r[i], in.v[i], in.t[i], type[i] != 0);
     }
 };
 
-template <int VW>
+template <int VW, bool AL = true>
 struct PriceI32F32 {
     static constexpr int kVW = VW;
     static constexpr int kElemBytes = 4;   // widest array element
@@ -146,12 +160,12 @@ struct PriceI32F32 {
     template <bool NT, class Ix = int64_t>
     __device__ __forceinline__ Group load(Ix g) const {
         Group x;
-        x.s = ld<NT>(at(reinterpret_cast<const F*>(in.s), g));
-        x.k = ld<NT>(at(reinterpret_cast<const F*>(in.k), g));
-        x.r = ld<NT>(at(reinterpret_cast<const F*>(in.r), g));
-        x.v = ld<NT>(at(reinterpret_cast<const F*>(in.v), g));
-        x.t = ld<NT>(at(reinterpret_cast<const F*>(in.t), g));
-        x.ty = ld<NT>(at(reinterpret_cast<const I*>(type), g));
+        x.s = ld<NT && AL>(at(reinterpret_cast<const F*>(in.s), g));
+        x.k = ld<NT && AL>(at(reinterpret_cast<const F*>(in.k), g));
+        x.r = ld<NT && AL>(at(reinterpret_cast<const F*>(in.r), g));
+        x.v = ld<NT && AL>(at(reinterpret_cast<const F*>(in.v), g));
+        x.t = ld<NT && AL>(at(reinterpret_cast<const F*>(in.t), g));
+        x.ty = ld<NT && AL>(at(reinterpret_cast<const I*>(type), g));
         return x;
     }
     template <bool NT, class Ix = int64_t>
@@ -160,7 +174,7 @@ struct PriceI32F32 {
 #pragma unroll
         for (int j = 0; j < VW; ++j)
             p[j] = bs_price<Ref32>(x.s[j], x.k[j], x.r[j], x.v[j], x.t[j], x.ty[j] != 0);
-        st<NT>(at(reinterpret_cast<F*>(out), g), p);
+        st<NT, AL>(at(reinterpret_cast<F*>(out), g), p);
     }
     __device__ __forceinline__ void scalar(int64_t i) const {
         out[i] = bs_price<Ref32>(in.s[i], in.k[i], in.r[i], in.v[i], in.t[i], type[i] != 0);
@@ -168,7 +182,7 @@ struct PriceI32F32 {
 };
 
 // fptype = double: a group is VW = 2 options (one 128-bit load per array).
-template <int VW>
+template <int VW, bool AL = true>
 struct PriceF64 {
     static constexpr int kVW = 2;
     static constexpr int kElemBytes = 8;   // widest array element
@@ -188,12 +202,12 @@ struct PriceF64 {
     template <bool NT, class Ix = int64_t>
     __device__ __forceinline__ Group load(Ix g) const {
         Group x;
-        x.s = ld<NT>(at(reinterpret_cast<const D*>(in.s), g));
-        x.k = ld<NT>(at(reinterpret_cast<const D*>(in.k), g));
-        x.r = ld<NT>(at(reinterpret_cast<const D*>(in.r), g));
-        x.v = ld<NT>(at(reinterpret_cast<const D*>(in.v), g));
-        x.t = ld<NT>(at(reinterpret_cast<const D*>(in.t), g));
-        x.ty = ld<NT>(at(reinterpret_cast<const uint16_t*>(type), g));
+        x.s = ld<NT && AL>(at(reinterpret_cast<const D*>(in.s), g));
+        x.k = ld<NT && AL>(at(reinterpret_cast<const D*>(in.k), g));
+        x.r = ld<NT && AL>(at(reinterpret_cast<const D*>(in.r), g));
+        x.v = ld<NT && AL>(at(reinterpret_cast<const D*>(in.v), g));
+        x.t = ld<NT && AL>(at(reinterpret_cast<const D*>(in.t), g));
+        x.ty = ld<NT && AL>(at(reinterpret_cast<const uint16_t*>(type), g));
         return x;
     }
     template <bool NT, class Ix = int64_t>
@@ -202,14 +216,14 @@ struct PriceF64 {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
             p[j] = bs_price<Ref64>(x.s[j], x.k[j], x.r[j], x.v[j], x.t[j], put_of(x.ty, j));
-        st<NT>(at(reinterpret_cast<D*>(out), g), p);
+        st<NT, AL>(at(reinterpret_cast<D*>(out), g), p);
     }
     __device__ __forceinline__ void scalar(int64_t i) const {
         out[i] = bs_price<Ref64>(in.s[i], in.k[i], in.r[i], in.v[i], in.t[i], type[i] != 0);
     }
 };
 
-template <int VW>
+template <int VW, bool AL = true>
 struct GreeksF32 {
     static constexpr int kVW = VW;
     static constexpr int kElemBytes = 4;   // widest array element
@@ -230,12 +244,12 @@ struct GreeksF32 {
     template <bool NT, class Ix = int64_t>
     __device__ __forceinline__ Group load(Ix g) const {
         Group x;
-        x.s = ld<NT>(at(reinterpret_cast<const F*>(in.s), g));
-        x.k = ld<NT>(at(reinterpret_cast<const F*>(in.k), g));
-        x.r = ld<NT>(at(reinterpret_cast<const F*>(in.r), g));
-        x.v = ld<NT>(at(reinterpret_cast<const F*>(in.v), g));
-        x.t = ld<NT>(at(reinterpret_cast<const F*>(in.t), g));
-        x.ty = ld<NT>(at(reinterpret_cast<const tword<VW>*>(type), g));
+        x.s = ld<NT && AL>(at(reinterpret_cast<const F*>(in.s), g));
+        x.k = ld<NT && AL>(at(reinterpret_cast<const F*>(in.k), g));
+        x.r = ld<NT && AL>(at(reinterpret_cast<const F*>(in.r), g));
+        x.v = ld<NT && AL>(at(reinterpret_cast<const F*>(in.v), g));
+        x.t = ld<NT && AL>(at(reinterpret_cast<const F*>(in.t), g));
+        x.ty = ld<NT && AL>(at(reinterpret_cast<const tword<VW>*>(type), g));
         return x;
     }
     template <bool NT, class Ix = int64_t>
@@ -251,11 +265,11 @@ struct GreeksF32 {
             rh[j] = o.rho;
             th[j] = o.theta;
         }
-        st<NT>(at(reinterpret_cast<F*>(out.price), g), p);
-        st<NT>(at(reinterpret_cast<F*>(out.delta), g), d);
-        st<NT>(at(reinterpret_cast<F*>(out.vega), g), ve);
-        st<NT>(at(reinterpret_cast<F*>(out.rho), g), rh);
-        st<NT>(at(reinterpret_cast<F*>(out.theta), g), th);
+        st<NT, AL>(at(reinterpret_cast<F*>(out.price), g), p);
+        st<NT, AL>(at(reinterpret_cast<F*>(out.delta), g), d);
+        st<NT, AL>(at(reinterpret_cast<F*>(out.vega), g), ve);
+        st<NT, AL>(at(reinterpret_cast<F*>(out.rho), g), rh);
+        st<NT, AL>(at(reinterpret_cast<F*>(out.theta), g), th);
     }
     __device__ __forceinline__ void scalar(int64_t i) const {
         const Greeks32 o = bs_greeks<Ref32>(in.s[i], in.k[i], in.r[i], in.v[i], in.t[i],
@@ -268,7 +282,7 @@ struct GreeksF32 {
     }
 };
 
-template <int VW>
+template <int VW, bool AL = true>
 struct CndfF32 {
     static constexpr int kVW = VW;
     static constexpr int kElemBytes = 4;   // widest array element
@@ -285,21 +299,21 @@ struct CndfF32 {
     };
     template <bool NT, class Ix = int64_t>
     __device__ __forceinline__ Group load(Ix g) const {
-        return Group{ld<NT>(at(reinterpret_cast<const F*>(x), g))};
+        return Group{ld<NT && AL>(at(reinterpret_cast<const F*>(x), g))};
     }
     template <bool NT, class Ix = int64_t>
     __device__ __forceinline__ void finish(Ix g, const Group& a) const {
         F y;
 #pragma unroll
         for (int j = 0; j < VW; ++j) y[j] = Ref32::cndf<false>(a.x[j], nullptr);
-        st<NT>(at(reinterpret_cast<F*>(out), g), y);
+        st<NT, AL>(at(reinterpret_cast<F*>(out), g), y);
     }
     __device__ __forceinline__ void scalar(int64_t i) const {
         out[i] = Ref32::cndf<false>(x[i], nullptr);
     }
 };
 
-template <int VW>
+template <int VW, bool AL = true>
 struct CndfF64 {
     static constexpr int kVW = 2;
     static constexpr int kElemBytes = 8;   // widest array element
@@ -316,14 +330,14 @@ struct CndfF64 {
     };
     template <bool NT, class Ix = int64_t>
     __device__ __forceinline__ Group load(Ix g) const {
-        return Group{ld<NT>(at(reinterpret_cast<const D*>(x), g))};
+        return Group{ld<NT && AL>(at(reinterpret_cast<const D*>(x), g))};
     }
     template <bool NT, class Ix = int64_t>
     __device__ __forceinline__ void finish(Ix g, const Group& a) const {
         D y;
         y[0] = Ref64::cndf<false>(a.x[0], nullptr);
         y[1] = Ref64::cndf<false>(a.x[1], nullptr);
-        st<NT>(at(reinterpret_cast<D*>(out), g), y);
+        st<NT, AL>(at(reinterpret_cast<D*>(out), g), y);
     }
     __device__ __forceinline__ void scalar(int64_t i) const {
         out[i] = Ref64::cndf<false>(x[i], nullptr);

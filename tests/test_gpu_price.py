@@ -296,3 +296,47 @@ def test_fp64_primitives_against_the_c_library(gpu):
     p = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     print("\n" + p.stdout.strip())
     assert p.returncode == 0, p.stdout + p.stderr
+
+
+def _shifted(capi, book, n, pads, dtype=np.float32, type_dtype=np.uint8):
+    """Device arrays of book's first n options, array j starting pads[j]
+    elements into its buffer: (buffers, pointers)."""
+    bufs, ptrs = [], []
+    for a, pad in zip(book.arrays(), pads):
+        dt = np.dtype(type_dtype if a is book.otype else dtype)
+        b = capi.DeviceBuffer.from_array(np.concatenate([np.zeros(pad, dt), a[:n].astype(dt)]))
+        bufs.append(b)
+        ptrs.append(b.ptr + pad * dt.itemsize)
+    return bufs, ptrs
+
+
+@pytest.mark.parametrize("n", [1, 2, 5, 31, 33, 64, 129, 1000, 4099])
+@pytest.mark.parametrize("pads,out_pad", [
+    ((3,) * 6, 3),                    # a slice: every array starts at the same option
+    ((31,) * 6, 31), ((32,) * 6, 32), ((2,) * 6, 2), ((16,) * 6, 16),
+    ((3,) * 6, 0), ((0,) * 6, 3),     # inputs and output out of step
+    ((0, 1, 2, 3, 4, 5), 7), ((8, 8, 8, 8, 8, 1), 8),
+])
+def test_slices_give_the_same_bits(gpu, n, pads, out_pad):
+    """Every start of every array: the bits of the aligned book, and nothing
+    written outside [0, n)."""
+    book = books.make_book(n, books.SEED_BASE + 60 + n % 31)
+    for fn, tdt, dt, k in (("bs_price_f32", np.uint8, np.float32, 1),
+                           ("bs_price_i32type_f32", np.int32, np.float32, 1),
+                           ("bs_price_fast_f32", np.uint8, np.float32, 1),
+                           ("bs_price_f64", np.uint8, np.float64, 1),
+                           ("bs_price_greeks_f32", np.uint8, np.float32, 5)):
+        got = []
+        for p, op in (((0,) * 6, 0), (pads, out_pad)):
+            bufs, ptrs = _shifted(gpu, book, n, p, dt, tdt)
+            size = np.dtype(dt).itemsize
+            outs = [gpu.DeviceBuffer.from_array(np.full(op + n + 40, 7.25, dt)) for _ in range(k)]
+            gpu.call(fn, *ptrs, *[o.ptr + op * size for o in outs], n, None)
+            gpu.call("bs_stream_sync", None)
+            for o in outs:
+                a = o.download(dt, op + n + 40)
+                assert np.all(a[:op] == 7.25) and np.all(a[op + n:] == 7.25), (fn, p)
+                got.append(a[op:op + n].tobytes())
+            for b in bufs + outs:
+                b.free()
+        assert got[:k] == got[k:], (fn, n, pads)
