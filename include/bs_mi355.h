@@ -150,8 +150,12 @@ int bs_price_greeks_f32(const float *s, const float *k, const float *r, const fl
  * each per-option value exactly the one bs_price_f32 / bs_price_greeks_f32
  * computes.  weights may be NULL (every w_i = 1).  sums is a device array of 1
  * or 5 doubles.  Summed in FP64 in a fixed order: bit-reproducible for a given
- * n.  n == 0 writes zeros.  No reference counterpart: the MapReduce step that
- * follows the map (SkePU2 MapReduce, skepu2/backend/impl/mapreduce/). */
+ * n, wherever the arrays start.  n == 0 writes zeros.  Calls on different
+ * threads and streams are independent: each takes one of the library's 32
+ * scratch slots (12 MB on each device), or stream-ordered memory when none is
+ * free or the stream is being captured.  No reference counterpart: the
+ * MapReduce step that follows the map (SkePU2 MapReduce,
+ * skepu2/backend/impl/mapreduce/). */
 int bs_portfolio_f32(const float *s, const float *k, const float *r, const float *v,
                      const float *t, const uint8_t *otype, const float *weights, int64_t n,
                      int greeks, double *sums, bs_stream_t stream);
@@ -161,8 +165,8 @@ int bs_portfolio_f32(const float *s, const float *k, const float *r, const float
  * capture, serving loops and harnesses that forbid hipMalloc).  The same
  * arguments, checks and sums, bit for bit, for n <= 2^25 options
  * (BS_ERR_INVALID past that); the partial sums live in a fixed device array
- * of the library (2.6 MB on each device it runs on, held until the process
- * ends) instead of stream-ordered memory.  Calls that overlap on one device
+ * of the library (0.3 MB on each device it runs on, held until the process
+ * ends) instead of scratch that calls share out.  Calls that overlap on one device
  * share that array and race: issue them on one stream, or let one finish
  * before the next starts. */
 int bs_portfolio_f32_noalloc(const float *s, const float *k, const float *r, const float *v,

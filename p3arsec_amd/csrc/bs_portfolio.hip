@@ -6,26 +6,35 @@
 // the map computes (the same per-option code, bs_math.hpp) and w_i is the
 // position (1 when no weights are given).
 //
-// Two kernels on the caller's stream.  k_pf_rows: wave w of the grid owns
-// kPfRows consecutive rows of 64 two-option groups (the map's loads: one
-// 8-byte load per array per lane, so each wave instruction reads 512
-// contiguous bytes); a lane walks its column of those rows in order, the next
-// row's loads issued before the current row's arithmetic, and adds w*value to
-// FP64 accumulators; the wave then folds its lanes with a fixed butterfly into
-// one partial.  k_pf_final: one block of 1024 work-items adds the partials
-// (work-item j takes partials j, j + 1024, ... in order, then a fixed tree);
-// past 65536 partials (books over 2^29 options), k_pf_chunks blocks first add
-// contiguous chunks of 2048.  Every grid depends only on n, so the sums are
-// bit-reproducible for a given book.
+// One kernel on the caller's stream, k_pf_rows: a block owns `rows` consecutive
+// rows of 256 two-option groups (the map's loads: one 8-byte load per array per
+// lane, so each wave instruction reads 512 contiguous bytes), wave w of it the
+// w-th run of `rows` rows of 64; a lane walks its column of those rows in order,
+// the next row's loads issued before the current row's arithmetic, and adds
+// w*value to FP64 accumulators; each wave folds its lanes with a fixed
+// wave sum and the block its waves in order into one partial.  The last block
+// of every 64 to arrive folds their partials with one wave sum, and the last
+// of those folds the groups of 64: no second launch, and nothing waits.  The
+// shape of the sum depends only on n, so the sums are bit-reproducible for a
+// given book, wherever its arrays start.
 //
-// Scratch (the partials and the chunk sums): bs_portfolio_f32 takes it from
-// stream-ordered memory (hipMallocAsync/hipFreeAsync), so calls on different
-// streams never share it; bs_portfolio_f32_noalloc uses a fixed device array
-// of this file (g_pf_scratch) and allocates nothing.
+// A partial goes out as relaxed agent-scope stores (written through to memory,
+// past the L2 of the block's die), the wave waits for their acknowledgement,
+// then counts itself in with a relaxed agent-scope add; the block that counts
+// last loads the partials at the same scope.  A release fence in place of the
+// wait would write back the die's whole L2 for every block.
+//
+// Scratch (counters and partials): slots of a fixed device array, claimed on
+// the host by a flag in pinned memory that the kernel's last block clears, so
+// calls on any threads and streams never share one.  With no slot free, and
+// under stream capture (a graph may be replayed at any time), the partials go
+// to stream-ordered memory and a second launch, k_pf_final, adds them in the
+// same order; bs_portfolio_f32_noalloc does the same with an array of its own.
 //
 // Traffic: 21 bytes per option read (25 with weights), 8 or 40 bytes written
-// in all, plus 8 or 40 bytes of partials per kPfRows x 128 options.
+// in all, plus 8 or 40 bytes per block.
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -36,20 +45,32 @@
 namespace bs {
 namespace {
 
-constexpr int kPfRows = 8;                                      // rows of 64 groups per wave
-// LDS reserved per wave (caps the resident waves): price form none, Greeks
-// form 8 KB (20 waves per CU; 10M options 46.0 us against 47.9 with none)
-constexpr int pf_lds_per_wave(bool greeks) { return greeks ? 8192 : 0; }
-constexpr int kPfChunkThreads = 256;
-constexpr int kPfChunkPer = 8;                                  // partials per work-item
-constexpr int64_t kPfChunk = kPfChunkThreads * kPfChunkPer;     // partials per chunk block
+constexpr int kPfThreads = 256;
+constexpr int kPfWaves = kPfThreads / 64;
+constexpr int kPfGroup = 64;            // blocks per group of partials
+constexpr int64_t kPfMaxBlocks = 8192;  // 128 groups: two per lane of the last fold
+constexpr int kPfMaxGroups = kPfMaxBlocks / kPfGroup;
 
 struct PfArgs {
     SoaIn<float> in;
     const uint8_t* type;
     const float* w;   // NULL: every weight is 1
     int64_t n;
-    double* partial;  // [waves][NQ]
+    int64_t rows;     // rows of 64 groups per wave
+    double* partial;  // [blocks][NQ]
+};
+
+// A call's scratch in the one-launch form; the counters are zero between calls,
+// 256 bytes apart: adds from all dies to one line take turns, about 25 ns each.
+struct PfCounter {
+    uint32_t done;
+    uint32_t pad[63];
+};
+struct PfSlot {
+    PfCounter groups;
+    PfCounter blocks[kPfMaxGroups];
+    double group[kPfMaxGroups * 5];
+    double partial[kPfMaxBlocks * 5];
 };
 
 template <bool kGreeks>
@@ -68,270 +89,401 @@ __device__ __forceinline__ void add_option(double* acc, float s, float k, float 
     }
 }
 
-// One group's inputs: VW = 2 options of aligned arrays (8-byte loads), or
-// VW = 1 option of any alignment.  Ix = uint32_t when every array of the call
-// spans less than 4 GiB (32-bit offsets on the arrays' bases), else int64_t.
-template <int VW>
-struct PfGroup {
-    using F = vec<float, VW>;
-    F s, k, r, v, t, w;
+// One group's inputs.  Ix = uint32_t when every array of the call spans less
+// than 4 GiB (32-bit offsets on the arrays' bases), else int64_t.  AL false:
+// some array is not aligned for two options (cached loads, as in the maps).
+using F2 = vec<float, 2>;
+struct PfOptions {
+    F2 s, k, r, v, t, w;
     uint32_t ty;
 };
 
-template <int VW, class Ix>
-__device__ __forceinline__ PfGroup<VW> pf_load(const PfArgs& a, Ix g) {
-    using F = vec<float, VW>;
-    PfGroup<VW> x;
-    x.s = __builtin_nontemporal_load(at(reinterpret_cast<const F*>(a.in.s), g));
-    x.k = __builtin_nontemporal_load(at(reinterpret_cast<const F*>(a.in.k), g));
-    x.r = __builtin_nontemporal_load(at(reinterpret_cast<const F*>(a.in.r), g));
-    x.v = __builtin_nontemporal_load(at(reinterpret_cast<const F*>(a.in.v), g));
-    x.t = __builtin_nontemporal_load(at(reinterpret_cast<const F*>(a.in.t), g));
-    if constexpr (VW == 2)
-        x.ty = __builtin_nontemporal_load(at(reinterpret_cast<const uint16_t*>(a.type), g));
-    else
-        x.ty = __builtin_nontemporal_load(at(a.type, g));
-    if (a.w) x.w = __builtin_nontemporal_load(at(reinterpret_cast<const F*>(a.w), g));
-    else x.w = F(1.0f);
+template <bool AL, class Ix>
+__device__ __forceinline__ PfOptions pf_load(const PfArgs& a, Ix g) {
+    PfOptions x;
+    x.s = ld<AL>(at(reinterpret_cast<const F2*>(a.in.s), g));
+    x.k = ld<AL>(at(reinterpret_cast<const F2*>(a.in.k), g));
+    x.r = ld<AL>(at(reinterpret_cast<const F2*>(a.in.r), g));
+    x.v = ld<AL>(at(reinterpret_cast<const F2*>(a.in.v), g));
+    x.t = ld<AL>(at(reinterpret_cast<const F2*>(a.in.t), g));
+    x.ty = ld<AL>(at(reinterpret_cast<const uint16_t*>(a.type), g));
+    if (a.w) x.w = ld<AL>(at(reinterpret_cast<const F2*>(a.w), g));
+    else x.w = F2(1.0f);
     return x;
 }
 
-template <int VW, bool kGreeks>
-__device__ __forceinline__ void pf_add(double* acc, const PfGroup<VW>& x) {
+template <bool kGreeks>
+__device__ __forceinline__ void pf_add(double* acc, const PfOptions& x) {
 #pragma unroll
-    for (int j = 0; j < VW; ++j)
+    for (int j = 0; j < 2; ++j)
         add_option<kGreeks>(acc, x.s[j], x.k[j], x.r[j], x.v[j], x.t[j], put_of(x.ty, j), x.w[j]);
 }
 
-// Groups of the call: n / VW whole groups, plus (VW = 2, n odd) the last
-// option alone, priced by the lane that would own group n / 2.
-template <int VW, bool kGreeks, int NT, class Ix>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kGreeks ? 4 : 5)))
-void k_pf_rows(PfArgs a) {
+// x moved across lanes by a DPP control; lanes it does not reach, and rows
+// outside `rows`, give 0.
+template <int kControl, int kRows>
+__device__ __forceinline__ double dpp(double x) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), kControl, kRows, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), kControl, kRows, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// The wave's sum, in every lane: within rows of 16 lanes (shifts right by 1, 2,
+// 4, 8), then row totals into the next rows (broadcasts of lanes 15 and 31).
+// Three VALU instructions a step; through LDS (__shfl_xor) the five folds of a
+// wave cost as much as two of its options.
+__device__ __forceinline__ double wave_sum(double x) {
+    x += dpp<0x111, 0xf>(x);
+    x += dpp<0x112, 0xf>(x);
+    x += dpp<0x114, 0xf>(x);
+    x += dpp<0x118, 0xf>(x);
+    x += dpp<0x142, 0xa>(x);
+    x += dpp<0x143, 0xc>(x);
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
+                            __builtin_amdgcn_readlane(__double2loint(x), 63));
+}
+
+template <class T>
+__device__ __forceinline__ T agent_load(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void agent_store(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Waits until this wave's stores have been acknowledged.
+__device__ __forceinline__ void stores_done() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// Counts this wave in; true in the one that makes `full`.
+__device__ __forceinline__ bool arrive(uint32_t* counter, uint32_t full) {
+    uint32_t before = 0;
+    if ((threadIdx.x & 63) == 0)
+        before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)before) == full - 1;
+}
+
+// One wave's sums of NQ quantities: of group g's partials, and of the groups'.
+// load(i, q) gives quantity q of partial (group) i; both launch forms fold in
+// these shapes.
+template <int NQ, class Load>
+__device__ __forceinline__ void fold_blocks(int g, int blocks, int lane, double (&x)[NQ],
+                                            Load&& load) {
+    const int b = g * kPfGroup + lane;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) x[q] = b < blocks ? load(b, q) : 0.0;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) x[q] = wave_sum(x[q]);
+}
+template <int NQ, class Load>
+__device__ __forceinline__ void fold_groups(int groups, int lane, double (&x)[NQ], Load&& load) {
+    double hi[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        x[q] = lane < groups ? load(lane, q) : 0.0;
+        hi[q] = lane + 64 < groups ? load(lane + 64, q) : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) x[q] = wave_sum(x[q] + hi[q]);
+}
+
+// x[q] for q = lane, the same for every lane past NQ.
+template <int NQ>
+__device__ __forceinline__ double pick(const double (&x)[NQ], int lane) {
+    double v = x[0];
+#pragma unroll
+    for (int q = 1; q < NQ; ++q) v = lane == q ? x[q] : v;
+    return v;
+}
+
+// slot: the one-launch form's scratch, its host flag and the sums' place; NULL
+// leaves the partials in a.partial for k_pf_final.
+template <bool kGreeks, bool AL, class Ix>
+__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(kGreeks ? 4 : 5)))
+void k_pf_rows(PfArgs a, PfSlot* slot, uint32_t* busy, double* __restrict__ sums) {
     constexpr int NQ = kGreeks ? 5 : 1;
     double acc[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
-    const Ix ngroups = (Ix)(VW == 2 ? a.n / 2 : a.n);
-    const Ix lane = threadIdx.x & 63;
-    const Ix wave = (Ix)blockIdx.x * (NT / 64) + threadIdx.x / 64;
-    Ix g = wave * (64 * kPfRows) + lane;
-    const Ix g_end = g + 64 * kPfRows;
+    const Ix ngroups = (Ix)(a.n / 2);
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x / 64;
+    const Ix span = (Ix)a.rows * 64;
+    Ix g = ((Ix)blockIdx.x * kPfWaves + wave) * span + lane;
+    const Ix g_end = g + span;
     if (g < ngroups) {
-        PfGroup<VW> cur = pf_load<VW>(a, g);
+        PfOptions cur = pf_load<AL>(a, g);
         for (Ix gn = g + 64; gn < g_end && gn < ngroups; gn += 64) {
-            const PfGroup<VW> nxt = pf_load<VW>(a, gn);
-            pf_add<VW, kGreeks>(acc, cur);
+            const PfOptions nxt = pf_load<AL>(a, gn);
+            pf_add<kGreeks>(acc, cur);
             cur = nxt;
             g = gn;
         }
-        pf_add<VW, kGreeks>(acc, cur);
+        pf_add<kGreeks>(acc, cur);
         g += 64;
     }
-    if (VW == 2 && (a.n & 1) && g == ngroups && g < g_end) {   // the last option of an odd book
+    if ((a.n & 1) && g == ngroups && g < g_end) {   // the last option of an odd book
         const int64_t i = a.n - 1;
         add_option<kGreeks>(acc, a.in.s[i], a.in.k[i], a.in.r[i], a.in.v[i], a.in.t[i],
                             a.type[i] != 0, a.w ? a.w[i] : 1.0f);
     }
+    __shared__ double lds[kPfWaves][NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        double x = acc[q];
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, 64);
-        if (lane == 0) a.partial[(int64_t)wave * NQ + q] = x;
-    }
-}
-
-// Block b sums partials [b*kPfChunk, (b+1)*kPfChunk) (clipped to count): each
-// work-item adds its eight (stride kPfChunkThreads, all loads issued first) in
-// order, then a fixed tree over the block; out[b] is the chunk's sum.
-template <int NQ>
-__global__ __launch_bounds__(kPfChunkThreads) void k_pf_chunks(const double* __restrict__ in,
-                                                               int64_t count,
-                                                               double* __restrict__ out) {
-    __shared__ double lds[NQ][kPfChunkThreads];
-    const int64_t base = (int64_t)blockIdx.x * kPfChunk + threadIdx.x;
-    double v[kPfChunkPer][NQ];
-#pragma unroll
-    for (int j = 0; j < kPfChunkPer; ++j) {
-        const int64_t i = base + (int64_t)j * kPfChunkThreads;
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) v[j][q] = i < count ? in[i * NQ + q] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        double acc = v[0][q];
-#pragma unroll
-        for (int j = 1; j < kPfChunkPer; ++j) acc += v[j][q];
-        lds[q][threadIdx.x] = acc;
+        const double x = wave_sum(acc[q]);
+        if (lane == 0) lds[wave][q] = x;
     }
     __syncthreads();
-    for (int half = kPfChunkThreads / 2; half >= 1; half >>= 1) {
-        if ((int)threadIdx.x < half)
+    if (wave != 0) return;
+    if (lane < NQ) {
+        double v = lds[0][lane];
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) lds[q][threadIdx.x] += lds[q][threadIdx.x + half];
-        __syncthreads();
+        for (int w = 1; w < kPfWaves; ++w) v += lds[w][lane];
+        agent_store(a.partial + (int64_t)blockIdx.x * NQ + lane, v);
     }
-    if (threadIdx.x < NQ) out[(int64_t)blockIdx.x * NQ + threadIdx.x] = lds[threadIdx.x][0];
+    if (!slot) return;
+    stores_done();
+    const int blocks = gridDim.x, groups = (blocks + kPfGroup - 1) / kPfGroup;
+    const int gr = blockIdx.x / kPfGroup;
+    if (!arrive(&slot->blocks[gr].done, min(kPfGroup, blocks - gr * kPfGroup))) return;
+    double x[NQ];
+    fold_blocks(gr, blocks, lane, x, [&](int b, int q) {
+        return agent_load(a.partial + (int64_t)b * NQ + q);
+    });
+    if (lane < NQ) agent_store(&slot->group[gr * NQ + lane], pick(x, lane));
+    if (lane == 0) agent_store(&slot->blocks[gr].done, 0u);
+    stores_done();
+    if (!arrive(&slot->groups.done, groups)) return;
+    fold_groups(groups, lane, x, [&](int i, int q) { return agent_load(&slot->group[i * NQ + q]); });
+    if (lane < NQ) sums[lane] = pick(x, lane);
+    if (lane == 0) agent_store(&slot->groups.done, 0u);
+    stores_done();
+    if (lane == 0) __hip_atomic_store(busy, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// One block sums count <= kPfFinalMax partials: work-item j adds partials j,
-// j + 1024, j + 2048, ... in order, then a fixed tree over the block.
+// The second launch of the two-launch form: one block folds the partials, a
+// wave per group up to 16.
 constexpr int kPfFinalThreads = 1024;
-constexpr int64_t kPfFinalMax = int64_t(kPfFinalThreads) * 64;
 
 template <int NQ>
 __global__ __launch_bounds__(kPfFinalThreads) void k_pf_final(const double* __restrict__ in,
-                                                              int64_t count,
+                                                              int blocks,
                                                               double* __restrict__ out) {
-    __shared__ double lds[NQ][kPfFinalThreads];
-    double acc[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
-    for (int64_t i = threadIdx.x; i < count; i += kPfFinalThreads)
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) acc[q] += in[i * NQ + q];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) lds[q][threadIdx.x] = acc[q];
+    __shared__ double lds[kPfMaxGroups][NQ];
+    const int lane = threadIdx.x & 63;
+    const int groups = (blocks + kPfGroup - 1) / kPfGroup;
+    double x[NQ];
+    for (int g = threadIdx.x / 64; g < groups; g += (int)blockDim.x / 64) {
+        fold_blocks(g, blocks, lane, x, [&](int b, int q) { return in[(int64_t)b * NQ + q]; });
+        if (lane < NQ) lds[g][lane] = pick(x, lane);
+    }
     __syncthreads();
-    for (int half = kPfFinalThreads / 2; half >= 1; half >>= 1) {
-        if ((int)threadIdx.x < half)
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) lds[q][threadIdx.x] += lds[q][threadIdx.x + half];
-        __syncthreads();
-    }
-    if (threadIdx.x < NQ) out[threadIdx.x] = lds[threadIdx.x][0];
+    if (threadIdx.x >= 64) return;
+    fold_groups(groups, lane, x, [&](int i, int q) { return lds[i][q]; });
+    if (lane < NQ) out[lane] = pick(x, lane);
 }
 
-// Reduces count partials (count >= 1) to out[0..NQ) in a fixed order: chunk
-// sums while more than kPfFinalMax are left, then one final block.  tmp holds
-// ceil(count / kPfChunk) entries per chunk level (pf_scratch_doubles counts
-// them).
-template <int NQ>
-void reduce_partials(const double* in, int64_t count, double* tmp, double* out, hipStream_t st) {
-    while (count > kPfFinalMax) {
-        const int64_t nb = (count + kPfChunk - 1) / kPfChunk;
-        hipLaunchKernelGGL((k_pf_chunks<NQ>), dim3((unsigned)nb), dim3(kPfChunkThreads), 0, st,
-                           in, count, tmp);
-        in = tmp;
-        tmp += nb * NQ;
-        count = nb;
-    }
-    hipLaunchKernelGGL((k_pf_final<NQ>), dim3(1), dim3(kPfFinalThreads), 0, st, in, count, out);
+// Rows per wave: one while that makes fewer than pf_spread blocks, so that a
+// small book spreads over the chip; then up to the form's most, which keeps the
+// blocks' counting in rare against their options; more only to stay within
+// kPfMaxBlocks.  10M options: price sums 38.8 us with at most 2 rows, 39.0 with
+// 4, 42 with 8, 44 with 16; Greeks and weights 54.9 with 4 and 8, 56 with 16.
+//
+// The whole call, against one wave per 8 rows and one final block in two
+// launches with stream-ordered scratch: 65,537 options 5.9 us and 23.4 (the
+// host's allocation); 1M 8.6 and 25, with Greeks 13.6 and 25; 10M 39.0 and
+// 47.1, with Greeks and weights 54.9 and 61 (the final block alone 8.8).
+// Bound by HBM (price) and VALU issue (Greeks).
+// One-row blocks that spread a book far enough: with 512 for the Greeks form, the
+// two-launch sums of 1M options take 12.2 us, with 1024 13.7.
+constexpr int64_t pf_spread(bool greeks) { return greeks ? 512 : 1024; }
+constexpr int64_t pf_most_rows(bool greeks) { return greeks ? 8 : 4; }
+
+struct PfShape {
+    int64_t rows, blocks;
+};
+constexpr PfShape pf_shape(int64_t n, bool greeks) {
+    const int64_t items = n / 2 + (n & 1);
+    auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+    int64_t rows = std::min(pf_most_rows(greeks), std::max<int64_t>(1, items / (kPfThreads * pf_spread(greeks))));
+    rows = std::max(rows, up(items, kPfThreads * kPfMaxBlocks));
+    return {rows, std::max<int64_t>(1, up(items, kPfThreads * rows))};
 }
 
-constexpr int pf_threads(bool greeks) { return greeks ? 256 : 64; }
-
-// Waves of k_pf_rows for n options (VW-option groups plus the odd tail).
-constexpr int64_t pf_waves(int64_t n, int vw) {
-    const int64_t items = vw == 2 ? n / 2 + (n & 1) : n;
-    int64_t waves = (items + 64 * kPfRows - 1) / (64 * kPfRows);
-    return waves < 1 ? 1 : waves;
-}
-
-// Doubles of scratch one call needs: the partials (whole blocks of waves) and
-// every level of chunk sums.
-constexpr int64_t pf_scratch_doubles(int64_t n, int vw, bool greeks) {
-    const int nq = greeks ? 5 : 1;
-    const int64_t wpb = pf_threads(greeks) / 64;
-    const int64_t waves = (pf_waves(n, vw) + wpb - 1) / wpb * wpb;
-    int64_t room = waves, level = waves;
-    while (level > kPfFinalMax) {
-        level = (level + kPfChunk - 1) / kPfChunk;
-        room += level;
-    }
-    return room * nq;
-}
-
-template <int VW, bool kGreeks>
-hipError_t launch_pf(const PfArgs& a, double* sums, hipStream_t st) {
-    constexpr int NQ = kGreeks ? 5 : 1;
-    constexpr int NT = pf_threads(kGreeks);
-    constexpr int64_t wpb = NT / 64;
-    const int64_t waves = pf_waves(a.n, VW);
-    const int64_t nb = (waves + wpb - 1) / wpb;
-    if (nb > 0x7fffffff) return hipErrorInvalidValue;
-    // LDS reserved per block caps the waves resident on a CU (none is used)
+// slot NULL: the two-launch form with a.partial.
+template <bool kGreeks, bool AL>
+hipError_t launch_pf(PfArgs a, PfSlot* slot, uint32_t* busy, double* sums, hipStream_t st) {
+    const PfShape shape = pf_shape(a.n, kGreeks);
+    a.rows = shape.rows;
+    if (slot) a.partial = slot->partial;
+    // LDS reserved per block caps the waves resident on a CU: none by default
+    // (a block holds its LDS while its last wave counts it in: 10M options with
+    // Greeks and weights took 57.8 us with 8 KB per wave and 56.2 with none)
     const int lw = config().lds_per_wave.load(std::memory_order_relaxed);
-    const size_t lds =
-        std::min<size_t>((size_t)(lw < 0 ? pf_lds_per_wave(kGreeks) : lw) * wpb, 65536);
+    const size_t lds = std::min<size_t>((size_t)std::max(lw, 0) * kPfWaves, 65536 - 512);
+    const dim3 grid((unsigned)shape.blocks), block(kPfThreads);
     if (a.n < (int64_t(1) << 30))
-        hipLaunchKernelGGL((k_pf_rows<VW, kGreeks, NT, uint32_t>), dim3((unsigned)nb), dim3(NT),
-                           lds, st, a);
+        hipLaunchKernelGGL((k_pf_rows<kGreeks, AL, uint32_t>), grid, block, lds, st, a, slot, busy,
+                           sums);
     else
-        hipLaunchKernelGGL((k_pf_rows<VW, kGreeks, NT, int64_t>), dim3((unsigned)nb), dim3(NT),
-                           lds, st, a);
-    reduce_partials<NQ>(a.partial, nb * wpb, a.partial + nb * wpb * NQ, sums, st);
+        hipLaunchKernelGGL((k_pf_rows<kGreeks, AL, int64_t>), grid, block, lds, st, a, slot, busy,
+                           sums);
+    if (!slot)
+        hipLaunchKernelGGL((k_pf_final<kGreeks ? 5 : 1>), dim3(1),
+                           dim3((unsigned)std::min<int64_t>(
+                               (shape.blocks + kPfGroup - 1) / kPfGroup * 64, kPfFinalThreads)),
+                           0, st, a.partial, (int)shape.blocks, sums);
     return hipGetLastError();
 }
 
-bool pf_vec2(const PfArgs& a) {
+bool pf_aligned(const PfArgs& a) {
     auto al = [](const void* p, uintptr_t b) { return (reinterpret_cast<uintptr_t>(p) & (b - 1)) == 0; };
     return al(a.in.s, 8) && al(a.in.k, 8) && al(a.in.r, 8) && al(a.in.v, 8) && al(a.in.t, 8) &&
            al(a.type, 2) && (a.w == nullptr || al(a.w, 8));
 }
 
-hipError_t launch_pf_any(const PfArgs& a, bool greeks, double* sums, hipStream_t st) {
-    if (pf_vec2(a)) return greeks ? launch_pf<2, true>(a, sums, st) : launch_pf<2, false>(a, sums, st);
-    return greeks ? launch_pf<1, true>(a, sums, st) : launch_pf<1, false>(a, sums, st);
+hipError_t launch_pf_any(const PfArgs& a, bool greeks, PfSlot* slot, uint32_t* busy, double* sums,
+                         hipStream_t st) {
+    if (pf_aligned(a))
+        return greeks ? launch_pf<true, true>(a, slot, busy, sums, st)
+                      : launch_pf<false, true>(a, slot, busy, sums, st);
+    return greeks ? launch_pf<true, false>(a, slot, busy, sums, st)
+                  : launch_pf<false, false>(a, slot, busy, sums, st);
 }
 
-// ---- the form that allocates nothing -----------------------------------------
-// Its scratch is this fixed device array, sized for the largest call it takes
-// (kPfNoAllocMaxOptions options with Greeks on unaligned arrays, the most
-// partials any call of that size needs): 2.6 MB, held on every device the
-// library runs on until the process ends.  In host code the array's name is
-// not a device address: its address on each device comes from
+// ---- scratch ---------------------------------------------------------------------
+// Fixed device arrays, held on every device the library runs on until the
+// process ends: kPfSlots slots of the one-launch form (12 MB in all) and the
+// partials of bs_portfolio_f32_noalloc (0.3 MB).  In host code the arrays'
+// names are not device addresses: their addresses on each device come from
 // hipGetSymbolAddress, resolved once per device with that device current, and
-// only that address reaches a kernel.
-constexpr int64_t kPfScratchDoubles = pf_scratch_doubles(kPfNoAllocMaxOptions, 1, true);
-static_assert(kPfScratchDoubles >= pf_scratch_doubles(kPfNoAllocMaxOptions, 2, true) &&
-                  kPfScratchDoubles >= pf_scratch_doubles(kPfNoAllocMaxOptions, 1, false),
-              "scratch sized for the worst form");
-__device__ __align__(256) double g_pf_scratch[kPfScratchDoubles];
+// only those reach a kernel.
+constexpr int kPfSlots = 32;
+__device__ __align__(256) PfSlot g_pf_slots[kPfSlots];
+__device__ __align__(256) double g_pf_scratch[kPfMaxBlocks * 5];
 
 constexpr int kPfMaxDevices = 64;
-std::mutex g_pf_scratch_mu;
-double* g_pf_scratch_ptr[kPfMaxDevices] = {};
+struct PfDevice {
+    std::mutex mu;
+    PfSlot* slots = nullptr;
+    double* scratch = nullptr;
+    uint32_t* busy = nullptr;       // pinned, one flag per slot, a cache line apart
+    uint32_t* busy_dev = nullptr;   // the same memory, device address
+    std::atomic<unsigned> next{0};
+};
+constexpr int kPfFlagStride = 64 / sizeof(uint32_t);
+
+PfDevice& pf_device(int dev) {
+    static PfDevice* d = new PfDevice[kPfMaxDevices];   // lives until the process ends
+    return d[dev];
+}
+
+template <class T, class S>
+hipError_t symbol_address(T** p, const S& symbol) {
+    void* a = nullptr;
+    const hipError_t e = hipGetSymbolAddress(&a, symbol);
+    if (e == hipSuccess) *p = static_cast<T*>(a);
+    return e;
+}
 
 hipError_t pf_scratch_of(int dev, double** out) {
     if (dev < 0 || dev >= kPfMaxDevices) return hipErrorInvalidDevice;
-    std::lock_guard<std::mutex> lk(g_pf_scratch_mu);
-    if (!g_pf_scratch_ptr[dev]) {
-        void* p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(g_pf_scratch));
-        if (e != hipSuccess) return e;
-        g_pf_scratch_ptr[dev] = static_cast<double*>(p);
+    PfDevice& d = pf_device(dev);
+    std::lock_guard<std::mutex> lk(d.mu);
+    hipError_t e = hipSuccess;
+    if (!d.scratch) e = symbol_address(&d.scratch, HIP_SYMBOL(g_pf_scratch));
+    *out = d.scratch;
+    return e;
+}
+
+// Claims a free slot of the device, or returns -1 (none free, or no flags).
+int claim_slot(PfDevice& d) {
+    {
+        std::lock_guard<std::mutex> lk(d.mu);
+        if (!d.slots && symbol_address(&d.slots, HIP_SYMBOL(g_pf_slots)) != hipSuccess) {
+            (void)hipGetLastError();
+            return -1;
+        }
+        if (!d.busy) {
+            uint32_t* p = nullptr;
+            void* q = nullptr;
+            if (hipHostMalloc(reinterpret_cast<void**>(&p), kPfSlots * 64, hipHostMallocCoherent) !=
+                hipSuccess) {
+                (void)hipGetLastError();
+                return -1;
+            }
+            if (hipHostGetDevicePointer(&q, p, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                (void)hipHostFree(p);
+                return -1;
+            }
+            std::fill(p, p + kPfSlots * kPfFlagStride, 0u);
+            d.busy_dev = static_cast<uint32_t*>(q);
+            d.busy = p;
+        }
     }
-    *out = g_pf_scratch_ptr[dev];
-    return hipSuccess;
+    const unsigned first = d.next.fetch_add(1, std::memory_order_relaxed);
+    for (unsigned i = 0; i < kPfSlots; ++i) {
+        const unsigned s = (first + i) % kPfSlots;
+        uint32_t idle = 0;
+        if (__atomic_compare_exchange_n(d.busy + s * kPfFlagStride, &idle, 1u, false,
+                                        __ATOMIC_ACQUIRE, __ATOMIC_RELAXED))
+            return (int)s;
+    }
+    return -1;
+}
+
+bool capturing(hipStream_t st) {
+    if (!st) return false;   // the null stream cannot be captured
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
 }
 
 }  // namespace
 
-// bs_portfolio_f32 with the device's fixed scratch: no allocation.  The caller
+// bs_portfolio_f32 with the device's fixed partials: no allocation.  The caller
 // has checked n <= kPfNoAllocMaxOptions.  Calls that overlap on one device
-// share the scratch and race.
+// share the array and race (the two-launch form: a race leaves no counter
+// behind that a later call could meet).
 hipError_t launch_portfolio_f32_noalloc(SoaIn<float> in, const uint8_t* type, const float* w,
                                         int64_t n, bool greeks, double* sums, hipStream_t st) {
     if (n > kPfNoAllocMaxOptions) return hipErrorInvalidValue;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    PfArgs a{in, type, w, n, nullptr};
+    PfArgs a{in, type, w, n, 0, nullptr};
     e = pf_scratch_of(dev, &a.partial);
     if (e != hipSuccess) return e;
-    return launch_pf_any(a, greeks, sums, st);
+    return launch_pf_any(a, greeks, nullptr, nullptr, sums, st);
 }
 
 hipError_t launch_portfolio_f32(SoaIn<float> in, const uint8_t* type, const float* w, int64_t n,
                                 bool greeks, double* sums, hipStream_t st) {
-    PfArgs a{in, type, w, n, nullptr};
-    const int64_t need = pf_scratch_doubles(n, pf_vec2(a) ? 2 : 1, greeks);
-    hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&a.partial),
-                                  (size_t)need * sizeof(double), st);
+    PfArgs a{in, type, w, n, 0, nullptr};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    e = launch_pf_any(a, greeks, sums, st);
+    if (dev < kPfMaxDevices && !capturing(st)) {
+        PfDevice& d = pf_device(dev);
+        const int s = claim_slot(d);
+        if (s >= 0) {
+            e = launch_pf_any(a, greeks, d.slots + s, d.busy_dev + s * kPfFlagStride, sums, st);
+            if (e != hipSuccess)   // nothing will run that clears the flag
+                __atomic_store_n(d.busy + s * kPfFlagStride, 0u, __ATOMIC_RELEASE);
+            return e;
+        }
+    }
+    e = hipMallocAsync(reinterpret_cast<void**>(&a.partial),
+                       (size_t)pf_shape(n, greeks).blocks * (greeks ? 5 : 1) * sizeof(double), st);
+    if (e != hipSuccess) return e;
+    e = launch_pf_any(a, greeks, nullptr, nullptr, sums, st);
     const hipError_t f = hipFreeAsync(a.partial, st);
     return e != hipSuccess ? e : f;
 }

@@ -116,3 +116,101 @@ def test_argument_errors(gpu):
     db.free()
     out.free()
     page.free()
+
+
+def _sums(capi, name, db, n, greeks, wptr, stream=None):
+    out = capi.DeviceBuffer(40)
+    capi.call(name, *db.ptrs(), wptr, n, greeks, out.ptr, stream)
+    capi.call("bs_stream_sync", stream)
+    got = out.download(np.uint64, 5 if greeks else 1)
+    out.free()
+    return got
+
+
+@pytest.mark.parametrize("n", [511, 512, 513, 64 * 512 - 1, 64 * 512, 64 * 512 + 1, 1024 * 512 - 1,
+                               1024 * 512, 2 * 1024 * 512 + 3, 8 * 1024 * 512 + 1,
+                               8192 * 2048 - 1, 8192 * 2048 + 1, 1 << 25])
+def test_one_launch_and_two_give_the_same_bits(gpu, n):
+    """At the edges of blocks (512 options with one row), groups of 64 blocks,
+    the rows per wave and the most blocks: the one-launch sums are the
+    two-launch ones, and those of the same book off a vector boundary, bit for
+    bit, and the exact sums within an FP64 reduction's rounding."""
+    book = books.make_book(n, books.SEED_BASE + 93)
+    w = np.random.default_rng(n).uniform(-1.0, 2.0, n).astype(np.float32)
+    db, off = gpu.DeviceBook(book), gpu.DeviceBook(book, pad=1)
+    wb = gpu.DeviceBuffer.from_array(w)
+    wo = gpu.DeviceBuffer.from_array(np.concatenate([np.zeros(1, np.float32), w]))
+    for greeks in (0, 1):
+        want = _sums(gpu, "bs_portfolio_f32_noalloc", db, n, greeks, wb.ptr)
+        got = _sums(gpu, "bs_portfolio_f32", db, n, greeks, wb.ptr)
+        shifted = _sums(gpu, "bs_portfolio_f32", off, n, greeks, wo.ptr + 4)
+        assert np.array_equal(got, want) and np.array_equal(shifted, want)
+        if n < 3_000_000:
+            ref, scale = exact_sums(map_outputs(gpu, db, n, greeks), w)
+            assert np.all(np.abs(got.view(np.float64) - ref) <= 1e-13 * scale)
+    for b in (db, off, wb, wo):
+        b.free()
+
+
+def test_many_calls_in_flight(gpu):
+    """More calls than scratch slots at once, on four streams from four
+    threads: every call's sums are its book's own."""
+    import threading
+    sizes = (700, 40_961, 300_001, 1_000_003)
+    dbs = [gpu.DeviceBook(books.make_book(n, books.SEED_BASE + 94 + i)) for i, n in enumerate(sizes)]
+    want = [[_sums(gpu, "bs_portfolio_f32_noalloc", d, n, g, None) for g in (0, 1)]
+            for d, n in zip(dbs, sizes)]
+    bad = []
+
+    def work(k):
+        st = gpu.Stream()
+        outs = [gpu.DeviceBuffer(40) for _ in range(60)]
+        for rep in range(5):
+            for i, o in enumerate(outs):
+                j = (i + k) % 4
+                gpu.call("bs_portfolio_f32", *dbs[j].ptrs(), None, sizes[j], i & 1, o.ptr,
+                         st.handle)
+            st.sync()
+            for i, o in enumerate(outs):
+                j = (i + k) % 4
+                if not np.array_equal(o.download(np.uint64, 5 if i & 1 else 1, st.handle),
+                                      want[j][i & 1]):
+                    bad.append((k, rep, i))
+        for o in outs:
+            o.free()
+        st.destroy()
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad, bad[:5]
+    for d in dbs:
+        d.free()
+
+
+def test_inside_a_callers_graph(gpu):
+    """Captured, the call takes the form whose scratch is the graph's own;
+    replays with eager calls between them give the eager sums."""
+    import ctypes
+    from test_gpu_capture import CAPTURE_THREAD_LOCAL, hip
+    H, L, n = hip(), gpu.load(), 100_003
+    db = gpu.DeviceBook(books.make_book(n, books.SEED_BASE + 98))
+    want = _sums(gpu, "bs_portfolio_f32", db, n, 1, None)
+    st, out = gpu.Stream(), gpu.DeviceBuffer(40)
+    graph, gexec = ctypes.c_void_p(), ctypes.c_void_p()
+    assert H.hipStreamBeginCapture(st.handle, CAPTURE_THREAD_LOCAL) == 0
+    rc = L.bs_portfolio_f32(*db.ptrs(), None, n, 1, out.ptr, st.handle)
+    assert H.hipStreamEndCapture(st.handle, ctypes.byref(graph)) == 0 and rc == 0
+    assert H.hipGraphInstantiate(ctypes.byref(gexec), graph, None, None, 0) == 0
+    for rep in range(4):
+        assert H.hipGraphLaunch(gexec, st.handle) == 0
+        gpu.call("bs_stream_sync", st.handle)
+        assert np.array_equal(out.download(np.uint64, 5), want), rep
+        assert np.array_equal(_sums(gpu, "bs_portfolio_f32", db, n, 1, None), want)
+    H.hipGraphExecDestroy(gexec)
+    H.hipGraphDestroy(graph)
+    st.destroy()
+    out.free()
+    db.free()
