@@ -28,8 +28,8 @@
 //            v_rcp_f32, v_sqrt_f32), Horner polynomial with FMA.  About a
 //            third of Ref32's VALU work; prices differ from the reference by
 //            up to ~1.2e-4 on a 10M book (mean 6e-6).
-//   Ref64    fptype = double: the same statements in FP64 (its log, CNDF
-//            reciprocal and CNDF polynomial are written out below).
+//   Ref64    fptype = double: the same statements in FP64.  Ordinary inputs
+//            take primitives without special-value handling (bs_fp64.hpp).
 //
 // Every function here is compiled with FMA contraction off; each FMA is
 // written out, so every kernel that inlines these functions computes the same
@@ -41,6 +41,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include "bs_fp64.hpp"
 
 namespace bs {
 
@@ -208,6 +210,11 @@ struct Ref32Arith {
 
 struct Ref32 : Ref32Arith<true> {
     using Unchecked = Ref32Arith<false>;
+    // Whether a price of the unchecked form stands for these inputs.
+    __device__ static __forceinline__ bool unchecked_holds(float, float, float, float, float,
+                                                           float price) {
+        return price == price;
+    }
 };
 
 // ---------------------------------------------------------------------------
@@ -302,6 +309,36 @@ __device__ __forceinline__ double log64(double x) {
     return x == 0.0 ? -__builtin_inf() : (x > 0.0 ? x : __builtin_nan(""));
 }
 
+// Ref64Ordinary: Ref64's statements for ordinary inputs (Ref64::unchecked_holds),
+// with the primitives of bs_fp64.hpp: quotients and the square root within half
+// an ulp and 2^-24 of one, as IEEE's to the eye, exp and log within an ulp, none
+// of them with code for special values.  |x| of CNDF is capped at 40, past
+// which e^{-x^2/2} is 0 and CNDF exactly 0 or 1.
+struct Ref64Ordinary {
+    using T = double;
+    static constexpr bool kSplitCndf = true;
+    __device__ static __forceinline__ double exp(double x) { return exp_mid(x); }
+    __device__ static __forceinline__ double log(double x) { return log_pos(x); }
+    __device__ static __forceinline__ double div(double a, double b) { return quot_pos(a, b); }
+    __device__ static __forceinline__ double sqrt(double x) { return sqrt_pos(x); }
+
+    // CNDF's value for |x|; see Ref32Arith::cndf_abs.
+    template <bool kGrad>
+    __device__ static __forceinline__ double cndf_abs(double x, double* /*grad*/) {
+#pragma clang fp contract(off)
+        static_assert(!kGrad, "FP64 prices only");
+        const double ax = __builtin_fmin(__builtin_fabs(x), 40.0);
+        const double n = exp_mid(-0.5 * ax * ax) * kInvSqrt2Pi;
+        const double k = recip_pos(__builtin_fma(kP, ax, 1.0));
+        double t1 = __builtin_fma(k, kB5, kB4);
+        t1 = __builtin_fma(k, t1, kB3);
+        t1 = __builtin_fma(k, t1, kB2);
+        t1 = __builtin_fma(k, t1, kB1);
+        t1 = t1 * k;
+        return __builtin_fma(-t1, n, 1.0);
+    }
+};
+
 // Ref64: fptype = double, the reference's statements with every step in FP64.
 // Division and square root are IEEE (the compiler's correctly rounded
 // sequences) and exp is the device library's; log is log64; CNDF's
@@ -310,10 +347,23 @@ __device__ __forceinline__ double log64(double x) {
 // denominator finite), and CNDF's polynomial is evaluated by Horner's rule
 // with FMA rather than from the powers of k.  Against the reference compiled
 // with fptype = double, prices differ by a few units in the last place.
+//
+// It prices the options that are not ordinary; Ref64Ordinary does the others:
+// s, k, v and t in [2^-100, 2^100) and |r t| < 700, where no quotient, square,
+// product or exponential of the price leaves FP64's normal range except
+// CNDF's tail towards 0.
 struct Ref64 {
     using T = double;
-    using Unchecked = Ref64;
+    using Unchecked = Ref64Ordinary;
     static constexpr bool kSplitCndf = false;
+    __device__ static __forceinline__ bool unchecked_holds(double s, double k, double r, double v,
+                                                           double t, double) {
+        const uint32_t a = (uint32_t)__double2hiint(s), b = (uint32_t)__double2hiint(k),
+                       c = (uint32_t)__double2hiint(v), d = (uint32_t)__double2hiint(t);
+        const uint32_t lo = min(min(a, b), min(c, d)), hi = max(max(a, b), max(c, d));
+        // high words of 2^-100 and 2^100; negative numbers and NaN are above both
+        return lo >= 0x39b00000u && hi < 0x46300000u && __builtin_fabs(r * t) < 700.0;
+    }
     __device__ static __forceinline__ double exp(double x) { return ::exp(x); }
     __device__ static __forceinline__ double log(double x) { return log64(x); }
     __device__ static __forceinline__ double div(double a, double b) { return a / b; }
@@ -410,7 +460,8 @@ __device__ __forceinline__ T bs_combine_split(T s, const Forward<T>& f, bool put
 }
 
 // A policy with a distinct unchecked form prices with it first and recomputes
-// with the checked one where the price is NaN (Ref32: identical bits).
+// with the checked one where that does not hold: Ref32 where the price is NaN
+// (identical bits), Ref64 where an input is not ordinary.
 template <class M>
 constexpr bool has_unchecked() {
     return !__is_same(typename M::Unchecked, M);
@@ -423,7 +474,8 @@ __device__ __forceinline__ typename M::T bs_price(typename M::T s, typename M::T
     if constexpr (has_unchecked<M>()) {
         using U = typename M::Unchecked;
         typename M::T p = bs_combine_split(s, bs_forward<U, false>(s, k, r, v, t), put);
-        if (__builtin_expect(p != p, 0)) p = bs_combine(s, bs_forward<M, false>(s, k, r, v, t), put);
+        if (__builtin_expect(!M::unchecked_holds(s, k, r, v, t, p), 0))
+            p = bs_combine(s, bs_forward<M, false>(s, k, r, v, t), put);
         return p;
     } else {
         return bs_combine(s, bs_forward<M, false>(s, k, r, v, t), put);

@@ -21,7 +21,7 @@
 // 65.9 us on two streams (14 KB: 65.7-65.9; 18 KB: 67.1; none: 77.1), two
 // options per work-item, 11 KB per wave 67.98 / 67.22 us (none: 74.16 /
 // 73.79; 9 KB: 68.18 / 68.52; 12 KB: 70.82 / 69.59); int32-type price 64
-// threads 44.9 us, FP64 64 threads pipelined 85 us.  Small blocks help:
+// threads 44.9 us; FP64 below.  Small blocks help:
 // one-wave workgroups retire and refill independently, so the tail of the
 // grid is short.  Fewer resident waves help the write-heavy Greeks stream
 // most: with 14 waves per CU instead of 32 its five output streams keep fewer
@@ -182,12 +182,17 @@ struct PriceI32F32 {
 };
 
 // fptype = double: a group is VW = 2 options (one 128-bit load per array).
+// 10M options on one stream, 490 MB: 81.2 us (6.0 TB/s) at 165 VALU
+// instructions per option and 5 waves per SIMD, where Ref64's general
+// primitives (230 instructions) took 94; with 3 waves per SIMD 82.9, not
+// pipelined 86.8, one option per work-item (8-byte stores) 84-87, the waves
+// capped by 8 KB of LDS each 84.
 template <int VW, bool AL = true>
 struct PriceF64 {
     static constexpr int kVW = 2;
     static constexpr int kElemBytes = 8;   // widest array element
     static constexpr int kLdsPerWave = 0;
-    static constexpr int kWaves = 5;
+    static constexpr int kWaves = 7;
     static constexpr int kThreadsPref = 64;
     static constexpr int64_t kBlocks = 0;
     static constexpr bool kPipe = true;

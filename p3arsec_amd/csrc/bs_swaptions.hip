@@ -54,6 +54,7 @@
 #include <mutex>
 #include <vector>
 
+#include "bs_fp64.hpp"
 #include "bs_internal.hpp"
 
 namespace bs {
@@ -223,62 +224,6 @@ static_assert(in_tail(kTailLo) && !in_tail(kTailLo + 1) && in_tail(kTailHi) &&
                   !in_tail(kTailHi - 1) && in_tail(0) && in_tail((uint32_t)kM31 - 1),
               "tail residues");
 
-// a / b for b in [0.007, 4]: with e = 1 - b y the error of v_rcp_f64's y (at
-// most 2^-24.3 there, measured), a y (1 + e + e^2), within an ulp of a / b.
-__device__ __forceinline__ double div_near1(double a, double b) {
-    const double y = __builtin_amdgcn_rcp(b);
-    const double e = __builtin_fma(-b, y, 1.0);
-    const double q = a * y;
-    return __builtin_fma(q, __builtin_fma(e, e, e), q);
-}
-
-// log(x) of a positive normal x: x = 2^e m, m in [sqrt(1/2), sqrt(2)) (the
-// exponent field counted from the high word of sqrt(1/2)), s = (m - 1) / (m + 1),
-// log m = 2 atanh(s) with (2 atanh(s) / s - 2) / s^2 interpolated at Chebyshev
-// nodes in s^2 (degree 6, relative error 5e-18).
-__device__ __forceinline__ double log_pos(double x) {
-    constexpr uint32_t kRootHalf = 0x3fe6a09eu;
-    const uint32_t b = (uint32_t)__double2hiint(x) - kRootHalf;
-    const int e = (int)b >> 20;
-    const double m = __hiloint2double((int)((b & 0xfffffu) + kRootHalf), __double2loint(x));
-    const double f = m - 1.0;
-    const double s = div_near1(f, m + 1.0);
-    const double z = s * s;
-    double p = 0.14616449685043406;
-    p = __builtin_fma(p, z, 0.15331721600556042);
-    p = __builtin_fma(p, z, 0.18182889125261723);
-    p = __builtin_fma(p, z, 0.2222221113479508);
-    p = __builtin_fma(p, z, 0.28571428625975487);
-    p = __builtin_fma(p, z, 0.39999999999899505);
-    p = __builtin_fma(p, z, 0.666666666666667);
-    const double h = 0.5 * (f * f);
-    const double lm = f + __builtin_fma(s, __builtin_fma(z, p, h), -h);
-    const double ed = (double)e;
-    // ln 2 in two parts, the first with 32 significant bits
-    return __builtin_fma(ed, 0.6931471803691238, __builtin_fma(ed, 1.9082149292705877e-10, lm));
-}
-
-// 2^x for |x| < 1000: (2^f - 1) / f interpolated at Chebyshev nodes over
-// |f| <= 1/2 (degree 10, relative error of 2^f 2e-17 with rounded
-// coefficients).
-__device__ __forceinline__ double exp2_mid(double x) {
-    const double k = __builtin_rint(x);
-    const double f = x - k;
-    double p = 4.4549605981865186e-10;
-    p = __builtin_fma(p, f, 7.072585949269223e-09);
-    p = __builtin_fma(p, f, 1.0178062445845774e-07);
-    p = __builtin_fma(p, f, 1.321544258792169e-06);
-    p = __builtin_fma(p, f, 1.525273382983612e-05);
-    p = __builtin_fma(p, f, 0.0001540353044173605);
-    p = __builtin_fma(p, f, 0.0013333558146416936);
-    p = __builtin_fma(p, f, 0.009618129107606888);
-    p = __builtin_fma(p, f, 0.0555041086648216);
-    p = __builtin_fma(p, f, 0.24022650695910097);
-    p = __builtin_fma(p, f, 0.6931471805599453);
-    p = __builtin_fma(p, f, 1.0);
-    return __builtin_amdgcn_ldexp(p, (int)k);
-}
-
 // A constant held in a vector register from here on.  An FP64 instruction reads
 // one scalar operand at most and there are not enough scalar registers for
 // every constant of k_sw_paths, so the compiler otherwise builds the central
@@ -306,7 +251,7 @@ struct MoroCentral {
         den = __builtin_fma(r, den, b3);
         den = __builtin_fma(r, den, b4);
         den = __builtin_fma(r, den, 1.0);   // 0.11 <= den <= 1 for |x| <= 0.42
-        return div_near1(x * num, den);
+        return quot_near(x * num, den);
     }
 };
 

@@ -340,3 +340,31 @@ def test_slices_give_the_same_bits(gpu, n, pads, out_pad):
             for b in bufs + outs:
                 b.free()
         assert got[:k] == got[k:], (fn, n, pads)
+
+
+@pytest.mark.parametrize("which", ["s", "k", "v", "t", "r"])
+def test_fp64_at_the_edges_of_ordinary_inputs(gpu, oracle, which):
+    """One input at and beyond the ends of the range that the primitives
+    without special-value handling take (2^-100 <= s, k, v, t < 2^100, |r t| <
+    700), the others as in a book.  Both sides round a price's terms, each at
+    most S or K in size, some 16 times within an ulp: 2 x 16 x 2^-53 (S + K),
+    3.6e-15, past the largest terms' size."""
+    n = 64
+    book = books.make_book(n, books.SEED_BASE + 61).astype(np.float64)
+    lo, hi = 2.0 ** -100, 2.0 ** 100
+    ends = [np.nextafter(lo, 0), lo, np.nextafter(lo, 1), 2.0 ** -60, 2.0 ** 60,
+            np.nextafter(hi, 0), hi, np.nextafter(hi, np.inf), 2.0 ** -1040, 2.0 ** 900]
+    if which == "r":
+        ends = [-699.0 / 2, 699.0 / 2, -701.0, 701.0, 0.0, -0.05, 1e-300, 300.0, -300.0, 1e4]
+    a = getattr(book, which)
+    a[:] = np.resize(np.array(ends), n)
+    got = run(gpu, book, "f64")
+    ref = oracle.price_f64(book)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    fin = np.isfinite(ref)
+    assert np.array_equal(got[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
+    with np.errstate(over="ignore"):
+        fv = book.k * np.exp(-book.r * book.t)
+    scale = (book.s + book.k + fv)[fin]
+    rel = np.maximum(1.0, np.abs(book.r * book.t))[fin]   # exp's own conditioning
+    assert np.all(np.abs(got[fin] - ref[fin]) <= 3.6e-15 * scale * rel)
