@@ -29,6 +29,7 @@
 #include <time.h>
 
 #include <algorithm>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -138,6 +139,41 @@ void k_serve(const uint8_t* __restrict__ slot) {
     }
 }
 
+// ---- replies -----------------------------------------------------------------
+// bs_result_copy's way to the host: one kernel writes the wanted span of a
+// request's outputs (contiguous in the arena) into pinned memory and then the
+// reply's sequence number, on which the caller spins; the arrays go on to the
+// caller's from there.  The runtime's own copies take 11-35 us each to pageable
+// memory (copy kernel, marker, interrupt), five of them for a Greeks request:
+// a round of 32 requests of up to 64K options, one third with Greeks, submitted,
+// waited for and copied out one by one takes 390 us, with those copies 1050.
+// Bound by the launch and the link's latency.  Every store is a relaxed
+// system-scope one (written through), acknowledged before the block counts
+// itself in.
+constexpr int kReplies = 2;                         // replies on their way at once
+constexpr size_t kReplyBytes = size_t(3) << 19;     // 1.5 MB: the Greeks of 64K options
+constexpr int kReplyBlocks = 64;
+
+__global__ __launch_bounds__(kThreads) void k_reply(const uint64_t* __restrict__ src,
+                                                    uint64_t* __restrict__ dst, int words,
+                                                    uint32_t* count, uint32_t* flag,
+                                                    uint32_t seq) {
+    for (int i = blockIdx.x * kThreads + threadIdx.x; i < words; i += gridDim.x * kThreads)
+        __hip_atomic_store(dst + i, src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);   // this wave's stores are acknowledged
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __syncthreads();
+    if (threadIdx.x == 0 &&
+        __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+            gridDim.x - 1) {
+        __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(flag, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+__global__ void k_zero_word(uint32_t* p) { *p = 0; }
+
 using ServePrice = PriceF32<Ref32, kVW>;
 using ServeGreeks = GreeksF32<kVW>;
 
@@ -185,6 +221,15 @@ struct HipExec {
     hipEvent_t ev[kSlots] = {};
     hipStream_t slot_stream[kSlots] = {};        // the stream slot s was last launched on
     int64_t seq = 0, nlaunch = 0;
+    struct Reply {
+        std::mutex mu;
+        hipStream_t stream = nullptr;
+        uint32_t seq = 0;
+    } reply[kReplies];
+    uint8_t* reply_host = nullptr;              // pinned: kReplies x (kReplyBytes, flag line)
+    uint8_t* reply_dev = nullptr;               // the same memory, device address
+    uint32_t* reply_count = nullptr;            // device: a counter per reply, zero between uses
+    static constexpr size_t kReplySpan = kReplyBytes + 256;
 
     hipError_t init(int dev, size_t arena_bytes, int graph_on, int grid_blocks, int block_threads) {
         device = dev;
@@ -205,6 +250,19 @@ struct HipExec {
             if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[s], hipEventDisableTiming);
             if (e == hipSuccess) ::memset(host_slot[s], 0, sizeof(SlotHeader));
         }
+        for (int r = 0; r < kReplies && e == hipSuccess; ++r)
+            e = hipStreamCreateWithFlags(&reply[r].stream, hipStreamNonBlocking);
+        if (e == hipSuccess)
+            e = hipHostMalloc((void**)&reply_host, kReplies * kReplySpan, hipHostMallocCoherent);
+        if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&reply_dev, reply_host, 0);
+        if (e == hipSuccess) e = hipMalloc((void**)&reply_count, kReplies * 256);
+        for (int r = 0; r < kReplies && e == hipSuccess; ++r) {
+            ::memset(reply_host + r * kReplySpan + kReplyBytes, 0, sizeof(uint32_t));
+            // counters 256 bytes apart; a plain store kernel, then done before use
+            hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, reply[r].stream,
+                               reply_count + r * 64);
+            e = hipGetLastError();
+        }
         if (grid_blocks > 0) grid_cap = std::min<int64_t>(grid_blocks, kMaxGrid);
         for (int s = 0; s < kSlots && e == hipSuccess && use_graph; ++s) e = capture(s);
         return e;
@@ -222,6 +280,10 @@ struct HipExec {
         if (stream) (void)hipStreamDestroy(stream);
         for (hipStream_t st : streams)
             if (st) (void)hipStreamDestroy(st);
+        for (Reply& r : reply)
+            if (r.stream) (void)hipStreamDestroy(r.stream);
+        if (reply_host) (void)hipHostFree(reply_host);
+        if (reply_count) (void)hipFree(reply_count);
         if (arena) (void)hipFree(arena);
     }
 
@@ -358,6 +420,66 @@ struct HipExec {
         if (stream) (void)hipStreamSynchronize(stream);
         for (hipStream_t st : streams)
             if (st) (void)hipStreamSynchronize(st);
+        for (Reply& r : reply)
+            if (r.stream) (void)hipStreamSynchronize(r.stream);
+    }
+
+    // Memory the CPU may write directly (what the runtime does not know is the
+    // caller's ordinary memory).
+    static bool host_memory(const void* p) {
+        hipPointerAttribute_t a;
+        ::memset(&a, 0, sizeof(a));
+        if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+            (void)hipGetLastError();
+            return true;
+        }
+        return a.type == hipMemoryTypeHost || a.type == hipMemoryTypeUnregistered;
+    }
+
+    // Copies k arrays of `bytes` bytes from the arena (src[j], ascending) to
+    // dst[j]: through a reply's pinned memory when one is free and the span
+    // from the first to the last fits it, else by the runtime's copies.
+    hipError_t copy_out(void* const* dst, char* const* src, int k, size_t bytes) {
+        const size_t span = k > 0 ? (size_t)(src[k - 1] - src[0]) + bytes : 0;
+        bool host = k > 0;
+        for (int j = 0; j < k; ++j) host = host && host_memory(dst[j]);
+        if (host && span <= kReplyBytes) {
+            for (int r = 0; r < kReplies; ++r) {
+                std::unique_lock<std::mutex> lk(reply[r].mu, std::try_to_lock);
+                if (!lk.owns_lock()) continue;
+                return reply_out(r, dst, src, k, bytes, span);
+            }
+        }
+        hipError_t e = hipSuccess;
+        for (int j = 0; j < k && e == hipSuccess; ++j)
+            e = hipMemcpy(dst[j], src[j], bytes, hipMemcpyDeviceToHost);
+        return e;
+    }
+
+    hipError_t reply_out(int r, void* const* dst, char* const* src, int k, size_t bytes,
+                         size_t span) {
+        uint8_t* host = reply_host + r * kReplySpan;
+        uint8_t* dev = reply_dev + r * kReplySpan;
+        const int words = (int)((span + 7) / 8);   // outputs are padded to 256 bytes
+        const uint32_t seq = ++reply[r].seq;
+        hipLaunchKernelGGL(k_reply, dim3(std::min((words + kThreads - 1) / kThreads, kReplyBlocks)),
+                           dim3(kThreads), 0, reply[r].stream,
+                           reinterpret_cast<const uint64_t*>(src[0]),
+                           reinterpret_cast<uint64_t*>(dev), words, reply_count + r * 64,
+                           reinterpret_cast<uint32_t*>(dev + kReplyBytes), seq);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        const uint32_t* flag = reinterpret_cast<const uint32_t*>(host + kReplyBytes);
+        auto arrived = [&] { return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq; };
+        const int64_t until = serve::steady_ns() + 200000;
+        while (!arrived() && serve::steady_ns() < until) __builtin_ia32_pause();
+        if (!arrived()) {
+            e = hipStreamSynchronize(reply[r].stream);
+            if (e != hipSuccess) return e;
+            if (!arrived()) return hipErrorUnknown;
+        }
+        for (int j = 0; j < k; ++j) ::memcpy(dst[j], host + (src[j] - src[0]), bytes);
+        return hipSuccess;
     }
 };
 
@@ -589,14 +711,22 @@ int bs_result_copy(bs_ctx_t ctx, bs_ticket_t ticket, float* price, float* delta,
         if (rc != BS_OK) return set_error(rc, "ticket not done");
         size_t oo[5];
         serve::output_layout(n, kind, oo);
-        float* dst[5] = {price, delta, vega, rho, theta};
+        float* want[5] = {price, delta, vega, rho, theta};
         hipError_t e = hipSetDevice(c->exec.device);
-        for (int j = 0; j < 5 && e == hipSuccess; ++j) {
-            if (!dst[j]) continue;
-            if (j > 0 && kind != serve::kGreeks) return set_error(BS_ERR_INVALID, "not a Greeks ticket");
-            e = hipMemcpy(dst[j], c->exec.arena + off + oo[j], (size_t)n * 4, hipMemcpyDeviceToHost);
+        void* dst[5];
+        char* src[5];
+        int k = 0;
+        bool refused = false;   // Greeks asked of a price ticket: after the price is copied
+        for (int j = 0; j < 5 && !refused; ++j) {
+            if (!want[j]) continue;
+            refused = j > 0 && kind != serve::kGreeks;
+            if (refused) break;
+            dst[k] = want[j];
+            src[k++] = c->exec.arena + off + oo[j];
         }
-        return e == hipSuccess ? BS_OK : hip_error(e, "bs_result_copy");
+        if (e == hipSuccess) e = c->exec.copy_out(dst, src, k, (size_t)n * 4);
+        if (e != hipSuccess) return hip_error(e, "bs_result_copy");
+        return refused ? set_error(BS_ERR_INVALID, "not a Greeks ticket") : BS_OK;
     });
 }
 

@@ -325,3 +325,37 @@ def test_reap_needs_completion_queue(gpu):
         assert ctx.L.bs_reap(ctx.h, (gpu.Completion * 4)(), 4, 0, ctypes.byref(cnt)) == -1
     finally:
         ctx.destroy()
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 4097, 16_384, 65_536, 75_001, 76_801, 200_003])
+def test_results_reach_the_host_whole(gpu, n):
+    """Replies of every size on both sides of the pinned reply's 1.5 MB (Greeks
+    of 76,800 options): all five outputs, some of them, and nothing past their
+    ends; from several threads at once, more than there are replies."""
+    book = books.make_book(n, books.SEED_BASE + 95)
+    want = [o.download(np.float32, n) for o in gpu.greeks(gpu.DeviceBook(book))]
+    ctx = Ctx(gpu, 64 << 20)
+    b = ctx.register(book)
+    t = ctx.submit(b, 2)
+    assert ctx.wait(t) == 0
+    bad = []
+
+    def copy(which):
+        for _ in range(4):
+            outs = [np.full(n + 8, 7.25, np.float32) for _ in range(5)]
+            ptrs = [o.ctypes.data if j in which else None for j, o in enumerate(outs)]
+            gpu.call("bs_result_copy", ctx.h, t, *ptrs)
+            for j, o in enumerate(outs):
+                ok = np.all(o[n:] == 7.25) and (np.array_equal(o[:n], want[j]) if j in which
+                                                else np.all(o == 7.25))
+                if not ok:
+                    bad.append((which, j))
+
+    ts = [threading.Thread(target=copy, args=(w,)) for w in
+          ((0, 1, 2, 3, 4), (0,), (4,), (1, 3), (0, 1, 2, 3, 4), ())]
+    for x in ts:
+        x.start()
+    for x in ts:
+        x.join()
+    assert not bad, bad
+    ctx.destroy()
