@@ -615,6 +615,13 @@ __global__ __launch_bounds__(kSwThreads) void k_sw_paths_steps(
     block_partial(sum, sumsq, partial);
 }
 
+// A call's parameters from pinned host memory (16-byte words).
+__global__ __launch_bounds__(kSwThreads) void k_sw_stage(const uint4* __restrict__ host,
+                                                         uint4* __restrict__ dev, int words) {
+    for (int i = blockIdx.x * kSwThreads + threadIdx.x; i < words; i += gridDim.x * kSwThreads)
+        dev[i] = host[i];
+}
+
 // Block i adds swaption i's bps partials (work-item t takes t, t + 256, ...
 // in order, then a fixed tree) and writes out[2i] = mean, out[2i+1] = standard
 // error (HJM_Swaption_Blocking.cpp:212-218).
@@ -857,11 +864,75 @@ bool draws_zero(int64_t c, int64_t count) {
     return c % m == 0 || c / m != (c + count - 1) / m;
 }
 
-// The per-call buffers (parameters, partial sums, results) come from one
-// stream-ordered pool per device that keeps freed memory up to 1 GiB: the
-// call ends with a stream synchronisation, at which the default pool would
-// hand its memory back to the device and the next call would allocate anew.
+// A call's buffers.  Most calls take one of up to kSwSpaces workspaces that the
+// library keeps per device, given back after the call's stream has been
+// synchronised: pinned memory, from which a kernel fetches the parameters and
+// into which the last kernel writes the results, and device memory for the
+// parameters and partial sums.  Stream-ordered allocation (22 us with its
+// free), a pageable upload (14 us) and a pageable download (20 us) cost more
+// than the kernels of a small call: 64 swaptions x 20,000 trials take 49 us
+// and took 91.
 constexpr int kSwDevices = 64;
+constexpr int kSwSpaces = 4;
+constexpr size_t kSpaceHost = size_t(1) << 20, kSpaceDev = size_t(4) << 20;
+
+struct SwSpace {
+    char* host = nullptr;       // pinned
+    char* host_dev = nullptr;   // the same memory, device address
+    char* dev = nullptr;
+};
+
+struct SwSpaces {
+    std::mutex mu;
+    std::vector<SwSpace> idle;   // room for all of them is reserved before the first
+    int made = 0;
+};
+
+SwSpaces& spaces_of(int dev) {
+    static SwSpaces* s = new SwSpaces[kSwDevices];   // lives until the process ends
+    return s[dev];
+}
+
+// Takes an idle workspace or makes one; false when all are in use or there is
+// no memory for another.
+bool take_space(int dev, SwSpace* x) {
+    if (dev < 0 || dev >= kSwDevices) return false;
+    SwSpaces& all = spaces_of(dev);
+    std::lock_guard<std::mutex> lk(all.mu);
+    all.idle.reserve(kSwSpaces);
+    if (!all.idle.empty()) {
+        *x = all.idle.back();
+        all.idle.pop_back();
+        return true;
+    }
+    if (all.made == kSwSpaces) return false;
+    void* p = nullptr;
+    if (hipHostMalloc(reinterpret_cast<void**>(&x->host), kSpaceHost, hipHostMallocCoherent) !=
+        hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (hipHostGetDevicePointer(&p, x->host, 0) != hipSuccess ||
+        hipMalloc(reinterpret_cast<void**>(&x->dev), kSpaceDev) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipHostFree(x->host);
+        return false;
+    }
+    x->host_dev = static_cast<char*>(p);
+    ++all.made;
+    return true;
+}
+
+void give_space(int dev, const SwSpace& x) {
+    SwSpaces& all = spaces_of(dev);
+    std::lock_guard<std::mutex> lk(all.mu);
+    all.idle.push_back(x);
+}
+
+// Calls that no workspace holds allocate from one stream-ordered pool per
+// device that keeps freed memory up to 1 GiB: they end with a stream
+// synchronisation, at which the default pool would hand its memory back to the
+// device and the next call would allocate anew.
 
 hipError_t pool_of(int dev, hipMemPool_t* out) {
     static std::mutex mu;
@@ -910,55 +981,93 @@ struct SwBatch {
     }
 };
 
+// The places of a call's parts: heads of both kernels | pool | partials.
+struct SwLayout {
+    size_t heads, pool, partial, bytes;   // offsets of the step-by-step heads, pool and
+                                          // partials, and what all of it takes
+    SwLayout(const SwBatch& b, size_t blocks) {
+        auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+        heads = up(b.lins.size() * sizeof(SwLin));
+        pool = heads + up(b.heads.size() * sizeof(SwHead));
+        partial = pool + up(b.pool.size() * sizeof(double));
+        bytes = partial + blocks * 2 * sizeof(double);
+    }
+    // Writes the parameters (everything before the partials), laid out as on the device.
+    void write(const SwBatch& b, char* to) const {
+        memcpy(to, b.lins.data(), b.lins.size() * sizeof(SwLin));
+        memcpy(to + heads, b.heads.data(), b.heads.size() * sizeof(SwHead));
+        memcpy(to + pool, b.pool.data(), b.pool.size() * sizeof(double));
+    }
+};
+
+// The kernels of a launch whose parameters are on the device at base.
+hipError_t launch_batch(const SwBatch& b, const SwLayout& at, int F, const SwGrid& grid,
+                        int64_t trials, char* base, double* out, hipStream_t st) {
+    const unsigned n = (unsigned)b.lins.size();
+    const unsigned blocks = (unsigned)grid.bps * n;
+    const SwLin* dl = reinterpret_cast<const SwLin*>(base);
+    const SwHead* dh = reinterpret_cast<const SwHead*>(base + at.heads);
+    const double* dp = reinterpret_cast<const double*>(base + at.pool);
+    double* dq = reinterpret_cast<double*>(base + at.partial);
+    linear_kernel(b.flows)(blocks, st, dl, dp, grid, dq);
+    if (b.steps) kStepsByFactors[F - 1](blocks, st, dl, dh, dp, grid, dq);
+    hipLaunchKernelGGL(k_sw_final, dim3(n), dim3(kSwThreads), 0, st, dq, grid.bps, trials, out);
+    return hipGetLastError();
+}
+
 int price_batch(const SwBatch& b, int F, const SwGrid& grid, int64_t trials, double* price,
                 double* std_error, hipStream_t st) {
     const size_t n = b.lins.size();
-    const unsigned blocks = (unsigned)(grid.bps * (int64_t)n);
-    // one device allocation: heads of both kernels | pool | partials | results
-    auto up = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
-    const size_t lb = up(n * sizeof(SwLin)), hb = lb + up(n * sizeof(SwHead));
-    const size_t pb = up(b.pool.size() * sizeof(double));
-    const size_t qb = up((size_t)blocks * 2 * sizeof(double));
+    const SwLayout at(b, (size_t)grid.bps * n);
     const size_t ob = n * 2 * sizeof(double);
+    auto deliver = [&](const double* out) {
+        for (size_t k = 0; k < n; ++k) {
+            price[b.index[k]] = out[2 * k];
+            std_error[b.index[k]] = out[2 * k + 1];
+        }
+        return BS_OK;
+    };
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_error(e, "hipGetDevice");
+    SwSpace space;
+    if (at.partial + ob <= kSpaceHost && at.bytes <= kSpaceDev && take_space(dev, &space)) {
+        at.write(b, space.host);
+        const int words = (int)(at.partial / sizeof(uint4));
+        hipLaunchKernelGGL(k_sw_stage, dim3(std::min((words + kSwThreads - 1) / kSwThreads, 64)),
+                           dim3(kSwThreads), 0, st, reinterpret_cast<const uint4*>(space.host_dev),
+                           reinterpret_cast<uint4*>(space.dev), words);
+        e = hipGetLastError();
+        if (e == hipSuccess)
+            e = launch_batch(b, at, F, grid, trials, space.dev,
+                             reinterpret_cast<double*>(space.host_dev + at.partial), st);
+        const hipError_t es = hipStreamSynchronize(st);
+        if (e == hipSuccess && es == hipSuccess)
+            deliver(reinterpret_cast<const double*>(space.host + at.partial));
+        if (es == hipSuccess) give_space(dev, space);   // else its work may still run
+        if (e != hipSuccess) return hip_error(e, "bs_swaptions_host_f64");
+        return es == hipSuccess ? BS_OK : hip_error(es, "hipStreamSynchronize");
+    }
     hipMemPool_t mem = nullptr;
     e = pool_of(dev, &mem);
     if (e != hipSuccess) return hip_error(e, "hipMemPoolCreate");
-    char* base = nullptr;
-    e = hipMallocFromPoolAsync(reinterpret_cast<void**>(&base), hb + pb + qb + ob, mem, st);
-    if (e != hipSuccess) return hip_error(e, "hipMallocFromPoolAsync");
-    SwLin* dl = reinterpret_cast<SwLin*>(base);
-    SwHead* dh = reinterpret_cast<SwHead*>(base + lb);
-    double* dp = reinterpret_cast<double*>(base + hb);
-    double* dq = reinterpret_cast<double*>(base + hb + pb);
-    double* dout = reinterpret_cast<double*>(base + hb + pb + qb);
     std::vector<double> out(n * 2);
-    // heads and pool leave the host as one copy, laid out as on the device
-    std::vector<char> staged(hb + b.pool.size() * sizeof(double));
-    memcpy(staged.data(), b.lins.data(), n * sizeof(SwLin));
-    memcpy(staged.data() + lb, b.heads.data(), n * sizeof(SwHead));
-    memcpy(staged.data() + hb, b.pool.data(), b.pool.size() * sizeof(double));
+    std::vector<char> staged(at.partial);
+    at.write(b, staged.data());
+    char* base = nullptr;
+    const size_t results = (at.bytes + 255) & ~(size_t)255;
+    e = hipMallocFromPoolAsync(reinterpret_cast<void**>(&base), results + ob, mem, st);
+    if (e != hipSuccess) return hip_error(e, "hipMallocFromPoolAsync");
+    double* dout = reinterpret_cast<double*>(base + results);
     e = hipMemcpyAsync(base, staged.data(), staged.size(), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) {
-        linear_kernel(b.flows)(blocks, st, dl, dp, grid, dq);
-        if (b.steps) kStepsByFactors[F - 1](blocks, st, dl, dh, dp, grid, dq);
-        hipLaunchKernelGGL(k_sw_final, dim3((unsigned)n), dim3(kSwThreads), 0, st, dq, grid.bps,
-                           trials, dout);
-        e = hipGetLastError();
-    }
+    if (e == hipSuccess) e = launch_batch(b, at, F, grid, trials, base, dout, st);
     if (e == hipSuccess) e = hipMemcpyAsync(out.data(), dout, ob, hipMemcpyDeviceToHost, st);
     const hipError_t ef = hipFreeAsync(base, st);
     const hipError_t es = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_error(e, "bs_swaptions_host_f64");
     if (ef != hipSuccess) return hip_error(ef, "hipFreeAsync");
     if (es != hipSuccess) return hip_error(es, "hipStreamSynchronize");
-    for (size_t k = 0; k < n; ++k) {
-        price[b.index[k]] = out[2 * k];
-        std_error[b.index[k]] = out[2 * k + 1];
-    }
-    return BS_OK;
+    return deliver(out.data());
 }
 
 }  // namespace

@@ -220,3 +220,35 @@ def test_rates_past_the_linear_bound(gpu):
     p, e = W.price([wide, sw(strike=0.13)], 3000, 31)
     for i, s in enumerate((wide, sw(strike=0.13))):
         check((p[i], e[i]), S.price_blocking(s, 31 + i, 3000), i)
+
+
+def test_calls_from_more_threads_than_workspaces(gpu):
+    import threading
+    sets = [W.parsec_portfolio(8 + k, 1979 + k) for k in range(8)]
+    want = [W.price(s, 3000, base) for s, base in sets]
+    bad = []
+
+    def work(k):
+        st = gpu.Stream()
+        for _ in range(20):
+            p, e = W.price(sets[k][0], 3000, sets[k][1], stream=st.handle)
+            if not (np.array_equal(p, want[k][0]) and np.array_equal(e, want[k][1])):
+                bad.append(k)
+        st.destroy()
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad, bad
+
+
+def test_parameters_past_a_workspace(gpu):
+    """6000 swaptions have more parameters than a workspace's 1 MB: the same
+    bits as the call in pieces that fit."""
+    sws, base = W.parsec_portfolio(6000)
+    p, e = W.price(sws, 64, base)
+    for lo in range(0, 6000, 500):
+        q, f = W.price(sws[lo:lo + 500], 64, base + lo)
+        assert np.array_equal(p[lo:lo + 500], q) and np.array_equal(e[lo:lo + 500], f), lo
