@@ -222,6 +222,12 @@ def test_rates_past_the_linear_bound(gpu):
         check((p[i], e[i]), S.price_blocking(s, 31 + i, 3000), i)
 
 
+def same_bits(a, b):
+    # a trial count that is no multiple of the block makes some of the
+    # reference's standard errors the root of a negative number
+    return np.array_equal(a.view(np.uint64), b.view(np.uint64))
+
+
 def test_calls_from_more_threads_than_workspaces(gpu):
     import threading
     sets = [W.parsec_portfolio(8 + k, 1979 + k) for k in range(8)]
@@ -232,7 +238,7 @@ def test_calls_from_more_threads_than_workspaces(gpu):
         st = gpu.Stream()
         for _ in range(20):
             p, e = W.price(sets[k][0], 3000, sets[k][1], stream=st.handle)
-            if not (np.array_equal(p, want[k][0]) and np.array_equal(e, want[k][1])):
+            if not (same_bits(p, want[k][0]) and same_bits(e, want[k][1])):
                 bad.append(k)
         st.destroy()
 
@@ -251,4 +257,4 @@ def test_parameters_past_a_workspace(gpu):
     p, e = W.price(sws, 64, base)
     for lo in range(0, 6000, 500):
         q, f = W.price(sws[lo:lo + 500], 64, base + lo)
-        assert np.array_equal(p[lo:lo + 500], q) and np.array_equal(e[lo:lo + 500], f), lo
+        assert same_bits(p[lo:lo + 500], q) and same_bits(e[lo:lo + 500], f), lo
