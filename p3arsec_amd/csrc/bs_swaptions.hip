@@ -37,7 +37,7 @@
 // A = 16807 * 1513517, the same residues as its Schrage factorisation, so the
 // residue of the next counter is one 32-bit addition away.
 //
-// Kernels (the caller's stream): k_sw_paths, 4 to 16 paths per work-item, and,
+// Kernels (the caller's stream): k_sw_paths, 2 to 16 paths per work-item, and,
 // where it left blocks out, k_sw_paths_steps, each block's sums of payoff and
 // payoff^2 folded in a fixed order into one partial; k_sw_final, one block per
 // swaption, adds its partials in a fixed order and forms the mean and standard
@@ -61,7 +61,7 @@ namespace bs {
 namespace {
 
 constexpr int kSwThreads = 256;
-constexpr int kSwRows = 4;                // fewest paths per work-item
+constexpr int kSwRows = 4;                // paths per work-item that limits are stated in
 constexpr int kSwMaxSteps = 64;           // n_steps
 constexpr int kSwMaxFactors = 8;          // n_factors
 constexpr int kSwMaxDraws = 64;           // start index x n_factors
@@ -531,7 +531,8 @@ __device__ __forceinline__ void linear_form(const SwLin& h, const double* __rest
     if constexpr (W <= 4) {
         const uint32_t wl = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / 64) *
                             (kSwBatch * 64 * 8);
-        if (h.draws <= 3) return linear_paths<W, 4, 3>(h, q, xb, p0, grid, lds, wl, sum, sumsq);
+        if (h.draws <= 3 && grid.rows >= 4)
+            return linear_paths<W, 4, 3>(h, q, xb, p0, grid, lds, wl, sum, sumsq);
         if (h.draws <= 6) return linear_paths<W, 2, 6>(h, q, xb, p0, grid, lds, wl, sum, sumsq);
     }
     linear_wide<W>(h, q, xb, p0, grid, lds, sum, sumsq);
@@ -752,30 +753,29 @@ void pack_swaption(const bs_swaption_t& s, const SwShape& x, int64_t seed, SwHea
     // forward curve from the yield curve
     f0[0] = s.yield[0];
     for (int j = 1; j < n; ++j) f0[j] = (j + 1) * s.yield[j] - j * s.yield[j - 1];
-    // drifts: sum_{l<=j} mu_k[l] = dt/2 (sum_{l<=j} sigma_k[l])^2, then the total
-    std::vector<double> drift((size_t)F * w);
+    // drifts: sum_{l<=j} mu_k[l] = dt/2 (sum_{l<=j} sigma_k[l])^2, then the total;
+    // the running sums d and vol add in the order of the reference's own loops
+    double drift[kSwMaxFactors][kSwMaxSteps];
     for (int k = 0; k < F; ++k) {
         const double* fk = s.factors + (size_t)k * w;
-        double* dk = drift.data() + (size_t)k * w;
+        double* dk = drift[k];
         dk[0] = 0.5 * dt * fk[0] * fk[0];
+        double d = 0, vol = 0 + fk[0];
         for (int j = 1; j < w; ++j) {
-            double d = 0;
-            for (int l = 0; l < j; ++l) d -= dk[l];
-            double vol = 0;
-            for (int l = 0; l <= j; ++l) vol += fk[l];
+            d -= dk[j - 1];
+            vol += fk[j];
             dk[j] = d + 0.5 * dt * vol * vol;
         }
         for (int l = 0; l < w; ++l) sig[(size_t)k * w + l] = fk[l];
     }
     for (int l = 0; l < w; ++l) {
         double t = 0;
-        for (int k = 0; k < F; ++k) t += drift[(size_t)k * w + l];
+        for (int k = 0; k < F; ++k) t += drift[k][l];
         mudt[l] = t * dt;
     }
     for (int l = 0; l < L; ++l) pay[l] = 0.0;
-    for (int l = freq; l <= points; l += freq)
-        pay[l] = l != points ? exp(strike_cont * s.payment_interval) - 1
-                             : exp(strike_cont * s.payment_interval);
+    const double grow = exp(strike_cont * s.payment_interval);
+    for (int l = freq; l <= points; l += freq) pay[l] = l != points ? grow - 1 : grow;
 }
 
 // Appends the linear form of the swaption that pack_swaption packed at h:
@@ -1107,22 +1107,29 @@ extern "C" int bs_swaptions_host_f64(const bs_swaption_t* sw, int64_t n, int64_t
                              "more than 2^24 blocks of 1024 paths (2^34 paths) in one call");
         // Paths per work-item: enough of them to spread the 100 or so
         // instructions of its set-up while several rounds of blocks are left
-        // (1024 are resident at once).  128 swaptions x 1M trials take 931 us
-        // with 4 rows, 844 with 8, 812 with 16 and 805 with 32; 32 swaptions x
-        // 50,000 trials (starts at steps 1-10, 4 factors) 171, 190, 282 and 468.
-        const int rows = bps_most * n >= 65536 ? 16 : bps_most * n >= 16384 ? 8 : kSwRows;
+        // (1024 are resident at once), and 2 where 4 would leave the chip
+        // idle.  Rows 2, 4, 8, 16 and 32: 8 swaptions x 50,000 trials (starts at
+        // steps 1-12, 4 factors; 392 blocks of 4 rows) 52, 70 and 107 us; 64 x
+        // 20,000 (1280 blocks) 51, 50, 51; 128 x 1M 931 with 4, 844, 812, 805;
+        // 32 x 50,000 (starts at steps 1-10, 1568 blocks) 126, 126, 140.
+        const int64_t blocks4 = bps_most * n;
+        const int rows = blocks4 >= 65536 ? 16 : blocks4 >= 16384 ? 8 : blocks4 >= 1024 ? 4 : 2;
         const int64_t bps = (paths + kSwThreads * rows - 1) / (kSwThreads * rows);
         // the swaptions whose paths cost most first, so that the launch ends on
         // its cheapest blocks
-        std::vector<int32_t> order((size_t)n);
-        for (int64_t i = 0; i < n; ++i) order[(size_t)i] = (int32_t)i;
-        auto cost = [&](int32_t i) {
+        std::vector<int32_t> order((size_t)n), cost((size_t)n);
+        bool even = true;
+        for (int64_t i = 0; i < n; ++i) {
             const SwShape& x = shapes[(size_t)i];
             const int W = lin_width(x.points / x.freq);
-            return x.m * F * (45 + W) + 20 * W;
-        };
-        std::stable_sort(order.begin(), order.end(),
-                         [&](int32_t a, int32_t b) { return cost(a) > cost(b); });
+            order[(size_t)i] = (int32_t)i;
+            cost[(size_t)i] = x.m * F * (45 + W) + 20 * W;
+            even = even && cost[(size_t)i] == cost[0];
+        }
+        if (!even)
+            std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
+                return cost[(size_t)a] > cost[(size_t)b];
+            });
         // parameters of more than 2^24 doubles go in several launches
         for (size_t first = 0; first < (size_t)n;) {
             SwBatch batch;
