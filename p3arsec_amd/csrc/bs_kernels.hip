@@ -404,9 +404,11 @@ hipError_t launch_price_f64(SoaIn<double> in, const uint8_t* type, double* out, 
 
 hipError_t launch_greeks_f32(SoaIn<float> in, const uint8_t* type, GreeksOut out, int64_t n,
                              hipStream_t st) {
-    // four options per work-item: 16-byte stores of the five outputs (65.5 against
-    // 66.5 us per 10M-option pass with two per work-item)
-    return launch_stream<GreeksF32>(GreeksArgs{in, type, out}, n, 4, st);
+    // Two options per work-item (8-byte agent-scope stores, 11 KB of LDS reserved per
+    // wave) against four (16-byte non-temporal stores, 16 KB), on one stream: 1M
+    // options 8.6 and 10.1 us, 3M 20.5 and 23.2, 6M 41.9 and 43.0, 10M 66.9 and
+    // 68.3, 30M 197.6 and 199; 10M on two streams 66.8 both.
+    return launch_stream<GreeksF32>(GreeksArgs{in, type, out}, n, 2, st);
 }
 
 hipError_t launch_cndf_f32(const float* x, float* out, int64_t n, hipStream_t st) {
