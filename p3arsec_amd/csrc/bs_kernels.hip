@@ -176,6 +176,12 @@ uintptr_t address(const T* p) { return reinterpret_cast<uintptr_t>(p); }
 // array's groups of vw elements are then aligned to their size.
 template <class Args>
 int head_for(const Args& a, int64_t n, int vw, bool* aligned) {
+    uintptr_t low = 0;
+    each(a, [&](auto* p) { low |= address(p); });
+    if (low % 128 == 0) {   // whole arrays from the allocator: nothing to align
+        *aligned = true;
+        return 0;
+    }
     int64_t head = -1;
     bool as_is = true;
     each(a, [&](auto* p) {

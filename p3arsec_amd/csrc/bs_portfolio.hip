@@ -14,15 +14,10 @@
 // w*value to FP64 accumulators; each wave folds its lanes with a fixed
 // wave sum and the block its waves in order into one partial.  The last block
 // of every 64 to arrive folds their partials with one wave sum, and the last
-// of those folds the groups of 64: no second launch, and nothing waits.  The
+// of those folds the groups of 64 (bs_arrive.hpp): no second launch, and nothing
+// waits.  The
 // shape of the sum depends only on n, so the sums are bit-reproducible for a
 // given book, wherever its arrays start.
-//
-// A partial goes out as relaxed agent-scope stores (written through to memory,
-// past the L2 of the block's die), the wave waits for their acknowledgement,
-// then counts itself in with a relaxed agent-scope add; the block that counts
-// last loads the partials at the same scope.  A release fence in place of the
-// wait would write back the die's whole L2 for every block.
 //
 // Scratch (counters and partials): slots of a fixed device array, claimed on
 // the host by a flag in pinned memory that the kernel's last block clears, so
@@ -38,6 +33,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "bs_arrive.hpp"
 #include "bs_internal.hpp"
 #include "bs_math.hpp"
 #include "bs_ops.hpp"
@@ -61,7 +57,7 @@ struct PfArgs {
 };
 
 // A call's scratch in the one-launch form; the counters are zero between calls,
-// 256 bytes apart: adds from all dies to one line take turns, about 25 ns each.
+// 256 bytes apart.
 struct PfCounter {
     uint32_t done;
     uint32_t pad[63];
@@ -141,31 +137,6 @@ __device__ __forceinline__ double wave_sum(double x) {
     x += dpp<0x143, 0xc>(x);
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
                             __builtin_amdgcn_readlane(__double2loint(x), 63));
-}
-
-template <class T>
-__device__ __forceinline__ T agent_load(const T* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <class T>
-__device__ __forceinline__ void agent_store(T* p, T v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Waits until this wave's stores have been acknowledged.
-__device__ __forceinline__ void stores_done() {
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0);
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
-// Counts this wave in; true in the one that makes `full`.
-__device__ __forceinline__ bool arrive(uint32_t* counter, uint32_t full) {
-    uint32_t before = 0;
-    if ((threadIdx.x & 63) == 0)
-        before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)before) == full - 1;
 }
 
 // One wave's sums of NQ quantities: of group g's partials, and of the groups'.
@@ -263,7 +234,7 @@ void k_pf_rows(PfArgs a, PfSlot* slot, uint32_t* busy, double* __restrict__ sums
     if (lane < NQ) sums[lane] = pick(x, lane);
     if (lane == 0) agent_store(&slot->groups.done, 0u);
     stores_done();
-    if (lane == 0) __hip_atomic_store(busy, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (lane == 0) system_store(busy, 0u);
 }
 
 // The second launch of the two-launch form: one block folds the partials, a

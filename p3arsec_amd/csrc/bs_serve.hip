@@ -33,6 +33,7 @@
 #include <string>
 #include <vector>
 
+#include "bs_arrive.hpp"
 #include "bs_internal.hpp"
 #include "bs_math.hpp"
 #include "bs_ops.hpp"
@@ -147,9 +148,7 @@ void k_serve(const uint8_t* __restrict__ slot) {
 // memory (copy kernel, marker, interrupt), five of them for a Greeks request:
 // a round of 32 requests of up to 64K options, one third with Greeks, submitted,
 // waited for and copied out one by one takes 390 us, with those copies 1050.
-// Bound by the launch and the link's latency.  Every store is a relaxed
-// system-scope one (written through), acknowledged before the block counts
-// itself in.
+// Bound by the launch and the link's latency.
 constexpr int kReplies = 2;                         // replies on their way at once
 constexpr size_t kReplyBytes = size_t(3) << 19;     // 1.5 MB: the Greeks of 64K options
 constexpr int kReplyBlocks = 64;
@@ -159,16 +158,12 @@ __global__ __launch_bounds__(kThreads) void k_reply(const uint64_t* __restrict__
                                                     uint32_t* count, uint32_t* flag,
                                                     uint32_t seq) {
     for (int i = blockIdx.x * kThreads + threadIdx.x; i < words; i += gridDim.x * kThreads)
-        __hip_atomic_store(dst + i, src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0);   // this wave's stores are acknowledged
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        system_store(dst + i, src[i]);
+    stores_done();
     __syncthreads();
-    if (threadIdx.x == 0 &&
-        __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-            gridDim.x - 1) {
-        __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(flag, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x == 0 && arrive_one(count, gridDim.x)) {
+        agent_store(count, 0u);   // for the next reply, which the stream orders behind this one
+        system_store(flag, seq);
     }
 }
 

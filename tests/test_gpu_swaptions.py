@@ -258,3 +258,21 @@ def test_parameters_past_a_workspace(gpu):
     for lo in range(0, 6000, 500):
         q, f = W.price(sws[lo:lo + 500], 64, base + lo)
         assert same_bits(p[lo:lo + 500], q) and same_bits(e[lo:lo + 500], f), lo
+
+
+@pytest.mark.parametrize("count,trials", [(1, 1), (511, 600), (512, 600), (513, 600),
+                                          (64, 131_072), (64, 131_200), (65, 131_072)])
+def test_both_ends_of_a_launch_give_the_same_bits(gpu, count, trials):
+    """A launch whose last blocks form the results (up to 512 swaptions and 8192
+    blocks) against the same swaptions one by one and in halves."""
+    sws, base = W.parsec_portfolio(count)
+    p, e = W.price(sws, trials, base, 1)
+    q, f = W.price(sws[:1], trials, base, 1)
+    check((p[0], e[0]), (q[0], f[0]), "first")
+    half = (count + 1) // 2
+    if half < count:
+        q, f = W.price(sws[half:], trials, base + half, 1)
+        for i in (0, count - half - 1):
+            check((p[half + i], e[half + i]), (q[i], f[i]), i)
+    again = W.price(sws, trials, base, 1)
+    assert same_bits(p, again[0]) and same_bits(e, again[1])
