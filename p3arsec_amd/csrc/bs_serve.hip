@@ -8,7 +8,9 @@
 //   * per batch, a stage kernel that copies the slot's table from pinned host
 //     memory to the device, then one fused kernel per section (the batch's
 //     price requests, its Greeks requests): a block prices one tile of 512
-//     options of one request, found by a 64-ary wave search of the table.
+//     options of one request, found by a 64-ary wave search of the table.  A
+//     batch of at most 32 requests and 2048 tiles is one kernel with the table
+//     as its argument.
 //     Launched directly (the default) each section's grid is one block per
 //     tile.  With use_graph the three kernels are captured once per slot and
 //     each batch is one hipGraphLaunch; before it, each section's node gets
@@ -172,6 +174,44 @@ __global__ void k_zero_word(uint32_t* p) { *p = 0; }
 using ServePrice = PriceF32<Ref32, kVW>;
 using ServeGreeks = GreeksF32<kVW>;
 
+// A small batch in one launch: its table travels as the kernel's argument, and
+// one grid holds the price section's tiles, then the Greeks section's.  The
+// stage kernel and a kernel per section cost 14 us of GPU time and two launches
+// for requests that price in 3: at 20,000 Poisson requests/s p50 is 20.6 us and
+// was 25, at 300,000 27-35 and 48 (p99 92-108 and 130).  Larger batches keep
+// those (at saturation one kernel for both sections, at the Greeks form's
+// registers, ran 1.73e11 options/s against 1.76e11).
+constexpr int kSmallDesc = 32;
+constexpr int64_t kSmallTiles = 2048;
+struct SmallBatch {
+    int32_t np, nd;         // price requests, all requests
+    int32_t price_tiles, pad;
+    Desc d[kSmallDesc];     // price requests first; tile_begin counts through the batch
+};
+static_assert(sizeof(SmallBatch) <= 4096, "fits a kernel's arguments");
+
+template <int kThr>
+__global__ __launch_bounds__(kThr) __attribute__((amdgpu_waves_per_eu(waves_for<ServeGreeks, false>())))
+void k_serve_small(const SmallBatch b) {
+    const int64_t t = blockIdx.x;
+    const int lane = threadIdx.x & 63;
+    const uint64_t before = __ballot(lane < b.nd && b.d[lane < kSmallDesc ? lane : 0].tile_begin <= t);
+    const Desc& x = b.d[__builtin_amdgcn_readfirstlane(__popcll(before) - 1)];
+    const int64_t n = x.n;
+    const int64_t g = (t - x.tile_begin) * kThr + threadIdx.x;
+    if (t < b.price_tiles) {
+        const ServePrice op = op_of<ServePrice>(x);
+        if ((g + 1) * kVW <= n) op.template finish<true>(g, op.template load<true>(g));
+        else
+            for (int64_t i = g * kVW; i < n; ++i) op.scalar(i);
+    } else {
+        const ServeGreeks op = op_of<ServeGreeks>(x);
+        if ((g + 1) * kVW <= n) op.template finish<true>(g, op.template load<true>(g));
+        else
+            for (int64_t i = g * kVW; i < n; ++i) op.scalar(i);
+    }
+}
+
 // The fused kernel of section sec with kThr threads per block.
 template <int kThr>
 const void* serve_fn(int sec) {
@@ -181,6 +221,11 @@ const void* serve_fn(int sec) {
 const void* serve_fn(int threads, int sec) {
     return threads == 64 ? serve_fn<64>(sec) : threads == 128 ? serve_fn<128>(sec)
                                                                 : serve_fn<256>(sec);
+}
+const void* small_fn(int threads) {
+    return threads == 64    ? reinterpret_cast<const void*>(&k_serve_small<64>)
+           : threads == 128 ? reinterpret_cast<const void*>(&k_serve_small<128>)
+                            : reinterpret_cast<const void*>(&k_serve_small<256>);
 }
 
 }  // namespace
@@ -382,6 +427,18 @@ struct HipExec {
                 e = set_section_grid(s, sec, (unsigned)blocks);
             }
             if (e == hipSuccess) e = hipGraphLaunch(graph[s], st);
+        } else if (h->ndesc[0] + h->ndesc[1] <= kSmallDesc &&
+                   h->tiles[0] + h->tiles[1] <= std::min(kSmallTiles, grid_cap)) {
+            SmallBatch b;
+            b.np = h->ndesc[0];
+            b.nd = h->ndesc[0] + h->ndesc[1];
+            b.price_tiles = (int32_t)h->tiles[0];
+            b.pad = 0;
+            ::memcpy(b.d, host_slot[s] + sizeof(SlotHeader), sizeof(Desc) * (size_t)b.nd);
+            for (int i = b.np; i < b.nd; ++i) b.d[i].tile_begin += h->tiles[0];
+            void* args[1] = {&b};
+            e = hipLaunchKernel(small_fn(threads), dim3((unsigned)(h->tiles[0] + h->tiles[1])),
+                                dim3(threads), args, 0, st);
         } else {
             hipLaunchKernelGGL(k_stage, dim3(kStageBlocks), dim3(kThreads), 0, st,
                                reinterpret_cast<const uint4*>(host_slot_dev[s]),

@@ -359,3 +359,30 @@ def test_results_reach_the_host_whole(gpu, n):
         x.join()
     assert not bad, bad
     ctx.destroy()
+
+
+@pytest.mark.parametrize("sizes", [
+    (1,), (511, 512, 513), (2, 1, 1025) + (700,) * 28, (3, 65_536) + (513,) * 30,
+    (5,) * 33, (1,) * 40,
+    (1_048_576,), (1_048_577,), (1_047_552, 1024), (1_047_552, 1025), (1_048_064, 512, 1),
+])
+def test_small_batches_in_one_launch(gpu, sizes):
+    """Batches on both sides of 32 requests and of 2048 tiles of 512 options,
+    price and Greeks sections mixed, in one lane: the bits of each book alone."""
+    bks = [books.make_book(n, books.SEED_BASE + 96 + i) for i, n in enumerate(sizes)]
+    want = {}
+    for kinds in ([1] * len(sizes), [2] * len(sizes), [1 + i % 2 for i in range(len(sizes))]):
+        ctx = Ctx(gpu, 128 << 20, use_graph=0, small=-1)
+        ids = [ctx.register(b) for b in bks]
+        n = len(sizes)
+        tickets = (i64 * n)()
+        gpu.call("bs_submit_many", ctx.h, (i64 * n)(*ids), (ctypes.c_int * n)(*kinds), None, n,
+                 tickets)
+        for i in range(n):
+            assert ctx.wait(tickets[i]) == 0
+            if i not in want:
+                want[i] = [o.download(np.uint32, sizes[i])
+                           for o in gpu.greeks(gpu.DeviceBook(bks[i]))]
+            for a, b in zip(ctx.result(tickets[i], sizes[i], kinds[i]), want[i]):
+                assert np.array_equal(a.view(np.uint32), b), (i, kinds[i])
+        ctx.destroy()
