@@ -125,7 +125,9 @@ __device__ __forceinline__ float exp_hw(float x) { return __builtin_amdgcn_exp2f
 __device__ __forceinline__ float log_hw(float x) { return __builtin_amdgcn_logf(x) * kLn2f; }
 
 // dCNDF/dx of the A&S approximation, given |x|, k = 1/(1+p|x|), the
-// polynomial P(k) and n(x):  g = n (|x| P + p k^2 P'(k)).  Float, Horner.
+// polynomial P(k) and n(x):  g = n (|x| P + p k^2 P'(k)).  Float, Horner.  (With
+// p in the coefficients it takes two multiplications fewer and vega and theta
+// come out 1% further from 64 bits.)
 __device__ __forceinline__ float cndf_grad(float ax, float k, float poly, float n) {
     float dp = __builtin_fmaf(k, float(5.0 * kB5), float(4.0 * kB4));
     dp = __builtin_fmaf(k, dp, float(3.0 * kB3));
@@ -493,28 +495,38 @@ struct Greeks32 {
 //   den = sigma sqrt(T),  A = (r + sigma^2/2) T + log(S/K).
 // Outputs: delta = dP/dS, vega = dP/dsigma, rho = dP/dr, theta = -dP/dT (per
 // year); vega and rho are per unit change, not per percent.
+//
+// The halves a_i that bs_combine_split multiplies S and FV by serve both option
+// types: with s_bar = +-a1 and z = +-FV a2 (minus for a put) the price is
+// S s_bar - z, the direct part of delta is s_bar (N1, or N1 - 1 for a put,
+// exactly), and dP/dFV FV is -z: 11 instructions fewer than from N1 and N2
+// (10M-option sums with Greeks and weights, bound by VALU issue: 54.7 us and
+// 53.2).
 template <class M, bool kSplitCombine>
 __device__ __forceinline__ Greeks32 bs_greeks_of(float s, float k, float r, float v, float t,
                                                  bool put) {
 #pragma clang fp contract(off)
     const Forward<float> f = bs_forward<M, true>(s, k, r, v, t);
     Greeks32 o;
-    if constexpr (kSplitCombine) o.price = bs_combine_split(s, f, put);
+    const float a1 = ((f.d1 < 0.0f) != put) ? 1.0f - f.y1 : f.y1;
+    const float a2 = ((f.d2 < 0.0f) != put) ? 1.0f - f.y2 : f.y2;
+    const float s_bar = put ? -a1 : a1;
+    const float z = f.fv * (put ? -a2 : a2);
+    if constexpr (kSplitCombine) o.price = s * s_bar - z;
     else o.price = bs_combine(s, f, put);
     const float rden = hw_rcp(f.den);
     // adjoints of N1 and N2 are S and -FV for both option types
-    const float s_bar0 = put ? f.n1 - 1.0f : f.n1;
-    const float fv_bar = put ? 1.0f - f.n2 : -f.n2;
-    const float d1_bar = __builtin_fmaf(s, f.g1, -(f.fv * f.g2));   // through d1 and d2
-    const float den_bar = __builtin_fmaf(-d1_bar, f.d1 * rden, f.fv * f.g2);
+    const float n2_bar = f.fv * f.g2;
+    const float d1_bar = __builtin_fmaf(s, f.g1, -n2_bar);            // through d1 and d2
     const float a_bar = d1_bar * rden;
-    const float sqrt_t_bar = den_bar * v;
-    o.delta = __builtin_fmaf(a_bar, hw_rcp(s), s_bar0);              // d log(S/K)/dS = 1/S
-    o.vega = __builtin_fmaf(den_bar, f.sqrt_t, a_bar * t * v);
-    const float fv_dr = fv_bar * f.fv;                                 // dFV = -FV (T dr + r dT)
-    o.rho = __builtin_fmaf(a_bar, t, -(fv_dr * t));
-    const float t_bar = __builtin_fmaf(a_bar, r + f.half_var,          // 1/sqrt(T) = v / den
-                                       __builtin_fmaf(0.5f * sqrt_t_bar, v * rden, -(fv_dr * r)));
+    const float den_bar = __builtin_fmaf(-a_bar, f.d1, n2_bar);
+    const float at_bar = a_bar * t;
+    o.delta = __builtin_fmaf(a_bar, hw_rcp(s), s_bar);                // d log(S/K)/dS = 1/S
+    o.vega = __builtin_fmaf(den_bar, f.sqrt_t, at_bar * v);
+    o.rho = __builtin_fmaf(z, t, at_bar);                             // dFV = -FV (T dr + r dT)
+    // 1/sqrt(T) = v / den: v/2 den_bar / sqrt(T) = den_bar v^2/2 / den
+    const float t_bar = __builtin_fmaf(a_bar, r + f.half_var,
+                                       __builtin_fmaf(den_bar * rden, f.half_var, z * r));
     o.theta = -t_bar;
     return o;
 }

@@ -182,9 +182,9 @@ struct PriceI32F32 {
 };
 
 // fptype = double: a group is VW = 2 options (one 128-bit load per array).
-// 10M options on one stream, 490 MB: 81.2 us (6.0 TB/s) at 165 VALU
+// 10M options on one stream, 490 MB: 81.2 us (6.0 TB/s) at 180 VALU
 // instructions per option and 5 waves per SIMD, where Ref64's general
-// primitives (230 instructions) took 94; with 3 waves per SIMD 82.9, not
+// primitives (248 instructions) took 94; with 3 waves per SIMD 82.9, not
 // pipelined 86.8, one option per work-item (8-byte stores) 84-87, the waves
 // capped by 8 KB of LDS each 84.
 template <int VW, bool AL = true>
