@@ -1211,10 +1211,13 @@ extern "C" int bs_swaptions_host_f64(const bs_swaption_t* sw, int64_t n, int64_t
         // (1024 are resident at once), and 2 where 4 would leave the chip
         // idle.  Rows 2, 4, 8, 16 and 32: 8 swaptions x 50,000 trials (starts at
         // steps 1-12, 4 factors; 392 blocks of 4 rows) 52, 70 and 107 us; 64 x
-        // 20,000 (1280 blocks) 51, 50, 51; 128 x 1M 931 with 4, 844, 812, 805;
-        // 32 x 50,000 (starts at steps 1-10, 1568 blocks) 126, 126, 140.
+        // 20,000 (1280 blocks) 51, 50, 51; 32 x 50,000 (starts at steps 1-10,
+        // 1568 blocks) 126, 126, 140.  Rows 16, 32 and 64: 128 x 1M (125,056
+        // blocks) 765, 755, 761, and 5202, 5208, 5295 with 24 steps, 4 factors
+        // and a start at step 8; 128 x 550,000 (68,864) 447, 441; rows 8, 32 and
+        // 64 at 128 x 500,000 (62,592) 430, 430, 431.
         const int64_t blocks4 = bps_most * n;
-        const int rows = blocks4 >= 65536 ? 16 : blocks4 >= 16384 ? 8 : blocks4 >= 1024 ? 4 : 2;
+        const int rows = blocks4 >= 65536 ? 32 : blocks4 >= 16384 ? 8 : blocks4 >= 1024 ? 4 : 2;
         const int64_t bps = (paths + kSwThreads * rows - 1) / (kSwThreads * rows);
         // the swaptions whose paths cost most first, so that the launch ends on
         // its cheapest blocks
