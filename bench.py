@@ -81,8 +81,8 @@ def measured_traffic(kernel: str, n: int):
 LAUNCH_CPU_US = {}
 # Streams the passes of each map alternate over, the faster schedule measured
 # on MI355X (10M options, 300 passes): price 37.25 / 37.52 us per pass on two
-# streams vs 37.98 / 39.41 on one (two boxes); Greeks 67.22 vs 67.98; FP64
-# 85 vs 89.  Over 20 passes the two schedules of the price map are within
+# streams vs 37.98 / 39.41 on one (two boxes); Greeks 66.4 vs 67.0; FP64
+# 74.9 vs 79.3.  Over 20 passes the two schedules of the price map are within
 # about 1 us of each other, either way round depending on the box.
 STREAMS = {"price": 2, "fast": 2, "greeks": 2, "fp64": 2}
 
@@ -425,9 +425,9 @@ def serve_bench(result: dict) -> dict:
         "p99_ms_le64k_20k": {"direct": d["p99_ms_le64k"], "graph_replay": g["p99_ms_le64k"]},
         "saturation_options_per_s": {"direct": out["saturation"]["options_per_s"],
                                      "graph_replay": out["saturation_graph"]["options_per_s"]},
-        "why": "graph replay costs more host time per launch than the three direct launches "
-               "it replaces, which sets the low-load latency; at saturation both forms reach "
-               "the same throughput"}
+        "why": "graph replay costs more host time per batch than the one direct launch of a "
+               "small batch or the three of a large one, which sets the low-load latency; at "
+               "saturation both forms reach the same throughput"}
     return out
 
 
@@ -448,7 +448,7 @@ def swaptions_bench(no_cpu: bool, calls: int = 5) -> dict:
     W.price(sws[:4], 10_000, base)            # first call: code object load
     prep = W.Prepared(sws)                    # the records, built once as the driver does
     st, e0, e1 = capi.Stream(), capi.Event(), capi.Event()
-    for _ in range(6):                        # clocks settle over ~20 ms of load
+    for _ in range(40):                       # clocks settle over ~30 ms of load
         W.price(prep, SW_TRIALS, base, stream=st.handle)
     wall, gpu = [], []
     for _ in range(calls):
@@ -669,18 +669,18 @@ def config4096_section(L, streams) -> dict:
     dsm, osm = capi.DeviceBook(small), capi.alloc_out(4096)
     t4 = timed_passes(lambda i, s: capi.check(L.bs_price_f32(*dsm.ptrs(), osm.ptr, 4096, s),
                                               "4096"), 1, 100, 100, streams[:1])
-    # the 100 passes as one call: replayed from a captured graph
+    # the 100 passes as one call, one launch
     sp = dsm.ptrs()
-    t4g = timed_passes(lambda i, s: capi.check(L.bs_price_passes_f32(
-        *sp[:5], sp[5], 1, osm.ptr, 4096, 100, s), "4096 graph"), 1, 20, 5, streams[:1]) / 100
+    t4p = timed_passes(lambda i, s: capi.check(L.bs_price_passes_f32(
+        *sp[:5], sp[5], 1, osm.ptr, 4096, 100, s), "4096 passes"), 1, 20, 5, streams[:1]) / 100
     p4 = osm.download(np.float32, 4096).astype(np.float64)
     e4 = np.abs(p4 - pyoracle.price_exact(small))
     r4, _, _ = pyoracle.price_f32(small)
     dsm.free()
     osm.free()
-    return {"us_per_pass": t4g * 1e3, "options_per_s": 4096 / (t4g * 1e-3),
-            "ms_100_passes": t4g * 100, "passes": 100,
-            "form": "bs_price_passes_f32 (100 passes, graph replay)",
+    return {"us_per_pass": t4p * 1e3, "options_per_s": 4096 / (t4p * 1e-3),
+            "ms_100_passes": t4p * 100, "passes": 100,
+            "form": "bs_price_passes_f32 (100 passes, one launch)",
             "us_per_pass_launch_by_launch": t4 * 1e3,
             "max_err_vs_fp64_closed_form": float(e4.max()),
             "mean_err_vs_fp64_closed_form": float(e4.mean()),

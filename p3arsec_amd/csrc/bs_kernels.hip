@@ -410,11 +410,15 @@ hipError_t launch_price_f64(SoaIn<double> in, const uint8_t* type, double* out, 
 
 hipError_t launch_greeks_f32(SoaIn<float> in, const uint8_t* type, GreeksOut out, int64_t n,
                              hipStream_t st) {
-    // Two options per work-item (8-byte agent-scope stores, 11 KB of LDS reserved per
-    // wave) against four (16-byte non-temporal stores, 16 KB), on one stream: 1M
-    // options 8.6 and 10.1 us, 3M 20.5 and 23.2, 6M 41.9 and 43.0, 10M 66.9 and
-    // 68.3, 30M 197.6 and 199; 10M on two streams 66.8 both.
-    return launch_stream<GreeksF32>(GreeksArgs{in, type, out}, n, 2, st);
+    // Two options per work-item (8-byte agent-scope stores, 11 KB of LDS reserved
+    // per wave) for what the 256 MB last-level cache takes in one launch, four
+    // (16-byte non-temporal stores, 16 KB) for streams past it.  us on one / two
+    // streams, two against four: 1M options 8.4 / 6.2 and 10.2 / 7.0, 3M 20.2 / 18.1
+    // and 23.1 / 20.2, 4M 30.4 / 28.9 and 30.7 / 28.7, 4.4M 32.5 / 32.3 and 32.4 /
+    // 30.1, 7M 48.8 / 47.4 and 48.6 / 46.7, 10M 67.0 / 66.5 and 68.0 / 66.0, 20M
+    // 132.3 / 135.2 and 133.0 / 132.5, 40M 259.2 / 269.8 and 261.2 / 262.5.
+    const int vw = n < (int64_t(1) << 22) ? 2 : 4;
+    return launch_stream<GreeksF32>(GreeksArgs{in, type, out}, n, vw, st);
 }
 
 hipError_t launch_cndf_f32(const float* x, float* out, int64_t n, hipStream_t st) {

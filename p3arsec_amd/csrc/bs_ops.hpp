@@ -17,14 +17,15 @@
 // two streams, with the agent-scope stores below: price (Ref32) 64 threads,
 // no LDS reserved 37.98 / 37.25 us (6 KB per wave: 38.64 / 37.90; 7 KB:
 // 40.1 / 39.3); Fast32 64 threads, 6 KB 37.56 / 36.95 us (none: 39.06 /
-// 37.80); Greeks 64 threads, two options per work-item, 11 KB per wave 66.9 /
-// 66.8 us (none: 74.16 / 73.79; 9 KB: 68.18 / 68.52; 12 KB: 70.82 / 69.59), four
-// options per work-item, 16 KB per wave 68.3 / 66.8 (14 KB: 67.8 / 67.5; 18 KB:
-// 72; none: 77); int32-type price 64
+// 37.80); Greeks 64 threads, four options per work-item, 16 KB per wave 67.9 /
+// 65.9 us (15 KB: 67.3 / 66.0-66.7; 14 KB: 67.3 / 66.2; 18 KB: 72; none: 77),
+// two options per work-item, 11 KB per wave 66.9 / 66.8 (none: 74.16 / 73.79;
+// 9 KB: 68.2 / 68.7; 10 KB: 68.3 / 68.8; 12 KB: 67.9 / 67.4; the faster form
+// of books under 2^22 options); int32-type price 64
 // threads 44.9 us; FP64 below.  Small blocks help:
 // one-wave workgroups retire and refill independently, so the tail of the
 // grid is short.  Fewer resident waves help the write-heavy Greeks stream
-// most: with 14 waves per CU instead of 32 its five output streams keep fewer
+// most: with 10 waves per CU instead of 32 its five output streams keep fewer
 // DRAM pages open at once.
 #pragma once
 #include <type_traits>
@@ -232,7 +233,7 @@ template <int VW, bool AL = true>
 struct GreeksF32 {
     static constexpr int kVW = VW;
     static constexpr int kElemBytes = 4;   // widest array element
-    // VW = 2 (the launcher's choice): 14 waves per CU; VW = 4 (16-byte stores): 10
+    // VW = 2 (books under 2^22 options): 14 waves per CU; VW = 4 (16-byte stores): 10
     static constexpr int kLdsPerWave = VW == 4 ? 16384 : 11264;
     static constexpr int kWaves = VW == 4 ? 5 : 8;
     static constexpr int kThreadsPref = 64;

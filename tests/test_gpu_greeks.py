@@ -106,6 +106,35 @@ def test_greeks_ragged_and_misaligned(gpu, n):
     assert np.array_equal(base, mis)
 
 
+@pytest.mark.parametrize("n", [(1 << 22) - 1, 1 << 22, (1 << 22) + 3])
+def test_width_by_size_gives_the_same_bits(gpu, n):
+    """Books from 2^22 options on take four options per work-item, smaller ones
+    two: on both sides of the line, whole and from an odd option on, the
+    outputs are those of either width, to the bit."""
+    db = gpu.DeviceBook(books.make_book(n, books.SEED_BASE + 5))
+    outs = [gpu.DeviceBuffer(4 * n) for _ in range(5)]
+    old = gpu.get_config(gpu.CFG_VECTOR_WIDTH)
+    try:
+        for first in (0, 3):
+            got = []
+            for width in (0, 2, 4):
+                gpu.set_config(gpu.CFG_VECTOR_WIDTH, width)
+                for o in outs:
+                    gpu.call("bs_memset", o.ptr, 0xff, 4 * n, None)
+                p = db.ptrs()
+                gpu.call("bs_price_greeks_f32", *[a + 4 * first for a in p[:5]], p[5] + first,
+                         *[o.ptr + 4 * first for o in outs], n - first, None)
+                got.append(np.stack([o.download(np.uint32, n) for o in outs]))
+            assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2]), first
+            assert np.all(got[0][:, :first] == 0xffffffff)
+            assert np.all(np.isfinite(got[0][:, first:].view(np.float32)))
+    finally:
+        gpu.set_config(gpu.CFG_VECTOR_WIDTH, old)
+        for o in outs:
+            o.free()
+        db.free()
+
+
 def test_price_output_on_degenerate_inputs(gpu):
     """On the degenerate book (T = 0, sigma = 0, zero and infinite S and K,
     NaN), the fused kernel's price output equals bs_price_f32's bit for bit,
