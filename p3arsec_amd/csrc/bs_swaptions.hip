@@ -37,7 +37,7 @@
 // A = 16807 * 1513517, the same residues as its Schrage factorisation, so the
 // residue of the next counter is one 32-bit addition away.
 //
-// Kernels (the caller's stream): k_sw_paths, 2 to 16 paths per work-item, and,
+// Kernels (the caller's stream): k_sw_paths, 2 to 32 paths per work-item, and,
 // where it left blocks out, k_sw_paths_steps, each block's sums of payoff and
 // payoff^2 folded in a fixed order into one partial; a swaption's partials are
 // added in a fixed order and its mean and standard error formed as the
@@ -612,11 +612,11 @@ __device__ __forceinline__ void linear_form(const SwLin& h, const double* __rest
 
 // Bound by FP64 issue (parameters and partial sums are all it reads and
 // writes): PARSEC's native run, 128 swaptions x 1M trials with 3 or 6 draws and
-// 1 to 3 cash flows, takes 0.80 ms at 200 VALU instructions per path, and
+// 1 to 3 cash flows, takes 0.755 ms at 195 VALU instructions per path, and
 // took 3.31 ms at 928 in the form that followed the forward-rate chains (a
 // 64-bit generator, 6 draws for every swaption, an exponential per curve
 // point); 32 swaptions x 50,000 trials with 4-40 draws 0.09 ms and 0.76 ms.
-// With 3 or 5 waves per SIMD in place of 4 the times are the same.
+// With 3 waves per SIMD in place of 4 the native run takes 0.79 ms, with 5 the same.
 template <int MAXW>
 __global__ __launch_bounds__(kSwThreads)
 __attribute__((amdgpu_waves_per_eu(MAXW <= 8 ? 4 : MAXW <= 32 ? 3 : 2))) void k_sw_paths(
