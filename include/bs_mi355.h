@@ -117,10 +117,10 @@ int bs_price_i32type_f32(const float *s, const float *k, const float *r, const f
  * BS:607-658, bs_thread's): prices the book `passes` times on `stream`, with
  * the same output as calling bs_price_f32 (otype_bytes = 1, uint8 types) or
  * bs_price_i32type_f32 (otype_bytes = 4, int32 types) `passes` times.  Every
- * pass loads, prices and stores every option, and the passes of each option
- * are in order; one launch carries them option by option, with no barrier over
- * the book between passes (small books are bound by kernel boundaries).  Where
- * price overlaps an input, each pass is a launch of its own, so that it reads
+ * pass loads, prices and stores every option.  No pass reads another's output,
+ * so one launch carries them all, with no barrier over the book between passes
+ * and side by side where the book leaves the chip idle (small books are bound
+ * by kernel boundaries).  Where price overlaps an input, each pass is a launch of its own, so that it reads
  * what the pass before it wrote. */
 int bs_price_passes_f32(const float *s, const float *k, const float *r, const float *v,
                         const float *t, const void *otype, int otype_bytes, float *price,

@@ -235,62 +235,47 @@ hipError_t launch_stream(const Args& a, int64_t n, int preferred_vw, hipStream_t
 }
 
 // ---- repeated passes ------------------------------------------------------------
-// `passes` passes over a book in one launch: a work-item owns its options and
-// prices them pass after pass, every pass loading its inputs, pricing and
-// storing.  Passes of one option are in order; no pass reads another's output
-// (the caller has checked that price overlaps no input), so options need not
-// wait for one another, and a book is read from HBM once: later passes find
-// their inputs in the caches.  TOGETHER passes are in flight at once: their
-// loads go out before their arithmetic, whose chains are then independent.
-// The compiler may not carry a value from one pass to the next: each load is
-// behind a compiler fence.
+// `passes` passes over a book in one launch: a work-item prices its options
+// pass after pass, every pass loading its inputs, pricing and storing.  No pass
+// reads another's output (the caller has checked that price overlaps no input)
+// and every pass stores the same bits, so neither options nor passes need wait
+// for one another: row y of the grid takes its share of the passes, and a book
+// that leaves the chip idle runs its passes side by side.  The stores are
+// relaxed atomics (plain stores in the machine, which cannot tear): rows on
+// different dies write one address, always with the same bits.  The compiler
+// may not carry a value from one pass to the next: each load is behind a
+// compiler fence.
 //
-// Bound by VALU issue, or by one wave's latency where a book leaves each SIMD
-// one wave or none.  100 passes, against a graph of 100 kernel nodes (1.9 us
-// each at least, the kernel boundary): 4096 options 27.4 us and 187 us, 65536
-// 29.3 and 201, 200,000 77 and 237, 1M 266 and 482; 10 passes of 10M 280 and
-// 403 us.  One pass at a time instead of four takes 35.4 us at 4096 options and
-// 39.9 at 65536; from 2 waves per SIMD on (2^17 options) it is as fast, and
-// with fewer registers faster past that (1M: 266 us against 288).
-constexpr int64_t kTogetherMaxOptions = int64_t(1) << 17;
+// Bound by VALU issue where the passes fill the chip (200,000 options x 100:
+// 52 us of it), by the launch where they don't.  100 passes, all of them in
+// one row (as many waves as the book has) / as here: 4096 options 35 / 5.7 us
+// (27.4 with four passes in flight per wave), 16,384 35 / 7.4, 65,536 38 / 20.5,
+// 131,072 44.5 / 37.4, 200,000 77.5 / 57; 10 passes of 200,000 9.8 / 8.9.  A
+// graph of 100 kernel nodes takes 1.9 us each at least, the kernel boundary:
+// 187 us at 4096 options, 201 at 65,536, 237 at 200,000, 482 at 1M (266 here).
+// Rows are added up to 16,384 waves, two rounds of them (200,000 options: 77.5
+// us with 4096, 64.3 with 8192, 56.9 with 16,384, 56.1 with 32,768; 16,384
+// options: 7.5, 7.6, 7.9, 8.3), of at least four passes each, which repay a
+// wave's start (200,000 x 10: 9.0 us with 5 a row, 9.4 with 2, 10.8 with
+// one).  Books of one row have the form without ROWS (3M x 10: 80.0 us and
+// 81.4 with it; agent-scope stores 84).
+constexpr int64_t kPassWaves = 16384;
+constexpr int kPassesPerRow = 4;
 
-template <class TY>
-struct PassIn {
-    float s, k, r, v, t;
-    TY ty;
-};
-
-template <class TY, class Ix>
-__device__ __forceinline__ PassIn<TY> load_pass(const SoaIn<float>& in, const TY* type, Ix i) {
-    asm volatile("" ::: "memory");
-    return {*at(in.s, i), *at(in.k, i), *at(in.r, i), *at(in.v, i), *at(in.t, i), *at(type, i)};
-}
-
-template <class TY, int TOGETHER, class Ix>
+template <class TY, bool ROWS, class Ix>
 __global__ __launch_bounds__(kThreads) void k_passes(SoaIn<float> in, const TY* type, float* out,
                                                      int64_t n, int passes) {
     const Ix stride = (Ix)gridDim.x * blockDim.x;
+    if constexpr (ROWS)
+        passes = (int)((int64_t)passes * (blockIdx.y + 1) / gridDim.y) -
+                 (int)((int64_t)passes * blockIdx.y / gridDim.y);
     for (Ix i = (Ix)blockIdx.x * blockDim.x + threadIdx.x; i < (Ix)n; i += stride) {
-        int p = 0;
-        for (; p + TOGETHER <= passes; p += TOGETHER) {
-            PassIn<TY> x[TOGETHER];
-            float price[TOGETHER];
-#pragma unroll
-            for (int j = 0; j < TOGETHER; ++j) x[j] = load_pass(in, type, i);
-#pragma unroll
-            for (int j = 0; j < TOGETHER; ++j)
-                price[j] = bs_price<Ref32>(x[j].s, x[j].k, x[j].r, x[j].v, x[j].t, x[j].ty != 0);
-#pragma unroll
-            for (int j = 0; j < TOGETHER; ++j) {
-                *at(out, i) = price[j];
-                asm volatile("" ::: "memory");
-            }
-        }
-        if constexpr (TOGETHER > 1) {
-            for (; p < passes; ++p) {
-                const PassIn<TY> x = load_pass(in, type, i);
-                *at(out, i) = bs_price<Ref32>(x.s, x.k, x.r, x.v, x.t, x.ty != 0);
-            }
+        for (int p = 0; p < passes; ++p) {
+            asm volatile("" ::: "memory");
+            const float price = bs_price<Ref32>(*at(in.s, i), *at(in.k, i), *at(in.r, i),
+                                                *at(in.v, i), *at(in.t, i), *at(type, i) != 0);
+            __hip_atomic_store(at(out, i), price, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            asm volatile("" ::: "memory");
         }
     }
 }
@@ -301,16 +286,19 @@ hipError_t launch_passes_t(SoaIn<float> in, const TY* type, float* out, int64_t 
     const int64_t cap = config().max_blocks.load(std::memory_order_relaxed);
     const int bt = config().block_threads.load(std::memory_order_relaxed);
     const int nt = bt > 0 ? bt : 64;
-    const dim3 grid(grid_for(n, cap, nt));
-    if (n <= kTogetherMaxOptions)
-        hipLaunchKernelGGL((k_passes<TY, 4, uint32_t>), grid, dim3(nt), 0, st, in, type, out, n,
-                           passes);
+    const unsigned blocks = grid_for(n, cap, nt);
+    int64_t rows = std::min<int64_t>(kPassWaves * 64 / ((int64_t)blocks * nt),
+                                     passes / kPassesPerRow);
+    if (cap > 0) rows = std::min(rows, cap / blocks);
+    if (rows > 1)   // the blocks cover the book, of at most 2^19 options
+        hipLaunchKernelGGL((k_passes<TY, true, uint32_t>), dim3(blocks, (unsigned)rows), dim3(nt), 0,
+                           st, in, type, out, n, passes);
     else if (n < (int64_t(1) << 30))
-        hipLaunchKernelGGL((k_passes<TY, 1, uint32_t>), grid, dim3(nt), 0, st, in, type, out, n,
-                           passes);
+        hipLaunchKernelGGL((k_passes<TY, false, uint32_t>), dim3(blocks), dim3(nt), 0, st, in, type,
+                           out, n, passes);
     else
-        hipLaunchKernelGGL((k_passes<TY, 1, int64_t>), grid, dim3(nt), 0, st, in, type, out, n,
-                           passes);
+        hipLaunchKernelGGL((k_passes<TY, false, int64_t>), dim3(blocks), dim3(nt), 0, st, in, type,
+                           out, n, passes);
     return hipGetLastError();
 }
 

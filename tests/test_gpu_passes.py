@@ -123,8 +123,8 @@ def test_argument_errors(gpu):
                                       (300_001, 2)])
 @pytest.mark.parametrize("type_dtype", [np.uint8, np.int32])
 def test_one_launch_of_several_passes(gpu, n, passes, type_dtype):
-    """Passes in fours and what is left of them, on both sides of the size from
-    which one is in flight at a time: the bits of a single pass."""
+    """A few passes on odd sizes, in one row of the grid or several: the bits of
+    a single pass."""
     book = books.make_book(n, books.SEED_BASE + 114 + n % 83)
     db = gpu.DeviceBook(book, type_dtype=type_dtype)
     want = eager(gpu, db, n)
@@ -132,6 +132,32 @@ def test_one_launch_of_several_passes(gpu, n, passes, type_dtype):
     passes_call(gpu, db, out, n, passes)
     gpu.call("bs_stream_sync", None)
     assert np.array_equal(out.download(np.float32, n).view(np.uint32), want.view(np.uint32))
+    db.free()
+    out.free()
+
+
+@pytest.mark.parametrize("n,passes,cap", [(1, 1000, 0), (64, 8, 0), (64, 7, 0), (4097, 100, 0),
+                                          (65_535, 11, 0), ((1 << 19) - 1, 8, 0), (1 << 19, 9, 0),
+                                          ((1 << 19) + 1, 8, 0), (4097, 100, 7), (4097, 100, 130)])
+def test_passes_side_by_side(gpu, n, passes, cap):
+    """Rows of the grid that share the passes, up to the book size from which
+    there is one, with and without a cap on the grid: the bits of a single
+    pass in every option, and nothing past the last."""
+    book = books.make_book(n, books.SEED_BASE + 117 + n % 79)
+    db = gpu.DeviceBook(book)
+    want = eager(gpu, db, n)
+    out = gpu.alloc_out(n, pad=64)
+    old = gpu.get_config(gpu.CFG_MAX_BLOCKS)
+    try:
+        gpu.set_config(gpu.CFG_MAX_BLOCKS, cap)
+        gpu.call("bs_memset", out.ptr, 0xff, (n + 64) * 4, None)
+        passes_call(gpu, db, out, n, passes)
+        gpu.call("bs_stream_sync", None)
+    finally:
+        gpu.set_config(gpu.CFG_MAX_BLOCKS, old)
+    got = out.download(np.uint32, n + 64)
+    assert np.array_equal(got[:n], want.view(np.uint32))
+    assert np.all(got[n:] == 0xffffffff)
     db.free()
     out.free()
 
