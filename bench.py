@@ -662,7 +662,7 @@ def portfolio_section(L, dbooks, n, streams, ms) -> dict:
 
 def config4096_section(L, streams) -> dict:
     """The 4096-option book of the reference's CPU-runnable case, 100 passes:
-    L2-resident, so a per-pass latency, not an HBM figure; errors against the
+    L2-resident, so the cost of the calls, not an HBM figure; errors against the
     FP64 closed form and the reference."""
     import pyoracle
     small = books.make_book(4096, books.SEED_BASE + 1)
