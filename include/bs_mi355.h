@@ -221,7 +221,8 @@ typedef struct {
  * i's Monte-Carlo mean and standard error, FP64, from the same random
  * stream as the reference (ceil(trials / block_size) * block_size paths,
  * sums divided by trials).  Every path of every swaption runs on the GPU.
- * Host arrays; synchronous on `stream`.  Limits: trials in [1, 2^40],
+ * Host arrays; synchronous on `stream`, so refused (BS_ERR_HIP) while that is
+ * being captured.  Limits: trials in [1, 2^40],
  * block_size >= 1, seed in [0, 2^42) and seed + n + paths * (n_steps - 1) *
  * n_factors below 2^42, at most 2^24 blocks of 1024 paths in one call
  * (n * ceil(paths / 1024) <= 2^24, about 2^34 paths in all: one launch of at

@@ -47,6 +47,15 @@ int guarded(const char* what, F&& body) noexcept {
 int set_error(int status, const std::string& msg) noexcept;
 int hip_error(hipError_t e, const char* what);
 
+// Whether work on st would be recorded into a graph.
+inline bool capturing(hipStream_t st) {
+    if (!st) return false;   // the null stream cannot be captured
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 // Validates that [p, p + bytes) is memory the GPU may access.
 int check_device_range(const void* p, size_t bytes, const char* name);
 

@@ -409,14 +409,6 @@ int claim_slot(PfDevice& d) {
     return -1;
 }
 
-bool capturing(hipStream_t st) {
-    if (!st) return false;   // the null stream cannot be captured
-    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
-    (void)hipGetLastError();
-    return true;
-}
-
 }  // namespace
 
 // bs_portfolio_f32 with the device's fixed partials: no allocation.  The caller

@@ -1201,6 +1201,10 @@ extern "C" int bs_swaptions_host_f64(const bs_swaption_t* sw, int64_t n, int64_t
             if (paths > (kSwCounterLimit - (seed + i)) / draws)
                 return set_error(BS_ERR_INVALID, "seed + paths x draws exceeds 2^42");
         }
+        // A synchronous call waits for its results, which recorded kernels never
+        // write: a workspace taken for them would be lost.
+        if (capturing(static_cast<hipStream_t>(stream)))
+            return hip_error(hipErrorStreamCaptureUnsupported, "bs_swaptions_host_f64");
         // one launch of at most 2^32 work-items: 2^24 blocks of 1024 paths
         const int64_t bps_most = (paths + kSwThreads * kSwRows - 1) / (kSwThreads * kSwRows);
         if (bps_most * n > (int64_t(1) << 24))

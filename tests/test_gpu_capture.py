@@ -75,3 +75,43 @@ def test_captured_in_a_callers_graph(gpu, check_pointers):
         for o in [out] + gouts:
             o.free()
         db.free()
+
+
+def test_swaptions_on_a_capturing_stream_are_refused(gpu):
+    """bs_swaptions_host_f64 is synchronous: on a capturing stream it is refused
+    (BS_ERR_HIP) and leaves the capture as it was, six times over (a call has one
+    of four workspaces), and the call works again after the capture ends."""
+    from p3arsec_amd import swaptions
+    H = hip()
+    sws, base = swaptions.parsec_portfolio(4)
+    want = swaptions.price(sws, 2000, base)
+    n = 4097
+    db = gpu.DeviceBook(books.make_book(n, books.SEED_BASE + 141))
+    eager = gpu.price(db).download(np.float32, n)
+    out = gpu.alloc_out(n)
+    st = gpu.Stream()
+    graph, gexec = ctypes.c_void_p(), ctypes.c_void_p()
+    try:
+        assert H.hipStreamBeginCapture(st.handle, CAPTURE_THREAD_LOCAL) == 0
+        gpu.call("bs_price_f32", *db.ptrs(), out.ptr, n, st.handle)
+        for _ in range(6):
+            with pytest.raises(gpu.BSError) as e:
+                swaptions.price(sws, 2000, base, stream=st.handle)
+            assert e.value.status == -2
+        assert H.hipStreamEndCapture(st.handle, ctypes.byref(graph)) == 0
+        assert H.hipGraphInstantiate(ctypes.byref(gexec), graph, None, None, 0) == 0
+        assert H.hipGraphLaunch(gexec, st.handle) == 0
+        gpu.call("bs_stream_sync", st.handle)
+        assert np.array_equal(out.download(np.float32, n).view(np.uint32), eager.view(np.uint32))
+        for stream in (None, st.handle):
+            got = swaptions.price(sws, 2000, base, stream=stream)
+            for g, w in zip(got, want):
+                assert np.array_equal(g.view(np.uint64), w.view(np.uint64))
+    finally:
+        if gexec.value:
+            H.hipGraphExecDestroy(gexec)
+        if graph.value:
+            H.hipGraphDestroy(graph)
+        st.destroy()
+        out.free()
+        db.free()
