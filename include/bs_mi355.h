@@ -220,7 +220,9 @@ typedef struct {
  * (HJM_Swaption_Blocking.cpp:20-222): price[i] and std_error[i] are swaption
  * i's Monte-Carlo mean and standard error, FP64, from the same random
  * stream as the reference (ceil(trials / block_size) * block_size paths,
- * sums divided by trials).  Every path of every swaption runs on the GPU.
+ * sums divided by trials).  Every path of every swaption runs on the GPU.  A
+ * swaption's results are the same bits alone, in a shard (with its own seed + i)
+ * and in the whole portfolio.
  * Host arrays; synchronous on `stream`, so refused (BS_ERR_HIP) while that is
  * being captured.  Limits: trials in [1, 2^40],
  * block_size >= 1, seed in [0, 2^42) and seed + n + paths * (n_steps - 1) *

@@ -37,6 +37,7 @@
 #include "bs_internal.hpp"
 #include "bs_math.hpp"
 #include "bs_ops.hpp"
+#include "bs_wave.hpp"
 
 namespace bs {
 namespace {
@@ -113,30 +114,6 @@ __device__ __forceinline__ void pf_add(double* acc, const PfOptions& x) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
         add_option<kGreeks>(acc, x.s[j], x.k[j], x.r[j], x.v[j], x.t[j], put_of(x.ty, j), x.w[j]);
-}
-
-// x moved across lanes by a DPP control; lanes it does not reach, and rows
-// outside `rows`, give 0.
-template <int kControl, int kRows>
-__device__ __forceinline__ double dpp(double x) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), kControl, kRows, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), kControl, kRows, 0xf, true);
-    return __hiloint2double(hi, lo);
-}
-
-// The wave's sum, in every lane: within rows of 16 lanes (shifts right by 1, 2,
-// 4, 8), then row totals into the next rows (broadcasts of lanes 15 and 31).
-// Three VALU instructions a step; through LDS (__shfl_xor) the five folds of a
-// wave cost as much as two of its options.
-__device__ __forceinline__ double wave_sum(double x) {
-    x += dpp<0x111, 0xf>(x);
-    x += dpp<0x112, 0xf>(x);
-    x += dpp<0x114, 0xf>(x);
-    x += dpp<0x118, 0xf>(x);
-    x += dpp<0x142, 0xa>(x);
-    x += dpp<0x143, 0xc>(x);
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
-                            __builtin_amdgcn_readlane(__double2loint(x), 63));
 }
 
 // One wave's sums of NQ quantities: of group g's partials, and of the groups'.

@@ -38,10 +38,11 @@
 // residue of the next counter is one 32-bit addition away.
 //
 // Kernels (the caller's stream): k_sw_paths, 2 to 32 paths per work-item, and,
-// where it left blocks out, k_sw_paths_steps, each block's sums of payoff and
-// payoff^2 folded in a fixed order into one partial; a swaption's partials are
-// added in a fixed order and its mean and standard error formed as the
-// reference does, by its last block in a small launch and by k_sw_final else.  Results are bit-reproducible for given inputs.
+// where it left paths out, k_sw_paths_steps, each unit's sums of payoff and
+// payoff^2 (512 to 2048 paths) folded in a fixed order into one partial; a
+// swaption's partials are added in a fixed order and its mean and standard error
+// formed as the reference does, by its last block in a small launch and by
+// k_sw_final else.  A swaption's results are the same bits in every call.
 // The arithmetic is FP64 (the reference's FTYPE); this file is compiled
 // without FMA contraction, so the step-by-step kernel rounds every product and
 // sum as the reference does and the other one's FMAs are the ones written.
@@ -58,6 +59,7 @@
 #include "bs_arrive.hpp"
 #include "bs_fp64.hpp"
 #include "bs_internal.hpp"
+#include "bs_wave.hpp"
 
 namespace bs {
 namespace {
@@ -77,6 +79,26 @@ struct SwGrid {
     int64_t paths;
     int32_t bps, rows;
 };
+
+// A swaption's paths are summed in units of kSwThreads unit_rows paths, each
+// into a partial of its own.  The unit, and with it the order of the sums, comes
+// from the swaption and its number of paths alone, so a swaption's results are
+// the same bits in every call, whatever else the call prices and however its
+// blocks are cut (`rows` is a multiple of every unit).
+//
+// A unit costs a wave 18 VALU instructions beside the 200 or more of each row of
+// paths, and no work-item has fewer rows than a unit of its call, which leaves
+// small calls with too few blocks.  Units of 2, 4 and 8 rows, us a call: 128 of the
+// driver's swaptions (3 or 6 draws) x 1M trials 940, 867, 843, 1 x 1M 41, 29.7,
+// 25.6; 128 x 524,288 500, 457, 448; 8 x 262,144 38.3, 35.4, 33.2, 1 x 262,144 23.2,
+// 20.3, 20.8; 64 x 20,000 41.4, 40.3, 41.0, 16 x 10,000 22.5, 24.0, 27.8.  With more
+// draws (24 steps, 4 factors, starts at steps 1-12) 8 x 50,000 43.2, 58.2, 89.0,
+// and 1 x 1M (start at step 8) 87.7, 87.4, 105, 16 x 1M 900, 897, 901.
+constexpr int kSwMaxUnits = 16;   // of a block
+constexpr int kSwMaxUnitRows = 8;
+constexpr int unit_rows(bool narrow, int64_t paths) {
+    return !narrow || paths < (1 << 18) ? 2 : paths < (1 << 19) ? 4 : kSwMaxUnitRows;
+}
 
 // One swaption as the step-by-step kernel reads it.  pool + off holds f0[n] (the forward
 // curve at t = 0), mudt[n-1] (total drift x dt), sigma[F][n-1] and pay[L]
@@ -192,8 +214,11 @@ struct SwLin {
     int32_t flows;       // cash flows
     int32_t off;
     int32_t linear;      // 0: every block is left to k_sw_paths_steps
+    int32_t unit, units; // rows of a unit, and how many units hold the paths
+    int32_t unit0;       // the first one's place among the launch's partials
+    int32_t pad;
 };
-static_assert(sizeof(SwLin) == 48, "SwLin layout");
+static_assert(sizeof(SwLin) == 64, "SwLin layout");
 
 constexpr uint32_t kGenA = (uint32_t)(uint64_t(16807) * 1513517u % kM31);
 constexpr uint32_t gen_step(uint64_t counters) {
@@ -274,12 +299,50 @@ __device__ __forceinline__ double moro_tail_fma(uint32_t residue) {
     return upper ? v : -v;
 }
 
-// Whether the linear form takes the paths of block `chunk` of a swaption: it is
-// bounded and no counter of the block draws u = 0.
-__device__ __forceinline__ bool block_linear(const SwLin& h, const SwGrid& grid, int64_t chunk) {
-    const uint64_t span = (uint64_t)(kSwThreads * grid.rows) * h.per_path;
-    const uint64_t r = mod_m31((uint64_t)h.seed + (uint64_t)chunk * span);
+// Whether the linear form takes the kSwThreads rows paths from `first` on: the
+// swaption is bounded and none of their counters draws u = 0.
+__device__ __forceinline__ bool rows_linear(const SwLin& h, int64_t first, int rows) {
+    const uint64_t span = (uint64_t)(kSwThreads * rows) * h.per_path;
+    const uint64_t r = mod_m31((uint64_t)h.seed + (uint64_t)first * h.per_path);
     return h.linear && r != 0 && r + span <= kM31;
+}
+
+// A wave's sums of a unit, left in LDS: the two quantities are halved into one
+// register (the lower lanes' of sumsq against the upper lanes' of sum), then
+// both fold at once within 32 lanes, 18 instructions in all.
+using UnitSums = double[kSwThreads / 64][kSwMaxUnits][2];
+__device__ __forceinline__ void wave_sums(double sum, double sumsq, double* to) {
+    double x = swap_halves_add(sum, sumsq);
+    x = half_wave_sum(x);
+    const int lane = threadIdx.x & 63;
+    if ((lane & 31) == 31) to[lane >> 5] = x;
+}
+
+// A work-item's paths, a unit at a time: paths(at, &sum, &sumsq) adds the PP
+// paths at, at + kSwThreads, ... and advances xb past them.  Units that hold a
+// zero draw are left to k_sw_paths_steps (whole: none does).  Bit u of the
+// result: unit u was summed into sums[u].
+template <int PP, class Paths>
+__device__ __forceinline__ uint32_t over_units(const SwLin& h, const SwGrid& grid, int64_t first,
+                                               bool whole, uint32_t& xb,
+                                               double (*__restrict__ sums)[2], Paths&& paths) {
+    uint32_t done = 0;
+    int u = 0;
+#pragma unroll 1
+    for (int64_t at = first; at < first + kSwThreads * grid.rows && at < grid.paths;
+         ++u, at += kSwThreads * h.unit) {
+        if (!whole && !rows_linear(h, at, h.unit)) {
+            for (int row = 0; row < h.unit; ++row) xb = add_m31(xb, h.x_row);
+            continue;
+        }
+        double sum = 0.0, sumsq = 0.0;
+#pragma unroll 1
+        for (int row = 0; row < h.unit; row += PP)
+            paths(at + row * kSwThreads + (int)threadIdx.x, &sum, &sumsq);
+        wave_sums(sum, sumsq, sums[u]);
+        done |= 1u << u;
+    }
+    return done;
 }
 
 // Keeps the compiler from moving the lanes' accesses to their wave's LDS list
@@ -361,17 +424,17 @@ __device__ __forceinline__ void linear_batch(const SwLin& h, const double* __res
 
 // The paths of a work-item, PP at a time.
 template <int W, int PP, int DB>
-__device__ __forceinline__ void linear_paths(const SwLin& h, const double* __restrict__ q,
-                                             uint32_t xb, int64_t p0, const SwGrid& grid,
-                                             char* lds, uint32_t wl,
-                                             double* sum, double* sumsq) {
+__device__ __forceinline__ uint32_t linear_paths(const SwLin& h, const double* __restrict__ q,
+                                                 uint32_t xb, int64_t first, bool whole,
+                                                 const SwGrid& grid, char* lds, uint32_t wl,
+                                                 double (*__restrict__ sums)[2]) {
     const double* __restrict__ pay = q + W;
     const double* __restrict__ G = q + 2 * W;
     const double* __restrict__ gdf = G + h.draws * W;
     const double df0 = exp2_mid(h.c_df);
     const MoroCentral central;
-#pragma unroll 1
-    for (int row = 0; row < grid.rows; row += PP) {
+    return over_units<PP>(h, grid, first, whole, xb, sums,
+                          [&](int64_t p0, double* sum, double* sumsq) {
         double acc[PP][W], dfe[PP];
         uint32_t xs[PP];
 #pragma unroll
@@ -404,11 +467,11 @@ __device__ __forceinline__ void linear_paths(const SwLin& h, const double* __res
 #pragma unroll
         for (int p = 0; p < PP; ++p) {
             double v = (leg[p] > 0 ? leg[p] : 0) * df[p];
-            v = p0 + (row + p) * kSwThreads < grid.paths ? v : 0.0;
+            v = p0 + p * kSwThreads < grid.paths ? v : 0.0;
             *sum += v;
             *sumsq = __builtin_fma(v, v, *sumsq);
         }
-    }
+    });
 }
 
 // The paths of a work-item one at a time, for many draws or cash flows: only
@@ -419,9 +482,10 @@ constexpr int kWideDraws = 12;   // draws in a batch
 constexpr uint32_t kWideBytes = kWideDraws * 64 * (8 + 2);   // a wave's slots and list
 
 template <int W>
-__device__ __forceinline__ void linear_wide(const SwLin& h, const double* __restrict__ q,
-                                            uint32_t xb, int64_t p0, const SwGrid& grid,
-                                            char* lds, double* sum, double* sumsq) {
+__device__ __forceinline__ uint32_t linear_wide(const SwLin& h, const double* __restrict__ q,
+                                                uint32_t xb, int64_t first, bool whole,
+                                                const SwGrid& grid, char* lds,
+                                                double (*__restrict__ sums)[2]) {
     const double* __restrict__ pay = q + W;
     const double* __restrict__ G = q + 2 * W;
     const double* __restrict__ gdf = G + h.draws * W;
@@ -432,8 +496,8 @@ __device__ __forceinline__ void linear_wide(const SwLin& h, const double* __rest
     char* slots = lds + wave * kWideBytes;
     uint16_t* list = reinterpret_cast<uint16_t*>(slots + kWideDraws * 64 * 8);
     char* mine = slots + lane * 8;
-#pragma unroll 1
-    for (int row = 0; row < grid.rows; ++row) {
+    return over_units<1>(h, grid, first, whole, xb, sums,
+                         [&](int64_t p0, double* sum, double* sumsq) {
         double acc[W], dfe = h.c_df;
 #pragma unroll
         for (int c = 0; c < W; ++c) acc[c] = q[c];
@@ -481,10 +545,10 @@ __device__ __forceinline__ void linear_wide(const SwLin& h, const double* __rest
         for (int c = 0; c < W; ++c)
             if (c < h.flows) leg = __builtin_fma(pay[c], exp2_mid(acc[c]), leg);
         double v = (leg > 0 ? leg : 0) * (h.df_draws > 0 ? exp2_mid(dfe) : df0);
-        v = p0 + row * kSwThreads < grid.paths ? v : 0.0;
+        v = p0 < grid.paths ? v : 0.0;
         *sum += v;
         *sumsq = __builtin_fma(v, v, *sumsq);
-    }
+    });
 }
 
 // A block's sums of payoff and payoff^2, in a fixed order (thread 0's to use).
@@ -495,6 +559,7 @@ __device__ __forceinline__ void block_sums(double* sum, double* sumsq) {
         *sumsq += __shfl_xor(*sumsq, o, 64);
     }
     __shared__ double lds[2][kSwThreads / 64];
+    __syncthreads();   // the last call's reads
     if ((threadIdx.x & 63) == 0) {
         lds[0][threadIdx.x / 64] = *sum;
         lds[1][threadIdx.x / 64] = *sumsq;
@@ -512,13 +577,13 @@ __device__ __forceinline__ void block_sums(double* sum, double* sumsq) {
 }
 
 // A swaption's mean and standard error (HJM_Swaption_Blocking.cpp:212-218) from
-// its bps partials: work-item t takes t, t + 256, ... in order, then a fixed
+// its units' partials: work-item t takes t, t + 256, ... in order, then a fixed
 // tree; thread 0 hands both to put().  lds: 2 kSwThreads doubles.
 template <class Load, class Put>
-__device__ __forceinline__ void mean_and_error(int bps, int64_t trials, double* lds, Load&& load,
+__device__ __forceinline__ void mean_and_error(int units, int64_t trials, double* lds, Load&& load,
                                                Put&& put) {
     double a = 0.0, b = 0.0;
-    for (int i = threadIdx.x; i < bps; i += kSwThreads) {
+    for (int i = threadIdx.x; i < units; i += kSwThreads) {
         a += load(2 * i);
         b += load(2 * i + 1);
     }
@@ -553,25 +618,33 @@ struct SwDone {
     int64_t trials;
 };
 
-// Ends a block of swaption sw.  lds: as mean_and_error's, free to overwrite.
-__device__ __forceinline__ void finish_block(double sum, double sumsq, int sw, int bps,
-                                             double* partial, const SwDone& done, double* lds) {
-    block_sums(&sum, &sumsq);
+// Ends a block of swaption sw whose unit u (bit u of summed) has its waves' sums
+// in sums[wave][u]; mine: the partials from its first unit on, all: from the
+// swaption's.  lds: as mean_and_error's, free to overwrite once the block has met.
+__device__ __forceinline__ void finish_block(const UnitSums& sums, uint32_t summed, int sw,
+                                             const SwLin& h, const SwGrid& grid, double* all,
+                                             double* mine, const SwDone& done, double* lds) {
+    static_assert(2 * kSwMaxUnits <= 64, "one wave stores a block's partials");
     __shared__ int last;
-    if (threadIdx.x == 0) {
-        double* mine = partial + 2 * (int64_t)blockIdx.x;
-        agent_store(mine, sum);
-        agent_store(mine + 1, sumsq);
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const int u = threadIdx.x / 2, q = threadIdx.x & 1;
+        if (u < kSwMaxUnits && (summed >> u & 1)) {
+            double v = sums[0][u][q];
+#pragma unroll
+            for (int w = 1; w < kSwThreads / 64; ++w) v += sums[w][u][q];
+            agent_store(mine + 2 * u + q, v);
+        }
         if (done.counters) {
             stores_done();
-            last = arrive_one(done.counters + 64 * sw, (uint32_t)bps);
+            const bool full = arrive(done.counters + 64 * sw, (uint32_t)grid.bps);
+            if (threadIdx.x == 0) last = full;
         }
     }
     if (!done.counters) return;
     __syncthreads();
     if (!last) return;
-    const double* in = partial + 2 * (int64_t)sw * bps;
-    mean_and_error(bps, done.trials, lds, [&](int i) { return agent_load(in + i); },
+    mean_and_error(h.units, done.trials, lds, [&](int i) { return agent_load(all + i); },
                    [&](double mean, double error) {
                        system_store(done.out + 2 * sw, mean);
                        system_store(done.out + 2 * sw + 1, error);
@@ -582,7 +655,8 @@ __device__ __forceinline__ void finish_block(double sum, double sumsq, int sw, i
                    });
 }
 
-constexpr int kSwBatch = 12;   // draws of a work-item in one batch of the narrow form
+constexpr int kSwBatch = 12;     // draws of a work-item in one batch of the narrow form
+constexpr int kNarrowFlows = 4;   // cash flows it takes
 
 // Widths of the linear form's accumulators: the smallest that holds the cash
 // flows.  A launch's kernel holds the forms up to the widest of its swaptions
@@ -597,17 +671,19 @@ constexpr int lin_width(int flows) {
 // Few draws and cash flows (the reference driver's swaptions have 3 or 6 and 1
 // to 3): several paths at a time in registers.  Otherwise the wide form.
 template <int W>
-__device__ __forceinline__ void linear_form(const SwLin& h, const double* __restrict__ q,
-                                            uint32_t xb, int64_t p0, const SwGrid& grid,
-                                            char* lds, double* sum, double* sumsq) {
-    if constexpr (W <= 4) {
+__device__ __forceinline__ uint32_t linear_form(const SwLin& h, const double* __restrict__ q,
+                                                uint32_t xb, int64_t first, bool whole,
+                                                const SwGrid& grid, char* lds,
+                                                double (*__restrict__ sums)[2]) {
+    if constexpr (W <= kNarrowFlows) {
         const uint32_t wl = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / 64) *
                             (kSwBatch * 64 * 8);
-        if (h.draws <= 3 && grid.rows >= 4)
-            return linear_paths<W, 4, 3>(h, q, xb, p0, grid, lds, wl, sum, sumsq);
-        if (h.draws <= 6) return linear_paths<W, 2, 6>(h, q, xb, p0, grid, lds, wl, sum, sumsq);
+        if (h.draws <= 3 && h.unit >= 4)
+            return linear_paths<W, 4, 3>(h, q, xb, first, whole, grid, lds, wl, sums);
+        if (h.draws <= kSwBatch / 2)
+            return linear_paths<W, 2, kSwBatch / 2>(h, q, xb, first, whole, grid, lds, wl, sums);
     }
-    linear_wide<W>(h, q, xb, p0, grid, lds, sum, sumsq);
+    return linear_wide<W>(h, q, xb, first, whole, grid, lds, sums);
 }
 
 // Bound by FP64 issue (parameters and partial sums are all it reads and
@@ -623,48 +699,52 @@ __attribute__((amdgpu_waves_per_eu(MAXW <= 8 ? 4 : MAXW <= 32 ? 3 : 2))) void k_
     const SwLin* __restrict__ heads, const double* __restrict__ pool, SwGrid grid,
     double* partial, SwDone done) {
     __shared__ __align__(8) char lds[kSwThreads / 64 * kWideBytes];
+    __shared__ UnitSums unit_sums;
     static_assert(kSwThreads * kSwBatch * 8 <= sizeof lds, "the narrow form's lists");
     const int sw = (int)(blockIdx.x / (unsigned)grid.bps);
     const int64_t chunk = blockIdx.x % (unsigned)grid.bps;
     const SwLin h = heads[sw];
-    if (!block_linear(h, grid, chunk)) return;
+    if (!h.linear) return;
     const double* q = pool + h.off;
     const int64_t first = chunk * (kSwThreads * grid.rows);
+    const bool whole = rows_linear(h, first, grid.rows);
     // residue of this work-item's first draw: the block's (uniform) and the
     // work-item's path, A (seed + (first + t) per_path)
     const uint64_t xu = mod_m31(mod_m31((uint64_t)h.seed + (uint64_t)first * h.per_path) * kGenA);
     const uint32_t xb = add_m31((uint32_t)xu, (uint32_t)mod_m31((uint64_t)h.x_path * threadIdx.x));
-    const int64_t p0 = first + threadIdx.x;
-    double sum = 0.0, sumsq = 0.0;
+    double (*sums)[2] = unit_sums[__builtin_amdgcn_readfirstlane(threadIdx.x / 64)];
+    uint32_t summed = 0;
     const int W = h.flows;
-    if (W <= 1) linear_form<1>(h, q, xb, p0, grid, lds, &sum, &sumsq);
-    if (W == 2) linear_form<2>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+    if (W <= 1) summed = linear_form<1>(h, q, xb, first, whole, grid, lds, sums);
+    if (W == 2) summed = linear_form<2>(h, q, xb, first, whole, grid, lds, sums);
     if constexpr (MAXW >= 4) {
-        if (W == 3) linear_form<3>(h, q, xb, p0, grid, lds, &sum, &sumsq);
-        if (W == 4) linear_form<4>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W == 3) summed = linear_form<3>(h, q, xb, first, whole, grid, lds, sums);
+        if (W == 4) summed = linear_form<4>(h, q, xb, first, whole, grid, lds, sums);
     }
     if constexpr (MAXW >= 8) {
-        if (W > 4 && W <= 6) linear_form<6>(h, q, xb, p0, grid, lds, &sum, &sumsq);
-        if (W > 6 && W <= 8) linear_form<8>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W > 4 && W <= 6) summed = linear_form<6>(h, q, xb, first, whole, grid, lds, sums);
+        if (W > 6 && W <= 8) summed = linear_form<8>(h, q, xb, first, whole, grid, lds, sums);
     }
     if constexpr (MAXW >= 16) {
-        if (W > 8 && W <= 12) linear_form<12>(h, q, xb, p0, grid, lds, &sum, &sumsq);
-        if (W > 12 && W <= 16) linear_form<16>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W > 8 && W <= 12) summed = linear_form<12>(h, q, xb, first, whole, grid, lds, sums);
+        if (W > 12 && W <= 16) summed = linear_form<16>(h, q, xb, first, whole, grid, lds, sums);
     }
     if constexpr (MAXW >= 32) {
-        if (W > 16 && W <= 24) linear_form<24>(h, q, xb, p0, grid, lds, &sum, &sumsq);
-        if (W > 24 && W <= 32) linear_form<32>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W > 16 && W <= 24) summed = linear_form<24>(h, q, xb, first, whole, grid, lds, sums);
+        if (W > 24 && W <= 32) summed = linear_form<32>(h, q, xb, first, whole, grid, lds, sums);
     }
     if constexpr (MAXW >= 64) {
-        if (W > 32 && W <= 48) linear_form<48>(h, q, xb, p0, grid, lds, &sum, &sumsq);
-        if (W > 48) linear_form<64>(h, q, xb, p0, grid, lds, &sum, &sumsq);
+        if (W > 32 && W <= 48) summed = linear_form<48>(h, q, xb, first, whole, grid, lds, sums);
+        if (W > 48) summed = linear_form<64>(h, q, xb, first, whole, grid, lds, sums);
     }
     static_assert(2 * kSwThreads * sizeof(double) <= sizeof lds, "finish_block's sums");
     // finish_block synchronises the block before it overwrites the lists
-    finish_block(sum, sumsq, sw, grid.bps, partial, done, reinterpret_cast<double*>(lds));
+    double* all = partial + 2 * (int64_t)h.unit0;
+    finish_block(unit_sums, summed, sw, h, grid, all, all + 2 * (first / (kSwThreads * h.unit)),
+                 done, reinterpret_cast<double*>(lds));
 }
 
-// The blocks that k_sw_paths left out, one path at a time per work-item (the
+// The units that k_sw_paths left out, one path at a time per work-item (the
 // draws live in scratch).
 template <int F, int MAXM>
 __global__ __launch_bounds__(kSwThreads) void k_sw_paths_steps(
@@ -672,25 +752,33 @@ __global__ __launch_bounds__(kSwThreads) void k_sw_paths_steps(
     const double* __restrict__ pool, SwGrid grid, double* __restrict__ partial) {
     const int sw = (int)(blockIdx.x / (unsigned)grid.bps);
     const int64_t chunk = blockIdx.x % (unsigned)grid.bps;
-    if (block_linear(lin[sw], grid, chunk)) return;
+    const SwLin x = lin[sw];
+    const int64_t first = chunk * (kSwThreads * grid.rows);
+    if (rows_linear(x, first, grid.rows)) return;
     const SwHead h = heads[sw];
     const double* q = pool + h.off;
-    double sum = 0.0, sumsq = 0.0;
 #pragma unroll 1
-    for (int j = 0; j < grid.rows; ++j) {
-        const int64_t p = (chunk * grid.rows + j) * kSwThreads + threadIdx.x;
-        if (p < grid.paths) {
-            double z[MAXM][F];
-            draws<F, MAXM>(h, p, z);
-            const double v = path_payoff<F, MAXM>(h, q, z);
-            sum += v;
-            sumsq += v * v;
+    for (int64_t at = first; at < first + kSwThreads * grid.rows && at < grid.paths;
+         at += kSwThreads * x.unit) {
+        if (rows_linear(x, at, x.unit)) continue;
+        double sum = 0.0, sumsq = 0.0;
+#pragma unroll 1
+        for (int j = 0; j < x.unit; ++j) {
+            const int64_t p = at + j * kSwThreads + threadIdx.x;
+            if (p < grid.paths) {
+                double z[MAXM][F];
+                draws<F, MAXM>(h, p, z);
+                const double v = path_payoff<F, MAXM>(h, q, z);
+                sum += v;
+                sumsq += v * v;
+            }
         }
-    }
-    block_sums(&sum, &sumsq);
-    if (threadIdx.x == 0) {
-        partial[2 * (int64_t)blockIdx.x] = sum;
-        partial[2 * (int64_t)blockIdx.x + 1] = sumsq;
+        block_sums(&sum, &sumsq);
+        if (threadIdx.x == 0) {
+            double* mine = partial + 2 * (x.unit0 + at / (kSwThreads * x.unit));
+            mine[0] = sum;
+            mine[1] = sumsq;
+        }
     }
 }
 
@@ -704,13 +792,14 @@ __global__ __launch_bounds__(kSwThreads) void k_sw_stage(const uint4* __restrict
     for (int i = first; i < ncounters; i += stride) counters[64 * i] = 0;
 }
 
-// Block i forms swaption i's results from its bps partials.
-__global__ __launch_bounds__(kSwThreads) void k_sw_final(const double* __restrict__ partial,
-                                                         int bps, int64_t trials,
+// Block i forms swaption i's results from its units' partials.
+__global__ __launch_bounds__(kSwThreads) void k_sw_final(const SwLin* __restrict__ heads,
+                                                         const double* __restrict__ partial,
+                                                         int64_t trials,
                                                          double* __restrict__ out) {
     __shared__ double lds[2 * kSwThreads];
-    const double* in = partial + 2 * (int64_t)blockIdx.x * bps;
-    mean_and_error(bps, trials, lds, [&](int i) { return in[i]; },
+    const double* in = partial + 2 * (int64_t)heads[blockIdx.x].unit0;
+    mean_and_error(heads[blockIdx.x].units, trials, lds, [&](int i) { return in[i]; },
                    [&](double mean, double error) {
                        out[2 * blockIdx.x] = mean;
                        out[2 * blockIdx.x + 1] = error;
@@ -761,10 +850,11 @@ int round_index(double x) {
 struct SwShape {
     double dt;
     int m, L, freq, points;
+    int unit;
 };
 
-// Validates swaption i.
-int shape_of(const bs_swaption_t& s, int64_t i, SwShape* x) {
+// Validates swaption i of `paths` paths.
+int shape_of(const bs_swaption_t& s, int64_t i, int64_t paths, SwShape* x) {
     const int n = s.n_steps, F = s.n_factors;
     char msg[160];
     auto bad = [&](const char* why) {
@@ -784,7 +874,8 @@ int shape_of(const bs_swaption_t& s, int64_t i, SwShape* x) {
     if (m < 0 || m >= n) return bad("maturity outside the simulated horizon");
     if (L < 1 || points < 0 || points > L - 1) return bad("swap tenor outside the horizon");
     if (m * F > kSwMaxDraws) return bad("start step x n_factors exceeds 64");
-    *x = {dt, m, L, freq, points};
+    const bool narrow = m * F <= kSwBatch / 2 && points / freq <= kNarrowFlows;
+    *x = {dt, m, L, freq, points, unit_rows(narrow, paths)};
     return BS_OK;
 }
 
@@ -937,7 +1028,7 @@ bool draws_zero(int64_t c, int64_t count) {
 // and took 91.
 constexpr int kSwDevices = 64;
 constexpr int kSwSpaces = 4;
-constexpr size_t kSpaceHost = size_t(1) << 20, kSpaceDev = size_t(4) << 20;
+constexpr size_t kSpaceHost = size_t(1) << 20, kSpaceDev = size_t(16) << 20;
 constexpr size_t kSpaceFlag = 64;   // the end of the pinned memory
 
 // Launches that end by themselves (SwDone) save k_sw_final and the stream's
@@ -1053,18 +1144,23 @@ struct SwBatch {
     std::vector<double> pool;
     std::vector<int32_t> index;   // places in the caller's array
     int flows = 0;
-    bool steps = false;           // some block needs the step-by-step kernel
+    int32_t units = 0;
+    bool steps = false;           // some unit needs the step-by-step kernel
 
-    // paths: those the swaption's blocks cover.
     void add(const bs_swaption_t& s, const SwShape& x, int64_t seed, int32_t i, int64_t paths) {
         heads.emplace_back();
         lins.emplace_back();
         index.push_back(i);
         pack_swaption(s, x, seed, &heads.back(), &pool);
         pack_linear(heads.back(), s.n_factors, x.freq, x.points, &lins.back(), &pool);
-        flows = std::max(flows, lins.back().flows);
-        steps = steps || !lins.back().linear ||
-                draws_zero(seed, paths * lins.back().per_path);
+        SwLin& l = lins.back();
+        flows = std::max(flows, l.flows);
+        l.unit = x.unit;
+        l.units = (int32_t)((paths + kSwThreads * x.unit - 1) / (kSwThreads * x.unit));
+        l.unit0 = units;
+        units += l.units;
+        steps = steps || !l.linear ||
+                draws_zero(seed, (int64_t)l.units * kSwThreads * x.unit * l.per_path);
     }
 };
 
@@ -1072,12 +1168,12 @@ struct SwBatch {
 struct SwLayout {
     size_t heads, pool, partial, bytes;   // offsets of the step-by-step heads, pool and
                                           // partials, and what all of it takes
-    SwLayout(const SwBatch& b, size_t blocks) {
+    explicit SwLayout(const SwBatch& b) {
         auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
         heads = up(b.lins.size() * sizeof(SwLin));
         pool = heads + up(b.heads.size() * sizeof(SwHead));
         partial = pool + up(b.pool.size() * sizeof(double));
-        bytes = partial + blocks * 2 * sizeof(double);
+        bytes = partial + (size_t)b.units * 2 * sizeof(double);
     }
     // Writes the parameters (everything before the partials), laid out as on the device.
     void write(const SwBatch& b, char* to) const {
@@ -1101,14 +1197,14 @@ hipError_t launch_batch(const SwBatch& b, const SwLayout& at, int F, const SwGri
     linear_kernel(b.flows)(blocks, st, dl, dp, grid, dq, done);
     if (b.steps) kStepsByFactors[F - 1](blocks, st, dl, dh, dp, grid, dq);
     if (!done.counters)
-        hipLaunchKernelGGL(k_sw_final, dim3(n), dim3(kSwThreads), 0, st, dq, grid.bps, trials, out);
+        hipLaunchKernelGGL(k_sw_final, dim3(n), dim3(kSwThreads), 0, st, dl, dq, trials, out);
     return hipGetLastError();
 }
 
 int price_batch(const SwBatch& b, int F, const SwGrid& grid, int64_t trials, double* price,
                 double* std_error, hipStream_t st) {
     const size_t n = b.lins.size();
-    const SwLayout at(b, (size_t)grid.bps * n);
+    const SwLayout at(b);
     const size_t ob = n * 2 * sizeof(double);
     auto deliver = [&](const double* out) {
         for (size_t k = 0; k < n; ++k) {
@@ -1195,7 +1291,7 @@ extern "C" int bs_swaptions_host_f64(const bs_swaption_t* sw, int64_t n, int64_t
         for (int64_t i = 0; i < n; ++i) {
             if (sw[i].n_factors != F)
                 return set_error(BS_ERR_INVALID, "every swaption must have the same n_factors");
-            const int rc = shape_of(sw[i], i, &shapes[(size_t)i]);
+            const int rc = shape_of(sw[i], i, paths, &shapes[(size_t)i]);
             if (rc) return rc;
             const int64_t draws = (int64_t)(sw[i].n_steps - 1) * F;
             if (paths > (kSwCounterLimit - (seed + i)) / draws)
@@ -1213,7 +1309,7 @@ extern "C" int bs_swaptions_host_f64(const bs_swaption_t* sw, int64_t n, int64_t
         // Paths per work-item: enough of them to spread the 100 or so
         // instructions of its set-up while several rounds of blocks are left
         // (1024 are resident at once), and 2 where 4 would leave the chip
-        // idle.  Rows 2, 4, 8, 16 and 32: 8 swaptions x 50,000 trials (starts at
+        // idle.  Rows 2, 4 and 8: 8 swaptions x 50,000 trials (starts at
         // steps 1-12, 4 factors; 392 blocks of 4 rows) 52, 70 and 107 us; 64 x
         // 20,000 (1280 blocks) 51, 50, 51; 32 x 50,000 (starts at steps 1-10,
         // 1568 blocks) 126, 126, 140.  Rows 16, 32 and 64: 128 x 1M (125,056
@@ -1221,7 +1317,8 @@ extern "C" int bs_swaptions_host_f64(const bs_swaption_t* sw, int64_t n, int64_t
         // and a start at step 8; 128 x 550,000 (68,864) 447, 441; rows 8, 32 and
         // 64 at 128 x 500,000 (62,592) 430, 430, 431.
         const int64_t blocks4 = bps_most * n;
-        const int rows = blocks4 >= 65536 ? 32 : blocks4 >= 16384 ? 8 : blocks4 >= 1024 ? 4 : 2;
+        int rows = blocks4 >= 65536 ? 32 : blocks4 >= 16384 ? 8 : blocks4 >= 1024 ? 4 : 2;
+        for (const SwShape& x : shapes) rows = std::max(rows, x.unit);
         const int64_t bps = (paths + kSwThreads * rows - 1) / (kSwThreads * rows);
         // the swaptions whose paths cost most first, so that the launch ends on
         // its cheapest blocks
@@ -1243,7 +1340,7 @@ extern "C" int bs_swaptions_host_f64(const bs_swaption_t* sw, int64_t n, int64_t
             SwBatch batch;
             for (; first < (size_t)n && batch.pool.size() < (size_t(1) << 24); ++first) {
                 const int32_t i = order[first];
-                batch.add(sw[i], shapes[(size_t)i], seed + i, i, bps * kSwThreads * rows);
+                batch.add(sw[i], shapes[(size_t)i], seed + i, i, paths);
             }
             const int rc = price_batch(batch, F, {paths, (int32_t)bps, rows}, trials, price,
                                        std_error, static_cast<hipStream_t>(stream));

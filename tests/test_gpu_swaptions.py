@@ -276,3 +276,34 @@ def test_both_ends_of_a_launch_give_the_same_bits(gpu, count, trials):
             check((p[half + i], e[half + i]), (q[i], f[i]), i)
     again = W.price(sws, trials, base, 1)
     assert same_bits(p, again[0]) and same_bits(e, again[1])
+
+
+def desk(count):
+    """Swaptions with 4 to 40 draws and 2 to 10 cash flows, starts at steps 1-10."""
+    return [sw(n=24, F=4, years=6.0, maturity=0.25 * (1 + i % 10), tenor=2.5 - 0.5 * (i % 4),
+               interval=0.25, strike=0.11 + 0.002 * i) for i in range(count)]
+
+
+@pytest.mark.parametrize("sws,trials", [
+    # work-items of 2, 4, 8 and 32 rows in the whole call (8 to 125,056 blocks of
+    # 1024 paths), fewer in its parts; units of 2, 4 and 8 rows
+    (lambda: W.parsec_portfolio(600)[0], 600), (lambda: W.parsec_portfolio(70)[0], 16_385),
+    (lambda: W.parsec_portfolio(65)[0], 262_145), (lambda: W.parsec_portfolio(128)[0], 524_288),
+    (lambda: W.parsec_portfolio(128)[0], 1_000_000), (lambda: desk(40), 30_001),
+    (lambda: desk(20) + W.parsec_portfolio(20)[0], 1_000),
+    (lambda: [dict(s, factors=s["factors"][:1]) for s in W.parsec_portfolio(9)[0]], 40_000),
+])
+@pytest.mark.parametrize("seed", [1979, 2147483647 - 30 * 700])
+def test_a_swaptions_bits_do_not_depend_on_the_call(gpu, sws, trials, seed):
+    """A swaption priced alone, in a shard and in the portfolio: the same bits,
+    also where the second seed's zero draw leaves paths to the step-by-step
+    kernel, and in launches that end by themselves as in those that don't."""
+    sws = sws()
+    if len({len(s["factors"]) for s in sws}) > 1:
+        sws = [dict(s, factors=s["factors"][:3]) for s in sws]
+    p, e = W.price(sws, trials, seed)
+    parts = {(0, 1), (len(sws) - 1, len(sws)), (len(sws) // 2, len(sws) // 2 + 1),
+             (0, len(sws) // 3), (len(sws) // 3, len(sws))}
+    for lo, hi in sorted(parts):
+        q, f = W.price(sws[lo:hi], trials, seed + lo)
+        assert same_bits(p[lo:hi], q) and same_bits(e[lo:hi], f), (lo, hi)
