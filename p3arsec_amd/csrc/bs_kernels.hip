@@ -131,10 +131,11 @@ void k_stream(Op op, int64_t n, int head) {
         op.scalar((int64_t)gid < head ? (int64_t)gid - head : n - rest + ((int64_t)gid - head));
 }
 
+// Blocks of a grid-stride kernel; a launch holds fewer than 2^32 work-items.
 inline unsigned grid_for(int64_t work_items, int64_t cap, int threads = kThreads) {
     int64_t blocks = (work_items + threads - 1) / threads;
     if (cap > 0 && blocks > cap) blocks = cap;
-    if (blocks > 0x7fffffff) blocks = 0x7fffffff;
+    blocks = std::min<int64_t>(blocks, 0xffffffff / threads);
     return (unsigned)(blocks < 1 ? 1 : blocks);
 }
 

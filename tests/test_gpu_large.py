@@ -74,3 +74,39 @@ def test_price_and_greeks_past_2_31_options(gpu):
         for b in held:
             gpu.call("bs_free", b)
         db.free()
+
+
+@pytest.mark.parametrize("n", [(1 << 32) - 63, 1 << 32])
+def test_two_passes_over_2_32_options(gpu, n):
+    """As many options as a launch holds work-items, and the largest book whose
+    two passes still share one: every input is the same array, of 2^20 numbers
+    over and over (36 GB in all)."""
+    x = np.random.default_rng(122).uniform(0.05, 0.65, TILE).astype(np.float32)
+    ty = np.arange(TILE, dtype=np.uint8) % 3 % 2
+    small = books.Book(*[x] * 5, ty)
+    db = gpu.DeviceBook(small)
+    want = gpu.price(db).download(np.float32, TILE)
+    held = []
+    try:
+        big_x, big_ty = alloc(gpu, n * 4, held), alloc(gpu, n, held)
+        for big, src, es in ((big_x, db.ptrs()[0], 4), (big_ty, db.ptrs()[5], 1)):
+            gpu.call("bs_memcpy_d2d", big, src, TILE * es, None)
+            done = TILE
+            while done < n:      # what is there once more
+                cnt = min(done, n - done)
+                gpu.call("bs_memcpy_d2d", big + done * es, big, cnt * es, None)
+                done += cnt
+        out = alloc(gpu, n * 4, held)
+        gpu.call("bs_price_passes_f32", *[big_x] * 5, big_ty, 1, out, n, 2, None)
+        gpu.call("bs_stream_sync", None)
+        for first in (0, 1 << 30, 1 << 31, n - n % TILE - TILE, n - n % TILE):
+            cnt = min(TILE, n - first)
+            got = np.empty(cnt, np.float32)
+            if cnt:
+                gpu.call("bs_memcpy_d2h", got.ctypes.data, out + first * 4, cnt * 4, None)
+                gpu.call("bs_stream_sync", None)
+            assert np.array_equal(got.view(np.uint32), want[:cnt].view(np.uint32)), first
+    finally:
+        for b in held:
+            gpu.call("bs_free", b)
+        db.free()
