@@ -524,9 +524,10 @@ __device__ __forceinline__ Greeks32 bs_greeks_of(float s, float k, float r, floa
     o.delta = __builtin_fmaf(a_bar, hw_rcp(s), s_bar);                // d log(S/K)/dS = 1/S
     o.vega = __builtin_fmaf(den_bar, f.sqrt_t, at_bar * v);
     o.rho = __builtin_fmaf(z, t, at_bar);                             // dFV = -FV (T dr + r dT)
-    // 1/sqrt(T) = v / den: v/2 den_bar / sqrt(T) = den_bar v^2/2 / den
+    // 1/sqrt(T) = v / den.  den_bar v and v / den are of the size of the result;
+    // den_bar / den is not, and overflows where sigma sqrt(T) < 1e-37.
     const float t_bar = __builtin_fmaf(a_bar, r + f.half_var,
-                                       __builtin_fmaf(den_bar * rden, f.half_var, z * r));
+                                       __builtin_fmaf(0.5f * (den_bar * v), v * rden, z * r));
     o.theta = -t_bar;
     return o;
 }

@@ -154,3 +154,28 @@ def test_price_output_on_degenerate_inputs(gpu):
     for g in got[1:]:
         assert np.all(np.isfinite(g[ordinary]))
     db.free()
+
+
+def test_greeks_of_tiny_volatilities(gpu):
+    """sigma sqrt(T) from FP32's smallest normal numbers up to 1e-20.  At the
+    money with r = 0, vega is S n(0) sqrt(T) and theta -S n(0) sigma / (2 sqrt(T));
+    off the money the option is the forward or nothing: vega 0, theta
+    -r K e^{-rT} of a call that will be exercised and + that of such a put.
+    CNDF's derivative at 0 is 6e-6 off n(0) and a dozen roundings add 1e-6."""
+    rows = [(100.0, 100.0, 0.0, v, t) for v in (2e-38, 1e-37, 1e-36, 1e-30, 1e-20)
+            for t in (0.5, 1.0, 4.0)]
+    rows += [(s, 190.0 - s, 0.05, v, 1.0) for s in (100.0, 90.0) for v in (2e-38, 1e-30, 1e-20)]
+    a = np.array(rows)
+    at_money = np.tile(a[:, 0] == a[:, 1], 2)
+    book = books.Book(*[np.concatenate([a[:, j]] * 2).astype(np.float32) for j in range(5)],
+                      np.repeat([0, 1], len(rows)).astype(np.uint8))
+    got, _ = gpu_greeks(gpu, book)
+    s, k, r, v, t = (x.astype(np.float64) for x in book.arrays()[:5])
+    put = book.otype != 0
+    n0 = s / np.sqrt(2 * np.pi)
+    vega = np.where(at_money, n0 * np.sqrt(t), 0.0)
+    exercised = np.where(s > k, ~put, put)
+    theta = np.where(at_money, -n0 * v / (2 * np.sqrt(t)),
+                     np.where(exercised, np.where(put, 1.0, -1.0) * r * k * np.exp(-r * t), 0.0))
+    assert np.all(np.abs(got[2] - vega) <= 2e-5 * vega)
+    assert np.all(np.abs(got[4] - theta) <= 2e-5 * np.abs(theta))
