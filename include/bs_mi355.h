@@ -150,7 +150,8 @@ int bs_price_greeks_f32(const float *s, const float *k, const float *r, const fl
  * each per-option value exactly the one bs_price_f32 / bs_price_greeks_f32
  * computes.  weights may be NULL (every w_i = 1).  sums is a device array of 1
  * or 5 doubles.  Summed in FP64 in a fixed order: bit-reproducible for a given
- * n, wherever the arrays start.  n == 0 writes zeros.  Calls on different
+ * n, wherever the arrays start, and sums[0] is the same bits with Greeks and
+ * without.  n == 0 writes zeros.  Calls on different
  * threads and streams are independent: each takes one of the library's 32
  * scratch slots (12 MB on each device), or stream-ordered memory when none is
  * free or the stream is being captured.  No reference counterpart: the

@@ -236,29 +236,34 @@ __global__ __launch_bounds__(kPfFinalThreads) void k_pf_final(const double* __re
     if (lane < NQ) out[lane] = pick(x, lane);
 }
 
-// Rows per wave: one while that makes fewer than pf_spread blocks, so that a
-// small book spreads over the chip; then up to the form's most, which keeps the
+// Rows per wave: one while that makes fewer than kPfSpread blocks, so that a
+// small book spreads over the chip; then up to kPfMostRows, which keeps the
 // blocks' counting in rare against their options; more only to stay within
-// kPfMaxBlocks.  10M options: price sums 38.8 us with at most 2 rows, 39.0 with
-// 4, 42 with 8, 44 with 16; Greeks and weights 54.9 with 4 and 8, 56 with 16.
+// kPfMaxBlocks.  With and without Greeks alike, so that the sum of prices has
+// the same bits in both.  us a call, price sums / with Greeks, for (rows, spread):
+//   1M options    (4, 1024)  8.4 / 13.1   (4, 512)  9.2 / 13.4   (8, 512)  9.2 / 13.4
+//   1.5M         10.4 / 15.1             10.5 / 15.2             11.6 / 16.5
+//   4M           19.6 / 26.7             19.2 / 26.7             20.0 / 25.7
+//   10M          40.8 / 53.2             40.9 / 52.8             41.5 / 50.7
+// and, of the Greeks form with weights, 10M 52.9, 53.6 and 54.2; price sums with
+// 16 rows 44.  In two launches the Greeks sums of 1M options take 12.2 us with a
+// spread of 512 and 13.7 with 1024.
 //
 // The whole call, against one wave per 8 rows and one final block in two
 // launches with stream-ordered scratch: 65,537 options 5.9 us and 23.4 (the
-// host's allocation); 1M 8.6 and 25, with Greeks 13.6 and 25; 10M 39.0 and
-// 47.1, with Greeks and weights 54.9 and 61 (the final block alone 8.8).
+// host's allocation); 1M 8.5 and 25, with Greeks 13.1 and 25; 10M 39.0 and
+// 47.1, with Greeks and weights 52.9 and 61 (the final block alone 8.8).
 // Bound by HBM (price) and VALU issue (Greeks).
-// One-row blocks that spread a book far enough: with 512 for the Greeks form, the
-// two-launch sums of 1M options take 12.2 us, with 1024 13.7.
-constexpr int64_t pf_spread(bool greeks) { return greeks ? 512 : 1024; }
-constexpr int64_t pf_most_rows(bool greeks) { return greeks ? 8 : 4; }
+constexpr int64_t kPfSpread = 1024;
+constexpr int64_t kPfMostRows = 4;
 
 struct PfShape {
     int64_t rows, blocks;
 };
-constexpr PfShape pf_shape(int64_t n, bool greeks) {
+constexpr PfShape pf_shape(int64_t n) {
     const int64_t items = n / 2 + (n & 1);
     auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-    int64_t rows = std::min(pf_most_rows(greeks), std::max<int64_t>(1, items / (kPfThreads * pf_spread(greeks))));
+    int64_t rows = std::min(kPfMostRows, std::max<int64_t>(1, items / (kPfThreads * kPfSpread)));
     rows = std::max(rows, up(items, kPfThreads * kPfMaxBlocks));
     return {rows, std::max<int64_t>(1, up(items, kPfThreads * rows))};
 }
@@ -266,7 +271,7 @@ constexpr PfShape pf_shape(int64_t n, bool greeks) {
 // slot NULL: the two-launch form with a.partial.
 template <bool kGreeks, bool AL>
 hipError_t launch_pf(PfArgs a, PfSlot* slot, uint32_t* busy, double* sums, hipStream_t st) {
-    const PfShape shape = pf_shape(a.n, kGreeks);
+    const PfShape shape = pf_shape(a.n);
     a.rows = shape.rows;
     if (slot) a.partial = slot->partial;
     // LDS reserved per block caps the waves resident on a CU: none by default
@@ -421,7 +426,7 @@ hipError_t launch_portfolio_f32(SoaIn<float> in, const uint8_t* type, const floa
         }
     }
     e = hipMallocAsync(reinterpret_cast<void**>(&a.partial),
-                       (size_t)pf_shape(n, greeks).blocks * (greeks ? 5 : 1) * sizeof(double), st);
+                       (size_t)pf_shape(n).blocks * (greeks ? 5 : 1) * sizeof(double), st);
     if (e != hipSuccess) return e;
     e = launch_pf_any(a, greeks, nullptr, nullptr, sums, st);
     const hipError_t f = hipFreeAsync(a.partial, st);

@@ -214,3 +214,18 @@ def test_inside_a_callers_graph(gpu):
     st.destroy()
     out.free()
     db.free()
+
+
+@pytest.mark.parametrize("n", [1, 4097, 524_287, 1_048_577, 1_600_001, 2_500_003, 10_000_000])
+@pytest.mark.parametrize("name", ["bs_portfolio_f32", "bs_portfolio_f32_noalloc"])
+def test_price_sum_with_and_without_greeks(gpu, name, n):
+    """sums[0] is the same bits whether Greeks are asked for or not, at every
+    number of rows a wave takes, with weights and without."""
+    rng = np.random.default_rng(n)
+    db = gpu.DeviceBook(books.make_book(n, books.SEED_BASE + 84))
+    w = gpu.DeviceBuffer.from_array(rng.uniform(-3.0, 10.0, n).astype(np.float32))
+    for wptr in (None, w.ptr):
+        one, five = (_sums(gpu, name, db, n, greeks, wptr) for greeks in (0, 1))
+        assert one[0] == five[0]
+    w.free()
+    db.free()
