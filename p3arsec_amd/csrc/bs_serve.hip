@@ -9,8 +9,8 @@
 //     memory to the device, then one fused kernel per section (the batch's
 //     price requests, its Greeks requests): a block prices one tile of 512
 //     options of one request, found by a 64-ary wave search of the table.  A
-//     batch of at most 32 requests and 2048 tiles is one kernel with the table
-//     as its argument.
+//     batch of at most 32 requests and 2048 tiles that finds nothing in flight
+//     is one kernel with the table as its argument.
 //     Launched directly (the default) each section's grid is one block per
 //     tile.  With use_graph the three kernels are captured once per slot and
 //     each batch is one hipGraphLaunch; before it, each section's node gets
@@ -177,10 +177,17 @@ using ServeGreeks = GreeksF32<kVW>;
 // A small batch in one launch: its table travels as the kernel's argument, and
 // one grid holds the price section's tiles, then the Greeks section's.  The
 // stage kernel and a kernel per section cost 14 us of GPU time and two launches
-// for requests that price in 3: at 20,000 Poisson requests/s p50 is 20.6 us and
-// was 25, at 300,000 27-35 and 48 (p99 92-108 and 130).  Larger batches keep
-// those (at saturation one kernel for both sections, at the Greeks form's
-// registers, ran 1.73e11 options/s against 1.76e11).
+// for requests that price in 3: 32 requests submitted together are done in 19 us
+// and 25, one of 1M options in 21 and 25.  Only a batch that finds nothing else
+// in flight takes it.  Where others are, a batch's wait is what the dispatcher's
+// next round can be filled with: with every small batch in this form, rounds
+// came more often and smaller, and the bulk lane's tail grew.  Three forms, all
+// small batches / those with nothing in flight / none, at a Poisson rate:
+//   20,000/s   p50 20.5, 22.2, 25.5 us     300,000/s  p50 38, 49, 49 us
+//   800,000/s  p99 209, 159, 151 us (of books up to 64K options 140, 132, 124)
+//   1,200,000/s p99 235, 183, 182 us (200, 140, 138)
+// Larger batches keep the three kernels (at saturation one kernel for both
+// sections, at the Greeks form's registers, ran 1.73e11 options/s against 1.76e11).
 constexpr int kSmallDesc = 32;
 constexpr int64_t kSmallTiles = 2048;
 struct SmallBatch {
@@ -260,6 +267,7 @@ struct HipExec {
     void* section_args[kSlots][1] = {};         // kernel arguments: &dev_slot[s]
     hipEvent_t ev[kSlots] = {};
     hipStream_t slot_stream[kSlots] = {};        // the stream slot s was last launched on
+    bool in_flight[kSlots] = {};                 // launched and not seen to end (dispatcher only)
     int64_t seq = 0, nlaunch = 0;
     struct Reply {
         std::mutex mu;
@@ -411,10 +419,12 @@ struct HipExec {
     void thread_start() { (void)hipSetDevice(device); }
 
     // Launches slot s on its lane's stream (the bulk lane alternates between
-    // two): graph replay, or the stage kernel
-    // and the fused kernel of each non-empty section directly; each section's
-    // grid is one block per tile.  Then records the slot's event.
+    // two): graph replay, or directly: a small batch with nothing else in flight
+    // as one kernel, any other as the stage kernel and the fused kernel of each
+    // non-empty section; each section's grid is one block per tile.  Then
+    // records the slot's event.
     int launch(int s, const std::vector<serve::Admitted>& reqs, std::string* err) {
+        const bool alone = std::none_of(in_flight, in_flight + kSlots, [](bool f) { return f; });
         write_slot(s, reqs);
         hipStream_t st = s < kSmallSlots ? streams[2] : streams[nlaunch++ & 1];
         slot_stream[s] = st;
@@ -427,7 +437,7 @@ struct HipExec {
                 e = set_section_grid(s, sec, (unsigned)blocks);
             }
             if (e == hipSuccess) e = hipGraphLaunch(graph[s], st);
-        } else if (h->ndesc[0] + h->ndesc[1] <= kSmallDesc &&
+        } else if (alone && h->ndesc[0] + h->ndesc[1] <= kSmallDesc &&
                    h->tiles[0] + h->tiles[1] <= std::min(kSmallTiles, grid_cap)) {
             SmallBatch b;
             b.np = h->ndesc[0];
@@ -453,11 +463,13 @@ struct HipExec {
         }
         if (e == hipSuccess) e = hipEventRecord(ev[s], st);
         if (e != hipSuccess) *err = hipGetErrorString(e);
+        in_flight[s] = e == hipSuccess;   // a failed launch is quiesced before the next
         return e == hipSuccess ? 0 : -1;
     }
     int query(int s, std::string* err) {
         const hipError_t q = hipEventQuery(ev[s]);
         if (q == hipErrorNotReady) return 0;
+        in_flight[s] = false;
         if (q == hipSuccess) return 1;
         *err = hipGetErrorString(q);
         return -1;

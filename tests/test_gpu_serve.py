@@ -386,3 +386,21 @@ def test_small_batches_in_one_launch(gpu, sizes):
             for a, b in zip(ctx.result(tickets[i], sizes[i], kinds[i]), want[i]):
                 assert np.array_equal(a.view(np.uint32), b), (i, kinds[i])
         ctx.destroy()
+
+
+def test_small_batches_behind_others(gpu):
+    """Small requests that come while a large batch runs, and alone after it:
+    both forms of a small batch give the bits of each book alone."""
+    sizes = (3_000_001, 700, 65_536, 513, 1)
+    bks = [books.make_book(n, books.SEED_BASE + 97 + i) for i, n in enumerate(sizes)]
+    want = [[o.download(np.uint32, b.n) for o in gpu.greeks(gpu.DeviceBook(b))] for b in bks]
+    ctx = Ctx(gpu, 1 << 30, use_graph=0)
+    ids = [ctx.register(b) for b in bks]
+    for rnd in range(6):
+        batch = [(i, 1 + (i + rnd) % 2) for i in ((0, 1, 0, 2, 3, 4, 1) if rnd % 2 else (4, 2, 1))]
+        for (i, kind), t in [(x, ctx.submit(ids[x[0]], x[1])) for x in batch]:
+            assert ctx.wait(t) == 0
+            for a, b in zip(ctx.result(t, sizes[i], kind), want[i]):
+                assert np.array_equal(a.view(np.uint32), b), (rnd, i, kind)
+            gpu.call("bs_result_release", ctx.h, t)
+    ctx.destroy()
