@@ -266,10 +266,6 @@ __device__ __forceinline__ double recip64(double b) {
 }
 
 constexpr double kSqrtHalf = 0.70710678118654752440;
-// ln 2 = kLn2Hi + kLn2Lo; kLn2Hi keeps 32 significant bits, so e * kLn2Hi is
-// exact for every binary exponent e of a double.
-constexpr double kLn2Hi = 0.6931471803691238;        // 0x3fe62e42fee00000
-constexpr double kLn2Lo = 1.9082149292705877e-10;
 
 // Natural logarithm.  x = 2^e m with m in [sqrt(1/2), sqrt(2)); f = m - 1 is
 // exact and s = f / (2 + f), |s| <= 0.1716.  Then
@@ -312,9 +308,9 @@ __device__ __forceinline__ double log64(double x) {
 }
 
 // Ref64Ordinary: Ref64's statements for ordinary inputs (Ref64::unchecked_holds),
-// with the primitives of bs_fp64.hpp: quotients and the square root within half
-// an ulp and 2^-24 of one, as IEEE's to the eye, exp and log within an ulp, none
-// of them with code for special values.  |x| of CNDF is capped at 40, past
+// with the primitives of bs_fp64.hpp, none of which has code for special values
+// and none a larger error than the general one: quotients and the square root
+// within half an ulp and 2^-19 of one, exp and log within 0.88.  |x| of CNDF is capped at 40, past
 // which e^{-x^2/2} is 0 and CNDF exactly 0 or 1.
 struct Ref64Ordinary {
     using T = double;

@@ -287,7 +287,7 @@ __device__ __forceinline__ double moro_tail_fma(uint32_t residue) {
     const bool upper = residue > (uint32_t)kM31 / 2;
     const double w = __builtin_fma((double)residue, upper ? -4.656612875e-10 : 4.656612875e-10,
                                    upper ? 1.0 : 0.0);
-    const double t = log_pos(-log_pos(w));
+    const double t = log_near(-log_near(w));
     double v = __builtin_fma(t, 0.0000003960315187, 0.0000002888167364);
     v = __builtin_fma(t, v, 0.0000321767881768);
     v = __builtin_fma(t, v, 0.0003951896511919);

@@ -368,3 +368,37 @@ def test_fp64_at_the_edges_of_ordinary_inputs(gpu, oracle, which):
     scale = (book.s + book.k + fv)[fin]
     rel = np.maximum(1.0, np.abs(book.r * book.t))[fin]   # exp's own conditioning
     assert np.all(np.abs(got[fin] - ref[fin]) <= 3.6e-15 * scale * rel)
+
+
+@pytest.fixture(scope="module")
+def fp64_errors():
+    """{function: (largest, mean) error} of tests/native/fp64_ordinary.hip."""
+    import subprocess
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native", "fp64_ordinary")
+    assert os.path.exists(exe), "build it: make -C tests/native fp64_ordinary"
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    print(r.stdout)
+    assert r.returncode == 0, r.stderr
+    return {f[0]: (float(f[2]), float(f[4])) for f in map(str.split, r.stdout.splitlines())}
+
+
+@pytest.mark.parametrize("ordinary,general", [("recip_pos", "recip64"), ("quot_pos", "division"),
+                                              ("sqrt_pos", "sqrt"), ("log_pos", "log64"),
+                                              ("exp_mid", "exp")])
+def test_fp64_primitives_for_ordinary_numbers(gpu, fp64_errors, ordinary, general):
+    """On the same inputs, the primitives of ordinary options have no larger an
+    error, at most and on average, than those of the general path.  Quotients and
+    roots leave out relative terms of 2^-72, 2^-19 ulp."""
+    (most, mean), (most_general, mean_general) = fp64_errors[ordinary], fp64_errors[general]
+    slack = 2.0 ** -19 if most_general < 0.51 else 0.0
+    assert most <= most_general + slack and mean <= mean_general + slack
+
+
+def test_fp64_seeds_and_ends_of_the_range(gpu, fp64_errors):
+    """The hardware's reciprocal and reciprocal root over every binade, which the
+    Newton steps' error rests on (2^-24), e^x down to the smallest subnormal (its
+    last rounding is a second one) and 2^x."""
+    assert fp64_errors["rcp_relative"][0] < 2.0 ** -24
+    assert fp64_errors["rsq_relative"][0] < 2.0 ** -24
+    assert fp64_errors["exp_mid_subnormal"][0] <= 1.0
+    assert fp64_errors["exp2_mid"][0] <= 1.0
