@@ -59,6 +59,7 @@
 #include "bs_arrive.hpp"
 #include "bs_fp64.hpp"
 #include "bs_internal.hpp"
+#include "bs_moro.hpp"
 #include "bs_wave.hpp"
 
 namespace bs {
@@ -70,7 +71,6 @@ constexpr int kSwMaxSteps = 64;           // n_steps
 constexpr int kSwMaxFactors = 8;          // n_factors
 constexpr int kSwMaxDraws = 64;           // start index x n_factors
 constexpr int64_t kSwCounterLimit = int64_t(1) << 42;
-constexpr uint64_t kM31 = 2147483647u;
 
 // How a launch's blocks cover the paths: block b takes swaption b / bps, its
 // paths [(b % bps) kSwThreads rows, + kSwThreads rows), `rows` of them per
@@ -121,34 +121,6 @@ __device__ __forceinline__ double ran_unif(int64_t c) {
     uint64_t x = mod_m31((uint64_t)c * 1513517u);
     x = mod_m31(x * 16807u);
     return (double)(int64_t)x * 4.656612875e-10;
-}
-
-// Moro's inverse normal (Moro 1995; Glasserman, Monte Carlo Methods in
-// Financial Engineering, fig. 2.13), as PARSEC's CumNormalInv evaluates it:
-// a rational function of x = u - 0.5 for |x| < 0.42, a Chebyshev series in
-// log(-log(min(u, 1 - u))) outside.
-__device__ __forceinline__ double moro_central(double x) {
-    const double r = x * x;
-    const double num = x * (((-25.44106049637 * r + 41.39119773534) * r + -18.61500062529) * r +
-                            2.50662823884);
-    const double den = (((3.13082909833 * r + -21.06224101826) * r + 23.08336743743) * r +
-                        -8.47351093090) * r + 1.0;
-    return num / den;
-}
-
-__device__ __forceinline__ double moro_tail(double u) {
-    const double x = u - 0.5;
-    double t = x > 0.0 ? 1.0 - u : u;
-    t = log(-log(t));
-    t = 0.3374754822726147 + t * (0.9761690190917186 + t * (0.1607979714918209 +
-        t * (0.0276438810333863 + t * (0.0038405729373609 + t * (0.0003951896511919 +
-        t * (0.0000321767881768 + t * (0.0000002888167364 + t * 0.0000003960315187)))))));
-    return x < 0.0 ? -t : t;
-}
-
-__device__ __forceinline__ double moro_inv(double u) {
-    const double x = u - 0.5;
-    return fabs(x) < 0.42 ? moro_central(x) : moro_tail(u);
 }
 
 // The normal draws of path p: z[s][k] = Z_k(s + 1) for s < m.
@@ -229,74 +201,6 @@ constexpr uint32_t gen_step(uint64_t counters) {
 __device__ __forceinline__ uint32_t add_m31(uint32_t a, uint32_t b) {
     const uint32_t t = a + b;
     return min(t, t - (uint32_t)kM31);   // t < M: t - M wraps past it
-}
-
-// Residues whose uniform |u - 0.5| >= 0.42 takes Moro's tail: x <= kTailLo or
-// x >= kTailHi, u rounded as in ran_unif.
-constexpr bool in_tail(uint32_t x) {
-    const double d = (double)x * 4.656612875e-10 - 0.5;
-    return !((d < 0 ? -d : d) < 0.42);
-}
-constexpr uint32_t tail_edge(bool upper) {
-    uint32_t a = upper ? (uint32_t)kM31 / 2 : 0, b = upper ? (uint32_t)kM31 - 1 : (uint32_t)kM31 / 2;
-    while (b - a > 1) {   // upper: b is in the tail and a is not; lower: a is and b is not
-        const uint32_t c = a + (b - a) / 2;
-        if (in_tail(c) == upper) b = c;
-        else a = c;
-    }
-    return upper ? b : a;
-}
-constexpr uint32_t kTailLo = tail_edge(false), kTailHi = tail_edge(true);
-static_assert(in_tail(kTailLo) && !in_tail(kTailLo + 1) && in_tail(kTailHi) &&
-                  !in_tail(kTailHi - 1) && in_tail(0) && in_tail((uint32_t)kM31 - 1),
-              "tail residues");
-
-// A constant held in a vector register from here on.  An FP64 instruction reads
-// one scalar operand at most and there are not enough scalar registers for
-// every constant of k_sw_paths, so the compiler otherwise builds the central
-// branch's constants anew for every draw, 6 of its 23 instructions.
-__device__ __forceinline__ double pinned(double c) {
-    asm("" : "+v"(c));
-    return c;
-}
-
-// Moro's two branches (moro_central, moro_tail) with FMAs.
-struct MoroCentral {
-    double scale = pinned(4.656612875e-10);
-    double a1 = pinned(-25.44106049637), a2 = pinned(41.39119773534),
-           a3 = pinned(-18.61500062529), a4 = pinned(2.50662823884);
-    double b1 = pinned(3.13082909833), b2 = pinned(-21.06224101826),
-           b3 = pinned(23.08336743743), b4 = pinned(-8.47351093090);
-    // The normal of residue x's uniform, for the residues outside the tail.
-    __device__ __forceinline__ double operator()(uint32_t residue) const {
-        const double x = __builtin_fma((double)residue, scale, -0.5);
-        const double r = x * x;
-        double num = __builtin_fma(r, a1, a2);
-        num = __builtin_fma(r, num, a3);
-        num = __builtin_fma(r, num, a4);
-        double den = __builtin_fma(r, b1, b2);
-        den = __builtin_fma(r, den, b3);
-        den = __builtin_fma(r, den, b4);
-        den = __builtin_fma(r, den, 1.0);   // 0.11 <= den <= 1 for |x| <= 0.42
-        return quot_near(x * num, den);
-    }
-};
-
-// The normal of a nonzero residue in the tail: log(-log(min(u, 1 - u))).
-__device__ __forceinline__ double moro_tail_fma(uint32_t residue) {
-    const bool upper = residue > (uint32_t)kM31 / 2;
-    const double w = __builtin_fma((double)residue, upper ? -4.656612875e-10 : 4.656612875e-10,
-                                   upper ? 1.0 : 0.0);
-    const double t = log_near(-log_near(w));
-    double v = __builtin_fma(t, 0.0000003960315187, 0.0000002888167364);
-    v = __builtin_fma(t, v, 0.0000321767881768);
-    v = __builtin_fma(t, v, 0.0003951896511919);
-    v = __builtin_fma(t, v, 0.0038405729373609);
-    v = __builtin_fma(t, v, 0.0276438810333863);
-    v = __builtin_fma(t, v, 0.1607979714918209);
-    v = __builtin_fma(t, v, 0.9761690190917186);
-    v = __builtin_fma(t, v, 0.3374754822726147);
-    return upper ? v : -v;
 }
 
 // Whether the linear form takes the kSwThreads rows paths from `first` on: the

@@ -4,11 +4,12 @@
 // device library's exp, log64 and recip64 of bs_math.hpp, IEEE division and
 // square root).  Inputs: random numbers of the ranges the map and the swaptions
 // meet, every binade of the range a function states, and the neighbourhoods of
-// sqrt(1/2), 1 and sqrt(2).
+// sqrt(1/2), 1 and sqrt(2).  Moro's inverse normal (bs_moro.hpp) in the form the
+// linear kernel takes and in the reference's, in absolute error.
 //
 //   fp64_ordinary     prints "name inputs max at mean" per function: errors in
 //                     ulps, relative ones of the hardware's reciprocal and
-//                     reciprocal root over every binade.
+//                     reciprocal root over every binade, absolute ones of Moro's.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -20,6 +21,7 @@
 #include <vector>
 
 #include "bs_math.hpp"
+#include "bs_moro.hpp"
 
 #define HIP_OK(x)                                                                  \
     do {                                                                           \
@@ -31,7 +33,7 @@
     } while (0)
 
 enum Fn { kQuotPos, kDiv, kRecipPos, kRecip64, kSqrtPos, kSqrt, kLogPos, kLog64, kExpMid, kExp,
-          kExp2Mid, kRcp, kRsq, kLog };
+          kExp2Mid, kRcp, kRsq, kMoro, kMoroRef, kLog };
 
 __global__ void k_eval(int fn, const double* a, const double* b, double* y, int64_t n) {
 #pragma clang fp contract(off)
@@ -53,12 +55,40 @@ __global__ void k_eval(int fn, const double* a, const double* b, double* y, int6
         case kRcp: y[i] = __builtin_amdgcn_rcp(x); break;
         case kRsq: y[i] = __builtin_amdgcn_rsq(x); break;
         case kLog: y[i] = ::log(x); break;
+        case kMoro: {   // x: a residue
+            const uint32_t r = (uint32_t)x;
+            const bs::MoroCentral central;
+            y[i] = r > bs::kTailLo && r < bs::kTailHi ? central(r) : bs::moro_tail_fma(r);
+            break;
+        }
+        case kMoroRef: y[i] = bs::moro_inv(x * 4.656612875e-10); break;
     }
+}
+
+// Moro's inverse normal of u (Glasserman 2003, fig. 2.13).
+static long double moro(long double u) {
+    static const double A[] = {2.50662823884, -18.61500062529, 41.39119773534, -25.44106049637};
+    static const double B[] = {-8.47351093090, 23.08336743743, -21.06224101826, 3.13082909833};
+    static const double C[] = {0.3374754822726147, 0.9761690190917186, 0.1607979714918209,
+                               0.0276438810333863, 0.0038405729373609, 0.0003951896511919,
+                               0.0000321767881768, 0.0000002888167364, 0.0000003960315187};
+    const long double x = u - 0.5L;
+    auto horner = [](const double* c, int n, long double t) {
+        long double v = c[n - 1];
+        for (int i = n - 2; i >= 0; --i) v = v * t + c[i];
+        return v;
+    };
+    if (fabs((double)x) < 0.42)
+        return x * horner(A, 4, x * x) / (horner(B, 4, x * x) * (x * x) + 1.0L);
+    const long double v = horner(C, 9, logl(-logl(x > 0 ? 1.0L - u : u)));
+    return x < 0 ? -v : v;
 }
 
 static long double exact(int fn, double a, double b) {
     const long double x = a;
     switch (fn) {
+        case kMoro:
+        case kMoroRef: return moro(a * 4.656612875e-10);   // u as ran_unif rounds it
         case kQuotPos:
         case kDiv: return x / b;
         case kRecipPos:
@@ -156,6 +186,16 @@ int main() {
     x.clear();
     uniform(-4.0, 4.0, N, &x), uniform(-1000.0, 1000.0, N, &x);
     run("exp2_mid", kExp2Mid, x, none);
+    for (bool tail : {false, true}) {
+        x.clear();
+        for (size_t i = 0; i < N; ++i) {
+            const uint64_t width = tail ? bs::kTailLo : bs::kTailHi - bs::kTailLo - 1;
+            const uint64_t r = rng() % width + (tail ? 1 : bs::kTailLo + 1);
+            x.push_back((double)(tail && i % 2 ? bs::kM31 - r : r));
+        }
+        run(tail ? "moro_tail" : "moro_central", kMoro, x, none, 'a');
+        run(tail ? "moro_tail_reference" : "moro_central_reference", kMoroRef, x, none, 'a');
+    }
     HIP_OK(hipFree(da));
     HIP_OK(hipFree(db));
     HIP_OK(hipFree(dy));

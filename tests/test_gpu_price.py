@@ -402,3 +402,12 @@ def test_fp64_seeds_and_ends_of_the_range(gpu, fp64_errors):
     assert fp64_errors["rsq_relative"][0] < 2.0 ** -24
     assert fp64_errors["exp_mid_subnormal"][0] <= 1.0
     assert fp64_errors["exp2_mid"][0] <= 1.0
+
+
+@pytest.mark.parametrize("branch", ["moro_central", "moro_tail"])
+def test_normals_of_the_linear_swaptions(gpu, fp64_errors, branch):
+    """Moro's inverse normal as the linear swaptions kernel forms it, from the
+    uniform that the reference rounds: no larger an error, at most and on
+    average, than the reference's own statements have."""
+    (most, mean), (most_ref, mean_ref) = fp64_errors[branch], fp64_errors[branch + "_reference"]
+    assert most <= most_ref and mean <= mean_ref
