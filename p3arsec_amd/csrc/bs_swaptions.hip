@@ -123,11 +123,19 @@ __device__ __forceinline__ double ran_unif(int64_t c) {
     return (double)(int64_t)x * 4.656612875e-10;
 }
 
-// The normal draws of path p: z[s][k] = Z_k(s + 1) for s < m.
+// Loops over a path's steps are unrolled where its draws then fit registers.
+constexpr int unrolled(int factors, int steps) {
+    return steps <= 8 && steps * factors <= 32 ? steps : 1;
+}
+
+// The normal draws of path p: z[s][k] = Z_k(s + 1) for s < m <= MAXM.
 template <int F, int MAXM>
 __device__ __forceinline__ void draws(const SwHead& h, int64_t p, double (&z)[MAXM][F]) {
+    constexpr int kUnroll = unrolled(F, MAXM);
     const int64_t c0 = h.seed + p * (int64_t)((h.n - 1) * F);
-    for (int s = 0; s < h.m; ++s) {
+#pragma unroll kUnroll
+    for (int s = 0; s < MAXM; ++s) {
+        if (s >= h.m) break;
 #pragma unroll
         for (int k = 0; k < F; ++k) z[s][k] = moro_inv(ran_unif(c0 + s * F + k));
     }
@@ -140,6 +148,7 @@ __device__ __forceinline__ void draws(const SwHead& h, int64_t p, double (&z)[MA
 template <int F, int MAXM>
 __device__ __forceinline__ double path_payoff(const SwHead& h, const double* __restrict__ q,
                                               const double (&z)[MAXM][F]) {
+    constexpr int kUnroll = unrolled(F, MAXM);
     const int n = h.n, m = h.m, L = h.L, w = n - 1;
     const double* f0 = q;
     const double* mudt = q + n;
@@ -150,7 +159,9 @@ __device__ __forceinline__ double path_payoff(const SwHead& h, const double* __r
     for (int d = 0; d < dend; ++d) {
         double x = f0[d];
         const int steps = min(d, m);
-        for (int s = 1; s <= steps; ++s) {
+#pragma unroll kUnroll
+        for (int s = 1; s <= MAXM; ++s) {
+            if (s > steps) break;
             const int l = d - s;
             double shock = 0.0;
 #pragma unroll
@@ -648,28 +659,25 @@ __attribute__((amdgpu_waves_per_eu(MAXW <= 8 ? 4 : MAXW <= 32 ? 3 : 2))) void k_
                  done, reinterpret_cast<double*>(lds));
 }
 
-// The units that k_sw_paths left out, one path at a time per work-item (the
-// draws live in scratch).
+// The units that k_sw_paths left out, one path at a time per work-item: block b
+// takes the units b % bps, + bps, ... of swaption b / bps.
 template <int F, int MAXM>
 __global__ __launch_bounds__(kSwThreads) void k_sw_paths_steps(
     const SwLin* __restrict__ lin, const SwHead* __restrict__ heads,
-    const double* __restrict__ pool, SwGrid grid, double* __restrict__ partial) {
-    const int sw = (int)(blockIdx.x / (unsigned)grid.bps);
-    const int64_t chunk = blockIdx.x % (unsigned)grid.bps;
+    const double* __restrict__ pool, int64_t paths, int bps, double* __restrict__ partial) {
+    const int sw = (int)(blockIdx.x / (unsigned)bps);
     const SwLin x = lin[sw];
-    const int64_t first = chunk * (kSwThreads * grid.rows);
-    if (rows_linear(x, first, grid.rows)) return;
-    const SwHead h = heads[sw];
-    const double* q = pool + h.off;
 #pragma unroll 1
-    for (int64_t at = first; at < first + kSwThreads * grid.rows && at < grid.paths;
-         at += kSwThreads * x.unit) {
-        if (rows_linear(x, at, x.unit)) continue;
+    for (int u = (int)(blockIdx.x % (unsigned)bps); u < x.units; u += bps) {
+        const int64_t first = (int64_t)u * (kSwThreads * x.unit);
+        if (rows_linear(x, first, x.unit)) continue;
+        const SwHead h = heads[sw];
+        const double* q = pool + h.off;
         double sum = 0.0, sumsq = 0.0;
 #pragma unroll 1
         for (int j = 0; j < x.unit; ++j) {
-            const int64_t p = at + j * kSwThreads + threadIdx.x;
-            if (p < grid.paths) {
+            const int64_t p = first + j * kSwThreads + threadIdx.x;
+            if (p < paths) {
                 double z[MAXM][F];
                 draws<F, MAXM>(h, p, z);
                 const double v = path_payoff<F, MAXM>(h, q, z);
@@ -679,7 +687,7 @@ __global__ __launch_bounds__(kSwThreads) void k_sw_paths_steps(
         }
         block_sums(&sum, &sumsq);
         if (threadIdx.x == 0) {
-            double* mine = partial + 2 * (x.unit0 + at / (kSwThreads * x.unit));
+            double* mine = partial + 2 * ((int64_t)x.unit0 + u);
             mine[0] = sum;
             mine[1] = sumsq;
         }
@@ -727,14 +735,37 @@ LaunchLin linear_kernel(int flows) {
                          : launch_linear<64>;
 }
 
+// What the step-by-step kernel covers.  Its form goes by the latest start of the
+// swaptions: up to 2, 4 or (4 factors at most) 8 steps the draws stay in registers
+// (56-116 VGPRs), beyond they live in scratch.  32 swaptions x 50,000 trials whose
+// rates are past the linear form's bound, us a call with the registers' form and
+// with the scratch's throughout: 3 factors, starts at steps 1-2 124 and 156; 4
+// factors, 1-4 243 and 438, 1-8 344 and 621; 1-10 (scratch) 672.  A linear
+// portfolio with a zero draw in one unit of each swaption, 128 x 1M: 867, and 769
+// without.
+struct SwSteps {
+    int64_t paths;
+    int start, units;   // the latest start and the most units of the swaptions
+};
+template <int F, int MAXM>
+void launch_steps_of(unsigned n, hipStream_t st, const SwLin* lin, const SwHead* heads,
+                     const double* pool, const SwSteps& x, double* partial) {
+    // a launch holds fewer than 2^32 work-items
+    const unsigned bps = std::min<unsigned>(x.units, std::max(1u, 0xffffffffu / kSwThreads / n));
+    hipLaunchKernelGGL((k_sw_paths_steps<F, MAXM>), dim3(n * bps), dim3(kSwThreads), 0, st, lin,
+                       heads, pool, x.paths, (int)bps, partial);
+}
 template <int F>
-void launch_steps(unsigned blocks, hipStream_t st, const SwLin* lin, const SwHead* heads,
-                  const double* pool, const SwGrid& grid, double* partial) {
-    hipLaunchKernelGGL((k_sw_paths_steps<F, kSwMaxDraws / F>), dim3(blocks), dim3(kSwThreads), 0,
-                       st, lin, heads, pool, grid, partial);
+void launch_steps(unsigned n, hipStream_t st, const SwLin* lin, const SwHead* heads,
+                  const double* pool, const SwSteps& x, double* partial) {
+    if (x.start <= 2) return launch_steps_of<F, 2>(n, st, lin, heads, pool, x, partial);
+    if (x.start <= 4) return launch_steps_of<F, 4>(n, st, lin, heads, pool, x, partial);
+    if constexpr (F <= 4)
+        if (x.start <= 8) return launch_steps_of<F, 8>(n, st, lin, heads, pool, x, partial);
+    launch_steps_of<F, kSwMaxDraws / F>(n, st, lin, heads, pool, x, partial);
 }
 using LaunchSteps = void (*)(unsigned, hipStream_t, const SwLin*, const SwHead*, const double*,
-                             const SwGrid&, double*);
+                             const SwSteps&, double*);
 constexpr LaunchSteps kStepsByFactors[kSwMaxFactors] = {
     launch_steps<1>, launch_steps<2>, launch_steps<3>, launch_steps<4>,
     launch_steps<5>, launch_steps<6>, launch_steps<7>, launch_steps<8>};
@@ -1049,6 +1080,7 @@ struct SwBatch {
     std::vector<int32_t> index;   // places in the caller's array
     int flows = 0;
     int32_t units = 0;
+    int start = 0, most = 0;      // the latest start and the most units of a swaption
     bool steps = false;           // some unit needs the step-by-step kernel
 
     void add(const bs_swaption_t& s, const SwShape& x, int64_t seed, int32_t i, int64_t paths) {
@@ -1059,12 +1091,15 @@ struct SwBatch {
         pack_linear(heads.back(), s.n_factors, x.freq, x.points, &lins.back(), &pool);
         SwLin& l = lins.back();
         flows = std::max(flows, l.flows);
-        l.unit = x.unit;
-        l.units = (int32_t)((paths + kSwThreads * x.unit - 1) / (kSwThreads * x.unit));
+        // swaptions that the step-by-step kernel prices whole: units of 2 rows
+        l.unit = l.linear ? x.unit : unit_rows(false, paths);
+        l.units = (int32_t)((paths + kSwThreads * l.unit - 1) / (kSwThreads * l.unit));
         l.unit0 = units;
         units += l.units;
+        start = std::max(start, x.m);
+        most = std::max(most, l.units);
         steps = steps || !l.linear ||
-                draws_zero(seed, (int64_t)l.units * kSwThreads * x.unit * l.per_path);
+                draws_zero(seed, (int64_t)l.units * kSwThreads * l.unit * l.per_path);
     }
 };
 
@@ -1099,7 +1134,8 @@ hipError_t launch_batch(const SwBatch& b, const SwLayout& at, int F, const SwGri
     const double* dp = reinterpret_cast<const double*>(base + at.pool);
     double* dq = reinterpret_cast<double*>(base + at.partial);
     linear_kernel(b.flows)(blocks, st, dl, dp, grid, dq, done);
-    if (b.steps) kStepsByFactors[F - 1](blocks, st, dl, dh, dp, grid, dq);
+    if (b.steps)
+        kStepsByFactors[F - 1](n, st, dl, dh, dp, {grid.paths, b.start, b.most}, dq);
     if (!done.counters)
         hipLaunchKernelGGL(k_sw_final, dim3(n), dim3(kSwThreads), 0, st, dl, dq, trials, out);
     return hipGetLastError();

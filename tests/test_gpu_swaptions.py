@@ -307,3 +307,25 @@ def test_a_swaptions_bits_do_not_depend_on_the_call(gpu, sws, trials, seed):
     for lo, hi in sorted(parts):
         q, f = W.price(sws[lo:hi], trials, seed + lo)
         assert same_bits(p[lo:hi], q) and same_bits(e[lo:hi], f), (lo, hi)
+
+
+@pytest.mark.parametrize("F", [1, 3, 4, 5, 8])
+@pytest.mark.parametrize("start", [1, 2, 3, 4, 5, 8, 9, 12])
+def test_step_by_step_forms(gpu, F, start):
+    """At the edges of the step-by-step kernel's forms (starts at up to 2, 4 and 8
+    steps, and beyond): path 700's last draw, which no payoff reads, is u = 0, so
+    its unit of paths goes to that kernel; beside a swaption that is priced by it
+    whole.  The bar is the file's."""
+    if start * F > 64:
+        pytest.skip("more than 64 draws")
+    n = 26
+    per_path = (n - 1) * F
+    seed = 2147483647 - 700 * per_path - (per_path - 1)
+    s = sw(n=n, F=F, years=0.25 * n, maturity=start * 0.25, tenor=1.0, interval=0.25, strike=0.13)
+    whole = dict(s, years=400.0 * n, maturity=start * 400.0, tenor=1600.0, interval=400.0,
+                 strike=0.01)
+    p, e = W.price([s, whole], 3000, seed, 1)
+    for i, x in enumerate((s, whole)):
+        check((p[i], e[i]), S.price_blocking(x, seed + i, 3000, 1), i)
+        q, f = W.price([x], 3000, seed + i, 1)
+        assert same_bits(p[i:i + 1], q) and same_bits(e[i:i + 1], f)
