@@ -143,30 +143,53 @@ void k_serve(const uint8_t* __restrict__ slot) {
 }
 
 // ---- replies -----------------------------------------------------------------
-// bs_result_copy's way to the host: one kernel writes the wanted span of a
-// request's outputs (contiguous in the arena) into pinned memory and then the
-// reply's sequence number, on which the caller spins; the arrays go on to the
-// caller's from there.  The runtime's own copies take 11-35 us each to pageable
-// memory (copy kernel, marker, interrupt), five of them for a Greeks request:
-// a round of 32 requests of up to 64K options, one third with Greeks, submitted,
-// waited for and copied out one by one takes 390 us, with those copies 1050.
+// bs_result_copy's way to the host: one kernel writes the wanted outputs of a
+// request (one span of the arena where they lie side by side) into pinned memory
+// and then the reply's sequence number, on which the caller spins; the arrays go
+// on to the caller's from there.  The runtime's own copies take 11-35 us each to pageable memory (copy
+// kernel, marker, interrupt), five of them for a Greeks request: a round of 32
+// requests of up to 64K options, one third with Greeks, submitted, waited for
+// and copied out one by one takes 390 us, with those copies 1050.
 // Bound by the launch and the link's latency.
+//
+// us a copy, reply and runtime: price of 1000 options 7.7 and 14.6, of 65,536
+// 18.2 and 20.1; all five Greeks outputs of 1000 9.3 and 70, of 65,536 61 and 96,
+// price and theta of 65,536 28 and 38.  A reply holds the largest request of the
+// small lane with Greeks; past it the gain is less (of 131,072, all five 121 and
+// 150, price alone 28 and 29).  Two replies, as one thread's memcpy is the other's
+// kernel: 1, 2, 4 and 8 threads copying 16,384 options with Greeks get one every
+// 22.2, 12.9, 11.9, 12.0 us (22.2, 13.0, 8.9, 9.5 with four; 61-69 by the runtime).
 constexpr int kReplies = 2;                         // replies on their way at once
 constexpr size_t kReplyBytes = size_t(3) << 19;     // 1.5 MB: the Greeks of 64K options
 constexpr int kReplyBlocks = 64;
 
-__global__ __launch_bounds__(kThreads) void k_reply(const uint64_t* __restrict__ src,
-                                                    uint64_t* __restrict__ dst, int words,
-                                                    uint32_t* count, uint32_t* flag,
-                                                    uint32_t seq) {
+// This block's part of `words` 8-byte words; the last block raises the flag.
+__device__ __forceinline__ void reply_words(const uint64_t* __restrict__ src,
+                                            uint64_t* __restrict__ dst, int words, uint32_t blocks,
+                                            uint32_t* count, uint32_t* flag, uint32_t seq) {
     for (int i = blockIdx.x * kThreads + threadIdx.x; i < words; i += gridDim.x * kThreads)
         system_store(dst + i, src[i]);
     stores_done();
     __syncthreads();
-    if (threadIdx.x == 0 && arrive_one(count, gridDim.x)) {
+    if (threadIdx.x == 0 && arrive_one(count, blocks)) {
         agent_store(count, 0u);   // for the next reply, which the stream orders behind this one
         system_store(flag, seq);
     }
+}
+__global__ __launch_bounds__(kThreads) void k_reply(const uint64_t* src, uint64_t* dst, int words,
+                                                    uint32_t* count, uint32_t* flag,
+                                                    uint32_t seq) {
+    reply_words(src, dst, words, gridDim.x, count, flag, seq);
+}
+// Outputs with others between them: row y of the grid takes the output
+// (order >> 4 y) & 15 after src, outputs `stride` words apart.  (Its arguments cost
+// a reply of one span 0.2 us.)
+__global__ __launch_bounds__(kThreads) void k_reply_rows(const uint64_t* src, uint64_t* dst,
+                                                         int words, int stride, uint32_t order,
+                                                         uint32_t* count, uint32_t* flag,
+                                                         uint32_t seq) {
+    reply_words(src + (int64_t)((order >> (4 * blockIdx.y)) & 15u) * stride,
+                dst + (int64_t)blockIdx.y * words, words, gridDim.x * gridDim.y, count, flag, seq);
 }
 
 __global__ void k_zero_word(uint32_t* p) { *p = 0; }
@@ -500,18 +523,22 @@ struct HipExec {
         return a.type == hipMemoryTypeHost || a.type == hipMemoryTypeUnregistered;
     }
 
-    // Copies k arrays of `bytes` bytes from the arena (src[j], ascending) to
-    // dst[j]: through a reply's pinned memory when one is free and the span
-    // from the first to the last fits it, else by the runtime's copies.
+    // Bytes from one output of a Greeks request to the next.
+    static size_t output_stride(size_t bytes) {
+        return serve::output_bytes((int64_t)(bytes / 4), serve::kPrice);
+    }
+
+    // Copies k of a request's outputs, of `bytes` bytes each, from the arena
+    // (src[j], ascending) to dst[j]: through a reply's pinned memory when one is
+    // free and they fit it, else by the runtime's copies.
     hipError_t copy_out(void* const* dst, char* const* src, int k, size_t bytes) {
-        const size_t span = k > 0 ? (size_t)(src[k - 1] - src[0]) + bytes : 0;
         bool host = k > 0;
         for (int j = 0; j < k; ++j) host = host && host_memory(dst[j]);
-        if (host && span <= kReplyBytes) {
+        if (host && k * output_stride(bytes) <= kReplyBytes) {
             for (int r = 0; r < kReplies; ++r) {
                 std::unique_lock<std::mutex> lk(reply[r].mu, std::try_to_lock);
                 if (!lk.owns_lock()) continue;
-                return reply_out(r, dst, src, k, bytes, span);
+                return reply_out(r, dst, src, k, bytes);
             }
         }
         hipError_t e = hipSuccess;
@@ -520,17 +547,29 @@ struct HipExec {
         return e;
     }
 
-    hipError_t reply_out(int r, void* const* dst, char* const* src, int k, size_t bytes,
-                         size_t span) {
+    hipError_t reply_out(int r, void* const* dst, char* const* src, int k, size_t bytes) {
         uint8_t* host = reply_host + r * kReplySpan;
         uint8_t* dev = reply_dev + r * kReplySpan;
-        const int words = (int)((span + 7) / 8);   // outputs are padded to 256 bytes
+        const size_t stride = output_stride(bytes);
+        const bool joined = (size_t)(src[k - 1] - src[0]) == (size_t)(k - 1) * stride;
+        const size_t apart = joined ? stride : (bytes + 7) / 8 * 8;   // in the reply
+        const int words = (int)(((joined ? (k - 1) * stride : 0) + bytes + 7) / 8);
+        const uint64_t* from = reinterpret_cast<const uint64_t*>(src[0]);
+        uint64_t* to = reinterpret_cast<uint64_t*>(dev);
+        uint32_t* count = reply_count + r * 64;
+        uint32_t* dev_flag = reinterpret_cast<uint32_t*>(dev + kReplyBytes);
         const uint32_t seq = ++reply[r].seq;
-        hipLaunchKernelGGL(k_reply, dim3(std::min((words + kThreads - 1) / kThreads, kReplyBlocks)),
-                           dim3(kThreads), 0, reply[r].stream,
-                           reinterpret_cast<const uint64_t*>(src[0]),
-                           reinterpret_cast<uint64_t*>(dev), words, reply_count + r * 64,
-                           reinterpret_cast<uint32_t*>(dev + kReplyBytes), seq);
+        const int blocks = (words + kThreads - 1) / kThreads;
+        if (joined) {
+            hipLaunchKernelGGL(k_reply, dim3(std::min(blocks, kReplyBlocks)), dim3(kThreads), 0,
+                               reply[r].stream, from, to, words, count, dev_flag, seq);
+        } else {
+            uint32_t order = 0;
+            for (int j = 0; j < k; ++j) order |= (uint32_t)((src[j] - src[0]) / stride) << (4 * j);
+            hipLaunchKernelGGL(k_reply_rows, dim3(std::min(blocks, kReplyBlocks / k), k),
+                               dim3(kThreads), 0, reply[r].stream, from, to, words,
+                               (int)(stride / 8), order, count, dev_flag, seq);
+        }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         const uint32_t* flag = reinterpret_cast<const uint32_t*>(host + kReplyBytes);
@@ -542,7 +581,7 @@ struct HipExec {
             if (e != hipSuccess) return e;
             if (!arrived()) return hipErrorUnknown;
         }
-        for (int j = 0; j < k; ++j) ::memcpy(dst[j], host + (src[j] - src[0]), bytes);
+        for (int j = 0; j < k; ++j) ::memcpy(dst[j], host + j * apart, bytes);
         return hipSuccess;
     }
 };

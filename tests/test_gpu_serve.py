@@ -404,3 +404,22 @@ def test_small_batches_behind_others(gpu):
                 assert np.array_equal(a.view(np.uint32), b), (rnd, i, kind)
             gpu.call("bs_result_release", ctx.h, t)
     ctx.destroy()
+
+
+@pytest.mark.parametrize("n", [1, 31, 64, 65, 4099, 65_536])
+def test_every_choice_of_outputs(gpu, n):
+    """All 31 choices of a Greeks request's outputs, side by side in the arena and
+    with others between them: each whole, nothing past its end, the others left."""
+    book = books.make_book(n, books.SEED_BASE + 98)
+    want = [o.download(np.uint32, n) for o in gpu.greeks(gpu.DeviceBook(book))]
+    ctx = Ctx(gpu, 64 << 20)
+    t = ctx.submit(ctx.register(book), 2)
+    assert ctx.wait(t) == 0
+    for mask in range(1, 32):
+        outs = [np.full(n + 8, 7.25, np.float32) for _ in range(5)]
+        gpu.call("bs_result_copy", ctx.h, t,
+                 *[o.ctypes.data if mask >> j & 1 else None for j, o in enumerate(outs)])
+        for j, o in enumerate(outs):
+            assert np.all(o[n:] == 7.25)
+            assert np.array_equal(o[:n].view(np.uint32), want[j]) if mask >> j & 1 else np.all(o == 7.25)
+    ctx.destroy()
