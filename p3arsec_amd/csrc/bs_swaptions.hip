@@ -86,18 +86,18 @@ struct SwGrid {
 // the same bits in every call, whatever else the call prices and however its
 // blocks are cut (`rows` is a multiple of every unit).
 //
-// A unit costs a wave 18 VALU instructions beside the 200 or more of each row of
-// paths, and no work-item has fewer rows than a unit of its call, which leaves
-// small calls with too few blocks.  Units of 2, 4 and 8 rows, us a call: 128 of the
-// driver's swaptions (3 or 6 draws) x 1M trials 940, 867, 843, 1 x 1M 41, 29.7,
-// 25.6; 128 x 524,288 500, 457, 448; 8 x 262,144 38.3, 35.4, 33.2, 1 x 262,144 23.2,
-// 20.3, 20.8; 64 x 20,000 41.4, 40.3, 41.0, 16 x 10,000 22.5, 24.0, 27.8.  With more
-// draws (24 steps, 4 factors, starts at steps 1-12) 8 x 50,000 43.2, 58.2, 89.0,
-// and 1 x 1M (start at step 8) 87.7, 87.4, 105, 16 x 1M 900, 897, 901.
+// A unit costs a wave 18 VALU instructions (two together 21) beside the 200 or
+// more of each row of paths, and no work-item has fewer rows than a unit of its
+// call, which leaves small calls with too few blocks.  Units of 2, 4 and 8 rows, us
+// a call, swaptions of the driver (3 or 6 draws): 128 x 1M trials 790, 793, 774,
+// 1 x 1M 41.6, 30.2, 25.8; 128 x 300,000 273, 274, 267; 8 x 262,144 36.3, 36.2,
+// 33.5, 1 x 262,144 23.4, 20.9, 21.2; 64 x 20,000 42.5, 42.0, 42.5, 16 x 10,000
+// 23.8, 25.2, 28.8.  With more draws (24 steps, 4 factors, starts at steps 1-12)
+// 8 x 50,000 43.2, 58.2, 89.0, and 1 x 1M (start at step 8) 87.7, 87.4, 105, 16 x 1M
+// 900, 897, 901.
 constexpr int kSwMaxUnits = 16;   // of a block
-constexpr int kSwMaxUnitRows = 8;
 constexpr int unit_rows(bool narrow, int64_t paths) {
-    return !narrow || paths < (1 << 18) ? 2 : paths < (1 << 19) ? 4 : kSwMaxUnitRows;
+    return narrow && paths >= (1 << 18) ? 8 : 2;
 }
 
 // One swaption as the step-by-step kernel reads it.  pool + off holds f0[n] (the forward
@@ -222,40 +222,72 @@ __device__ __forceinline__ bool rows_linear(const SwLin& h, int64_t first, int r
     return h.linear && r != 0 && r + span <= kM31;
 }
 
-// A wave's sums of a unit, left in LDS: the two quantities are halved into one
-// register (the lower lanes' of sumsq against the upper lanes' of sum), then
-// both fold at once within 32 lanes, 18 instructions in all.
+// A wave's sums of a unit, or of two next to one another, left in LDS: the two
+// quantities are halved into one register (the lower lanes' of sumsq against the
+// upper lanes' of sum), two units' registers into one (rows of 16 lanes against
+// rows), and all fold at once within a row; 18 instructions for one unit, 21 for
+// two.  The additions are the same ones either way.
 using UnitSums = double[kSwThreads / 64][kSwMaxUnits][2];
-__device__ __forceinline__ void wave_sums(double sum, double sumsq, double* to) {
-    double x = swap_halves_add(sum, sumsq);
-    x = half_wave_sum(x);
+__device__ __forceinline__ void wave_sums(double sum, double sumsq, double (&to)[2]) {
+    const double a = swap_halves_add(sum, sumsq);
+    const double x = row_sums(swap_rows_add(a, a));
     const int lane = threadIdx.x & 63;
-    if ((lane & 31) == 31) to[lane >> 5] = x;
+    if ((lane & 31) == 15) to[lane >> 5] = x;
+}
+__device__ __forceinline__ void wave_sums(double sum, double sumsq, double sum2, double sumsq2,
+                                          double (*to)[2]) {
+    const double x = row_sums(
+        swap_rows_add(swap_halves_add(sum, sumsq), swap_halves_add(sum2, sumsq2)));
+    const int lane = threadIdx.x & 63, row = lane >> 4;
+    if ((lane & 15) == 15) to[row & 1][row >> 1] = x;
 }
 
-// A work-item's paths, a unit at a time: paths(at, &sum, &sumsq) adds the PP
-// paths at, at + kSwThreads, ... and advances xb past them.  Units that hold a
-// zero draw are left to k_sw_paths_steps (whole: none does).  Bit u of the
+// Sums of payoff and payoff^2.
+struct SwSums {
+    double sum = 0.0, sumsq = 0.0;
+    __device__ __forceinline__ void add(double v) {
+        sum += v;
+        sumsq = __builtin_fma(v, v, sumsq);
+    }
+};
+
+// A work-item's paths, a unit at a time: paths(at, s, s') adds the PP paths at,
+// at + kSwThreads, ... and advances xb past them, the first half to s and the
+// second to s'.  PAIRS: two units of PP / 2 rows at a time.  Units that hold a
+// zero draw are left to k_sw_paths_steps (whole: none does; beside one that is
+// summed their paths are drawn all the same, and the sums dropped).  Bit u of the
 // result: unit u was summed into sums[u].
-template <int PP, class Paths>
+template <int PP, bool PAIRS, class Paths>
 __device__ __forceinline__ uint32_t over_units(const SwLin& h, const SwGrid& grid, int64_t first,
                                                bool whole, uint32_t& xb,
                                                double (*__restrict__ sums)[2], Paths&& paths) {
+    const int64_t end = min(first + kSwThreads * grid.rows, grid.paths);
+    const int unit = PAIRS ? PP / 2 : h.unit, rows = PAIRS ? PP : unit;
     uint32_t done = 0;
     int u = 0;
 #pragma unroll 1
-    for (int64_t at = first; at < first + kSwThreads * grid.rows && at < grid.paths;
-         ++u, at += kSwThreads * h.unit) {
-        if (!whole && !rows_linear(h, at, h.unit)) {
-            for (int row = 0; row < h.unit; ++row) xb = add_m31(xb, h.x_row);
+    for (int64_t at = first; at < end; at += kSwThreads * rows, u += PAIRS ? 2 : 1) {
+        uint32_t take = whole || rows_linear(h, at, unit) ? 1u : 0u;
+        if constexpr (PAIRS) {
+            const int64_t next = at + kSwThreads * unit;
+            if (next < end && (whole || rows_linear(h, next, unit))) take |= 2u;
+        }
+        if (!take) {
+            for (int row = 0; row < rows; ++row) xb = add_m31(xb, h.x_row);
             continue;
         }
-        double sum = 0.0, sumsq = 0.0;
+        const int64_t p = at + (int)threadIdx.x;
+        SwSums a;
+        if constexpr (PAIRS) {
+            SwSums b;
+            paths(p, a, b);
+            wave_sums(a.sum, a.sumsq, b.sum, b.sumsq, sums + u);
+        } else {
 #pragma unroll 1
-        for (int row = 0; row < h.unit; row += PP)
-            paths(at + row * kSwThreads + (int)threadIdx.x, &sum, &sumsq);
-        wave_sums(sum, sumsq, sums[u]);
-        done |= 1u << u;
+            for (int row = 0; row < rows; row += PP) paths(p + row * kSwThreads, a, a);
+            wave_sums(a.sum, a.sumsq, sums[u]);
+        }
+        done |= take << u;
     }
     return done;
 }
@@ -338,7 +370,7 @@ __device__ __forceinline__ void linear_batch(const SwLin& h, const double* __res
 }
 
 // The paths of a work-item, PP at a time.
-template <int W, int PP, int DB>
+template <int W, int PP, int DB, bool PAIRS>
 __device__ __forceinline__ uint32_t linear_paths(const SwLin& h, const double* __restrict__ q,
                                                  uint32_t xb, int64_t first, bool whole,
                                                  const SwGrid& grid, char* lds, uint32_t wl,
@@ -348,8 +380,8 @@ __device__ __forceinline__ uint32_t linear_paths(const SwLin& h, const double* _
     const double* __restrict__ gdf = G + h.draws * W;
     const double df0 = exp2_mid(h.c_df);
     const MoroCentral central;
-    return over_units<PP>(h, grid, first, whole, xb, sums,
-                          [&](int64_t p0, double* sum, double* sumsq) {
+    return over_units<PP, PAIRS>(h, grid, first, whole, xb, sums,
+                                 [&](int64_t p0, SwSums& low, SwSums& high) {
         double acc[PP][W], dfe[PP];
         uint32_t xs[PP];
 #pragma unroll
@@ -383,8 +415,7 @@ __device__ __forceinline__ uint32_t linear_paths(const SwLin& h, const double* _
         for (int p = 0; p < PP; ++p) {
             double v = (leg[p] > 0 ? leg[p] : 0) * df[p];
             v = p0 + p * kSwThreads < grid.paths ? v : 0.0;
-            *sum += v;
-            *sumsq = __builtin_fma(v, v, *sumsq);
+            (p < PP / 2 ? low : high).add(v);
         }
     });
 }
@@ -411,8 +442,8 @@ __device__ __forceinline__ uint32_t linear_wide(const SwLin& h, const double* __
     char* slots = lds + wave * kWideBytes;
     uint16_t* list = reinterpret_cast<uint16_t*>(slots + kWideDraws * 64 * 8);
     char* mine = slots + lane * 8;
-    return over_units<1>(h, grid, first, whole, xb, sums,
-                         [&](int64_t p0, double* sum, double* sumsq) {
+    return over_units<1, false>(h, grid, first, whole, xb, sums,
+                                [&](int64_t p0, SwSums& to, SwSums&) {
         double acc[W], dfe = h.c_df;
 #pragma unroll
         for (int c = 0; c < W; ++c) acc[c] = q[c];
@@ -461,8 +492,7 @@ __device__ __forceinline__ uint32_t linear_wide(const SwLin& h, const double* __
             if (c < h.flows) leg = __builtin_fma(pay[c], exp2_mid(acc[c]), leg);
         double v = (leg > 0 ? leg : 0) * (h.df_draws > 0 ? exp2_mid(dfe) : df0);
         v = p0 < grid.paths ? v : 0.0;
-        *sum += v;
-        *sumsq = __builtin_fma(v, v, *sumsq);
+        to.add(v);
     });
 }
 
@@ -593,10 +623,13 @@ __device__ __forceinline__ uint32_t linear_form(const SwLin& h, const double* __
     if constexpr (W <= kNarrowFlows) {
         const uint32_t wl = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / 64) *
                             (kSwBatch * 64 * 8);
-        if (h.draws <= 3 && h.unit >= 4)
-            return linear_paths<W, 4, 3>(h, q, xb, first, whole, grid, lds, wl, sums);
+        if (h.draws <= 3 && grid.rows > 2)   // 12 draws in a batch
+            return h.unit == 2
+                       ? linear_paths<W, 4, 3, true>(h, q, xb, first, whole, grid, lds, wl, sums)
+                       : linear_paths<W, 4, 3, false>(h, q, xb, first, whole, grid, lds, wl, sums);
         if (h.draws <= kSwBatch / 2)
-            return linear_paths<W, 2, kSwBatch / 2>(h, q, xb, first, whole, grid, lds, wl, sums);
+            return linear_paths<W, 2, kSwBatch / 2, false>(h, q, xb, first, whole, grid, lds, wl,
+                                                           sums);
     }
     return linear_wide<W>(h, q, xb, first, whole, grid, lds, sums);
 }
@@ -1247,17 +1280,21 @@ extern "C" int bs_swaptions_host_f64(const bs_swaption_t* sw, int64_t n, int64_t
             return set_error(BS_ERR_INVALID,
                              "more than 2^24 blocks of 1024 paths (2^34 paths) in one call");
         // Paths per work-item: enough of them to spread the 100 or so
-        // instructions of its set-up while several rounds of blocks are left
-        // (1024 are resident at once), and 2 where 4 would leave the chip
-        // idle.  Rows 2, 4 and 8: 8 swaptions x 50,000 trials (starts at
-        // steps 1-12, 4 factors; 392 blocks of 4 rows) 52, 70 and 107 us; 64 x
-        // 20,000 (1280 blocks) 51, 50, 51; 32 x 50,000 (starts at steps 1-10,
-        // 1568 blocks) 126, 126, 140.  Rows 16, 32 and 64: 128 x 1M (125,056
-        // blocks) 765, 755, 761, and 5202, 5208, 5295 with 24 steps, 4 factors
-        // and a start at step 8; 128 x 550,000 (68,864) 447, 441; rows 8, 32 and
-        // 64 at 128 x 500,000 (62,592) 430, 430, 431.
+        // instructions of its set-up and its units' sums while several rounds of
+        // blocks are left (1024 are resident at once), and 2 where 4 would leave
+        // the chip idle.  us a call with rows 2, 4, 8, 16 and 32, swaptions of the
+        // driver: 16 x 10,000 (160 blocks of 4 rows) 24.0, 25.5, 30.0, 39, 57; 64 x
+        // 20,000 (1280) 44.9, 41.9, 42.8, 49, 68; 128 x 50,000 (6272) 110, 88.7,
+        // 85.0, 86.8, 98; 128 x 131,000 (16,384) 210, 162, 150, 144.5, 148; 128 x
+        // 300,000 (37,504) -, -, 287, 275, 274; 128 x 1M (125,056) -, -, 823, 783,
+        // 774.  Of a desk with starts at steps 1-10 and 4 factors: 8 x 50,000 (392)
+        // 44.8, 60.5, 95.7, 165, 300; 32 x 50,000 (1568) 118.9, 119.1, 132, 224, 411.
         const int64_t blocks4 = bps_most * n;
-        int rows = blocks4 >= 65536 ? 32 : blocks4 >= 16384 ? 8 : blocks4 >= 1024 ? 4 : 2;
+        int rows = blocks4 >= 32768   ? 32
+                   : blocks4 >= 12288 ? 16
+                   : blocks4 >= 4096  ? 8
+                   : blocks4 >= 1024  ? 4
+                                      : 2;
         for (const SwShape& x : shapes) rows = std::max(rows, x.unit);
         const int64_t bps = (paths + kSwThreads * rows - 1) / (kSwThreads * rows);
         // the swaptions whose paths cost most first, so that the launch ends on
