@@ -329,3 +329,18 @@ def test_step_by_step_forms(gpu, F, start):
         check((p[i], e[i]), S.price_blocking(x, seed + i, 3000, 1), i)
         q, f = W.price([x], 3000, seed + i, 1)
         assert same_bits(p[i:i + 1], q) and same_bits(e[i:i + 1], f)
+
+
+@pytest.mark.parametrize("count,trials", [(128, 32_000), (128, 98_300), (128, 262_100)])
+@pytest.mark.parametrize("seed", [1979, 2147483647 - 30 * 700, 2147483647 - 30 * 256 - 29])
+def test_units_of_two_rows_in_pairs(gpu, count, trials, seed):
+    """Work-items of 8, 16 and 32 rows, whose units of 2 are folded in pairs, the
+    last pair cut by the end of the paths, against the swaption alone (4 rows or 2):
+    the same bits, also where a zero draw takes the first or the second unit of a
+    pair away."""
+    sws = W.parsec_portfolio(count)[0]
+    p, e = W.price(sws, trials, seed, 1)
+    for i in (0, 1, 2, count // 2, count - 1):
+        q, f = W.price(sws[i:i + 1], trials, seed + i, 1)
+        assert same_bits(p[i:i + 1], q) and same_bits(e[i:i + 1], f), i
+    check((p[1], e[1]), S.price_chain(sws[1], seed + 1, trials, 1), 1)
