@@ -56,6 +56,20 @@ inline bool capturing(hipStream_t st) {
     return true;
 }
 
+// While one lives, this thread may allocate although a stream is being captured:
+// in the default mode the allocation would be refused and would end every
+// capture of the global mode in the process.
+class RelaxedCapture {
+public:
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+    RelaxedCapture(const RelaxedCapture&) = delete;
+    RelaxedCapture& operator=(const RelaxedCapture&) = delete;
+
+private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 // Validates that [p, p + bytes) is memory the GPU may access.
 int check_device_range(const void* p, size_t bytes, const char* name);
 

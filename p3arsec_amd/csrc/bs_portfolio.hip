@@ -363,6 +363,7 @@ int claim_slot(PfDevice& d) {
             return -1;
         }
         if (!d.busy) {
+            const RelaxedCapture relaxed;
             uint32_t* p = nullptr;
             void* q = nullptr;
             if (hipHostMalloc(reinterpret_cast<void**>(&p), kPfSlots * 64, hipHostMallocCoherent) !=

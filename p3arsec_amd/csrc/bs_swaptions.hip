@@ -1049,6 +1049,7 @@ bool take_space(int dev, SwSpace* x) {
         return true;
     }
     if (all.made == kSwSpaces) return false;
+    const RelaxedCapture relaxed;
     void* p = nullptr;
     if (hipHostMalloc(reinterpret_cast<void**>(&x->host), kSpaceHost, hipHostMallocCoherent) !=
         hipSuccess) {
@@ -1086,6 +1087,7 @@ hipError_t pool_of(int dev, hipMemPool_t* out) {
     if (dev < 0 || dev >= kSwDevices) return hipErrorInvalidDevice;
     std::lock_guard<std::mutex> lk(mu);
     if (!pools[dev]) {
+        const RelaxedCapture relaxed;
         hipMemPoolProps props = {};
         props.allocType = hipMemAllocationTypePinned;
         props.location.type = hipMemLocationTypeDevice;

@@ -6,6 +6,9 @@ eager passes (on another output) between replays.  With the library's
 pointer checks on (the default) and off.  The HIP runtime is called directly
 (ctypes), as the caller would."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -115,3 +118,48 @@ def test_swaptions_on_a_capturing_stream_are_refused(gpu):
         st.destroy()
         out.free()
         db.free()
+
+
+FIRST_CALLS = """
+import ctypes, sys
+sys.path[:0] = {paths!r}
+import numpy as np
+from p3arsec_amd import books, capi, swaptions
+from test_gpu_capture import hip
+H, n = hip(), 5000
+db = capi.DeviceBook(books.make_book(n, books.SEED_BASE + 142))
+want = capi.price(db).download(np.uint32, n)
+out, sums, graph, gexec = capi.alloc_out(n), capi.DeviceBuffer(40), ctypes.c_void_p(), ctypes.c_void_p()
+a, b = capi.Stream(), capi.Stream()
+sws, base = swaptions.parsec_portfolio(4)
+def calls():
+    capi.call("bs_portfolio_f32", *db.ptrs(), None, n, 1, sums.ptr, b.handle)
+    return swaptions.price(sws, 2000, base, stream=b.handle)
+assert H.hipStreamBeginCapture(a.handle, 0) == 0
+capi.call("bs_price_f32", *db.ptrs(), out.ptr, n, a.handle)
+got = calls()
+assert H.hipStreamEndCapture(a.handle, ctypes.byref(graph)) == 0
+capi.call("bs_stream_sync", b.handle)
+first = sums.download(np.uint64, 5)
+assert H.hipGraphInstantiate(ctypes.byref(gexec), graph, None, None, 0) == 0
+assert H.hipGraphLaunch(gexec, a.handle) == 0
+capi.call("bs_stream_sync", a.handle)
+assert np.array_equal(out.download(np.uint32, n), want)
+again = calls()
+capi.call("bs_stream_sync", b.handle)
+assert np.array_equal(sums.download(np.uint64, 5), first)
+assert all(np.array_equal(x.view(np.uint64), y.view(np.uint64)) for x, y in zip(got, again))
+print("first calls ok")
+"""
+
+
+def test_first_calls_beside_another_streams_capture(gpu):
+    """A program's first portfolio and swaptions calls, which allocate what the
+    library keeps, while another stream is captured in the global mode: they work,
+    and the capture ends whole.  In a process of its own, where nothing is
+    allocated yet."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    r = subprocess.run([sys.executable, "-c",
+                        FIRST_CALLS.format(paths=[here, os.path.dirname(here)])],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "first calls ok" in r.stdout, r.stdout + r.stderr
