@@ -118,10 +118,16 @@ int bs_price_i32type_f32(const float *s, const float *k, const float *r, const f
  * the same output as calling bs_price_f32 (otype_bytes = 1, uint8 types) or
  * bs_price_i32type_f32 (otype_bytes = 4, int32 types) `passes` times.  Every
  * pass loads, prices and stores every option.  No pass reads another's output,
- * so one launch carries them all, with no barrier over the book between passes
- * and side by side where the book leaves the chip idle (small books are bound
- * by kernel boundaries).  Where price overlaps an input, each pass is a launch of its own, so that it reads
- * what the pass before it wrote. */
+ * so one launch carries them all and passes are not ordered: an option's passes
+ * run one after another, other options' beside them, and where the book leaves
+ * the chip idle (small books are bound by kernel boundaries) a book's passes
+ * side by side.  A book larger than the caches is therefore read from HBM about
+ * once, and the call's time divided by passes is neither the latency nor the
+ * streaming time of a pass; separate bs_price_f32 calls give those.  Of the
+ * configuration, BS_CFG_MAX_BLOCKS and BS_CFG_BLOCK_THREADS apply; vector width,
+ * non-temporal accesses, pipelining and LDS per wave are bs_price_f32's.  Where
+ * price overlaps an input, each pass is a launch of its own, as bs_price_f32's,
+ * so that it reads what the pass before it wrote. */
 int bs_price_passes_f32(const float *s, const float *k, const float *r, const float *v,
                         const float *t, const void *otype, int otype_bytes, float *price,
                         int64_t n, int passes, bs_stream_t stream);
@@ -232,11 +238,16 @@ typedef struct {
  * most 2^32 work-items), the swap's start step x n_factors <= 64; a record
  * the reference would index out of its arrays with (maturity past the
  * horizon, tenor past the curve, payment interval under one step) is
- * BS_ERR_INVALID.  A call's device buffers (about 1.5 KB per swaption, up to
- * 40 KB for one with many draws and cash flows, plus 16 bytes per 1024 paths)
- * come from a stream-ordered pool the library keeps
- * per device, which holds up to 1 GiB of freed memory for later calls until
- * the process ends.  Calls on different threads and streams are independent. */
+ * BS_ERR_INVALID.  A call takes one of up to four workspaces that the library
+ * keeps on each device until the process ends (1 MB of pinned and 16 MB of
+ * device memory each, made when first needed).  A call that finds all four in
+ * use, or whose parameters (about 1.5 KB per swaption, up to 40 KB for one with
+ * many draws and cash flows) or partial sums (16 bytes per 512 paths, per 2048
+ * of a swaption of 2^18 paths or more with up to 6 draws and 4 cash flows) do
+ * not fit, allocates from a stream-ordered pool of the library's that holds up
+ * to 1 GiB of freed memory per device.  The calling thread spins for up to 500
+ * us before it sleeps.  Calls on different threads and streams are
+ * independent. */
 int bs_swaptions_host_f64(const bs_swaption_t *sw, int64_t n, int64_t trials, int64_t seed,
                           int32_t block_size, double *price, double *std_error,
                           bs_stream_t stream);
@@ -363,10 +374,12 @@ int bs_submit_many(bs_ctx_t ctx, const bs_book_t *books, const int *kinds,
  * until released.  BS_ERR_INVALID when the context has no completion queue. */
 int bs_reap(bs_ctx_t ctx, bs_completion *out, int64_t max, int64_t timeout_us, int64_t *count);
 int bs_poll(bs_ctx_t ctx, bs_ticket_t ticket, int *state);
-/* timeout_us < 0 waits forever. */
+/* timeout_us < 0 waits forever.  Spins for up to 200 us before it sleeps, as
+ * bs_reap does. */
 int bs_wait(bs_ctx_t ctx, bs_ticket_t ticket, int64_t timeout_us);
 /* Copies a finished request's outputs to host arrays (NULL skips one; the
- * Greeks arrays only for BS_REQ_GREEKS). */
+ * Greeks arrays only for BS_REQ_GREEKS).  The calling thread spins for up to
+ * 200 us before it sleeps. */
 int bs_result_copy(bs_ctx_t ctx, bs_ticket_t ticket, float *price, float *delta,
                    float *vega, float *rho, float *theta);
 /* Device pointers of a finished request's outputs (valid until release). */

@@ -5,11 +5,12 @@
 // of VW consecutive options: one VW*4-byte load per float array, one VW-byte
 // load of the type bytes and one store per output array, so every wave64
 // instruction moves a contiguous 64*VW*4-byte span (fully coalesced).  VW is 4
-// (128-bit accesses) or 2 (64-bit): on MI355X the 2-wide form is the faster
-// one for every FP32 stream here (10M options: Greeks 71 vs 75 us, price 43
-// vs 46 us).  Groups are walked grid-stride, optionally software-pipelined
-// (the next group's loads issued before the current group's math).
-// Loads and stores are non-temporal: every byte is touched once.
+// (128-bit accesses) or 2 (64-bit): 2 for the prices, for the Greeks below 2^22
+// options, 4 from there and for CNDF.  Groups are walked grid-stride, optionally
+// software-pipelined (the next group's loads issued before the current group's
+// math).  Every byte is touched once: loads of aligned streams are non-temporal,
+// those of unaligned ones go through the caches, and stores have the policy that
+// bs_ops.hpp gives their size.
 //
 // The pricing arithmetic lives in bs_math.hpp; this file only moves data.
 #include <algorithm>
@@ -92,9 +93,7 @@ Op make_op(const CndfArgs<T>& a) { return Op{a.x, a.out}; }
 // ---- generic streaming kernels ----------------------------------------------
 // Grid-stride over the whole groups of VW options in the n from the op's arrays
 // on; the `head` options before them and the last n % VW, which do not fill a
-// group, are priced one per work-item by the first blocks.  What n and VW give
-// is no argument: a call on 4096 options takes 4.11 us, 4.17 with the group
-// count and the tail's begin handed over.  PIPE
+// group, are priced one per work-item by the first blocks.  PIPE
 // issues the loads of a work-item's next group before pricing the current one
 // (register double buffering), so a wave overlaps its own HBM latency with its
 // arithmetic; it holds one more group of registers, so its occupancy target

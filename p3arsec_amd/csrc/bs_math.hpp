@@ -310,8 +310,8 @@ __device__ __forceinline__ double log64(double x) {
 // Ref64Ordinary: Ref64's statements for ordinary inputs (Ref64::unchecked_holds),
 // with the primitives of bs_fp64.hpp, none of which has code for special values
 // and none a larger error than the general one: quotients and the square root
-// within half an ulp and 2^-19 of one, exp and log within 0.88.  |x| of CNDF is capped at 40, past
-// which e^{-x^2/2} is 0 and CNDF exactly 0 or 1.
+// within half an ulp and 2^-19 of one, exp and log within 0.88.  |x| of CNDF is
+// capped at 40, past which e^{-x^2/2} is 0 and CNDF exactly 0 or 1.
 struct Ref64Ordinary {
     using T = double;
     static constexpr bool kSplitCndf = true;
@@ -347,9 +347,9 @@ struct Ref64Ordinary {
 // with fptype = double, prices differ by a few units in the last place.
 //
 // It prices the options that are not ordinary; Ref64Ordinary does the others:
-// s, k, v and t in [2^-100, 2^100) and |r t| < 700, where no quotient, square,
-// product or exponential of the price leaves FP64's normal range except
-// CNDF's tail towards 0.
+// s, k, v and t in [2^-100, 2^100) and |r t| < 700, where no quotient, square or
+// exponential of the price leaves FP64's normal range except CNDF's tail towards
+// 0; K e^{-rT} may, and is the same product in both.
 struct Ref64 {
     using T = double;
     using Unchecked = Ref64Ordinary;
