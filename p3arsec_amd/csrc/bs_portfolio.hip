@@ -237,25 +237,28 @@ __global__ __launch_bounds__(kPfFinalThreads) void k_pf_final(const double* __re
 }
 
 // Rows per wave: one while that makes fewer than kPfSpread blocks, so that a
-// small book spreads over the chip; then up to kPfMostRows, which keeps the
-// blocks' counting in rare against their options; more only to stay within
-// kPfMaxBlocks.  With and without Greeks alike, so that the sum of prices has
-// the same bits in both.  us a call, price sums / with Greeks, for (rows, spread):
-//   1M options    (4, 1024)  8.4 / 13.1   (4, 512)  9.2 / 13.4   (8, 512)  9.2 / 13.4
-//   1.5M         10.4 / 15.1             10.5 / 15.2             11.6 / 16.5
-//   4M           19.6 / 26.7             19.2 / 26.7             20.0 / 25.7
-//   10M          40.8 / 53.2             40.9 / 52.8             41.5 / 50.7
-// and, of the Greeks form with weights, 10M 52.9, 53.6 and 54.2; price sums with
-// 16 rows 44.  In two launches the Greeks sums of 1M options take 12.2 us with a
-// spread of 512 and 13.7 with 1024.
+// small book spreads over the chip (1280 blocks of the price form are resident at
+// once); then up to kPfMostRows, which keeps the blocks' counting in rare against
+// their options; more only to stay within kPfMaxBlocks.  With and without Greeks
+// alike, so that the sum of prices has the same bits in both.  us a call, price
+// sums / with Greeks / with Greeks and weights, for (rows, spread), one stream:
+//         (4, 1024)            (6, 1536)            (6, 2048)            (8, 2048)
+//   1M     8.5 / 13.2 / 13.3    8.5 / 13.1 / 13.2    8.5 / 13.2 / 13.2    8.6 / 13.2 / 13.3
+//   1.5M  10.3 / 15.0 / 15.1   10.2 / 15.6 / 15.7   10.2 / 15.6 / 15.7   10.2 / 15.6 / 15.7
+//   2.5M  13.7 / 19.3 / 19.6   13.9 / 19.4 / 20.0   13.2 / 19.7 / 20.1   13.2 / 19.6 / 20.2
+//   4M    18.7 / 25.9 / 26.2   19.8 / 26.6 / 26.9   18.7 / 26.0 / 26.4   18.7 / 26.1 / 26.4
+//   6M    25.1 / 34.0 / 34.2   25.4 / 33.5 / 33.9   25.5 / 34.4 / 34.4   25.6 / 34.4 / 34.4
+//   10M   38.3 / 49.6 / 51.6   38.3 / 47.6 / 50.1   38.1 / 47.8 / 50.1   38.9 / 48.7 / 51.1
+// and on two streams 10M 34.8 / 45.2, 34.4 / 44.0, 34.4 / 44.0, 34.4 / 43.5; price
+// sums of 10M with weights 41.3, 41.7, 41.6, 43.2, and with 16 rows 44 without.
 //
 // The whole call, against one wave per 8 rows and one final block in two
 // launches with stream-ordered scratch: 65,537 options 5.9 us and 23.4 (the
-// host's allocation); 1M 8.5 and 25, with Greeks 13.1 and 25; 10M 39.0 and
-// 47.1, with Greeks and weights 52.9 and 61 (the final block alone 8.8).
+// host's allocation); 1M 8.5 and 25, with Greeks 13.2 and 25; 10M 38.1 and
+// 47.1, with Greeks and weights 50.1 and 61 (the final block alone 8.8).
 // Bound by HBM (price) and VALU issue (Greeks).
-constexpr int64_t kPfSpread = 1024;
-constexpr int64_t kPfMostRows = 4;
+constexpr int64_t kPfSpread = 2048;
+constexpr int64_t kPfMostRows = 6;
 
 struct PfShape {
     int64_t rows, blocks;
