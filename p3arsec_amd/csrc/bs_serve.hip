@@ -9,8 +9,8 @@
 //     memory to the device, then one fused kernel per section (the batch's
 //     price requests, its Greeks requests): a block prices one tile of 512
 //     options of one request, found by a 64-ary wave search of the table.  A
-//     batch of at most 32 requests and 2048 tiles that finds nothing in flight
-//     is one kernel with the table as its argument.
+//     batch of at most 32 requests and 2048 tiles that finds little or nothing in
+//     flight is one kernel with the table as its argument.
 //     Launched directly (the default) each section's grid is one block per
 //     tile.  With use_graph the three kernels are captured once per slot and
 //     each batch is one hipGraphLaunch; before it, each section's node gets
@@ -201,17 +201,20 @@ using ServeGreeks = GreeksF32<kVW>;
 // one grid holds the price section's tiles, then the Greeks section's.  The
 // stage kernel and a kernel per section cost 14 us of GPU time and two launches
 // for requests that price in 3: 32 requests submitted together are done in 19 us
-// and 25, one of 1M options in 21 and 25.  Only a batch that finds nothing else
-// in flight takes it.  Where others are, a batch's wait is what the dispatcher's
-// next round can be filled with: with every small batch in this form, rounds
-// came more often and smaller, and the bulk lane's tail grew.  Three forms, all
-// small batches / those with nothing in flight / none, at a Poisson rate:
-//   20,000/s   p50 20.5, 22.2, 25.5 us     300,000/s  p50 38, 49, 49 us
-//   800,000/s  p99 209, 159, 151 us (of books up to 64K options 140, 132, 124)
-//   1,200,000/s p99 235, 183, 182 us (200, 140, 138)
+// and 25, one of 1M options in 21 and 25.  Only a batch that finds nothing else in
+// flight takes it, or one of at most 4 requests that finds one other.  Where more
+// are, a batch's wait is what the dispatcher's next round can be filled with: with
+// every small batch in this form, rounds came more often and smaller, and the bulk
+// lane's tail grew.  Every small batch / by this rule / only with nothing else in
+// flight / none, at a Poisson rate, the middle of four runs in turn on one box:
+//   20,000/s     p50 20.0, 21.4, 22.4, 25.0 us
+//   200,000/s    p50 21-37, 29-42, 35-43, 33-44 us over the four
+//   800,000/s    p99 205, 152, 161, 158 us (of books up to 64K options 139, 129, 135, 128)
+//   1,200,000/s  p99 242, 178, 186, 175 us (207, 136, 140, 128)
 // Larger batches keep the three kernels (at saturation one kernel for both
 // sections, at the Greeks form's registers, ran 1.73e11 options/s against 1.76e11).
 constexpr int kSmallDesc = 32;
+constexpr int kSmallBeside = 4;   // with one other batch in flight
 constexpr int64_t kSmallTiles = 2048;
 struct SmallBatch {
     int32_t np, nd;         // price requests, all requests
@@ -442,16 +445,17 @@ struct HipExec {
     void thread_start() { (void)hipSetDevice(device); }
 
     // Launches slot s on its lane's stream (the bulk lane alternates between
-    // two): graph replay, or directly: a small batch with nothing else in flight
+    // two): graph replay, or directly: a small batch with little else in flight
     // as one kernel, any other as the stage kernel and the fused kernel of each
     // non-empty section; each section's grid is one block per tile.  Then
     // records the slot's event.
     int launch(int s, const std::vector<serve::Admitted>& reqs, std::string* err) {
-        const bool alone = std::none_of(in_flight, in_flight + kSlots, [](bool f) { return f; });
+        const int64_t others = std::count(in_flight, in_flight + kSlots, true);
         write_slot(s, reqs);
         hipStream_t st = s < kSmallSlots ? streams[2] : streams[nlaunch++ & 1];
         slot_stream[s] = st;
         const SlotHeader* h = reinterpret_cast<const SlotHeader*>(host_slot[s]);
+        const int nd = h->ndesc[0] + h->ndesc[1];
         hipError_t e = hipSuccess;
         if (graph[s]) {
             // an empty section keeps one block, which returns at once
@@ -460,11 +464,11 @@ struct HipExec {
                 e = set_section_grid(s, sec, (unsigned)blocks);
             }
             if (e == hipSuccess) e = hipGraphLaunch(graph[s], st);
-        } else if (alone && h->ndesc[0] + h->ndesc[1] <= kSmallDesc &&
+        } else if (nd <= (others == 0 ? kSmallDesc : others == 1 ? kSmallBeside : 0) &&
                    h->tiles[0] + h->tiles[1] <= std::min(kSmallTiles, grid_cap)) {
             SmallBatch b;
             b.np = h->ndesc[0];
-            b.nd = h->ndesc[0] + h->ndesc[1];
+            b.nd = nd;
             b.price_tiles = (int32_t)h->tiles[0];
             b.pad = 0;
             ::memcpy(b.d, host_slot[s] + sizeof(SlotHeader), sizeof(Desc) * (size_t)b.nd);
