@@ -636,7 +636,7 @@ __device__ __forceinline__ uint32_t linear_form(const SwLin& h, const double* __
 
 // Bound by FP64 issue (parameters and partial sums are all it reads and
 // writes): PARSEC's native run, 128 swaptions x 1M trials with 3 or 6 draws and
-// 1 to 3 cash flows, takes 0.755 ms at 195 VALU instructions per path, and
+// 1 to 3 cash flows, takes 0.776 ms at 204 VALU instructions per path, and
 // took 3.31 ms at 928 in the form that followed the forward-rate chains (a
 // 64-bit generator, 6 draws for every swaption, an exponential per curve
 // point); 32 swaptions x 50,000 trials with 4-40 draws 0.09 ms and 0.76 ms.
