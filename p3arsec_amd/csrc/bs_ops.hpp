@@ -183,11 +183,11 @@ struct PriceI32F32 {
 };
 
 // fptype = double: a group is VW = 2 options (one 128-bit load per array).
-// 10M options on one stream, 490 MB: 81.2 us (6.0 TB/s) at 180 VALU
+// 10M options on one stream, 490 MB: 82-83 us (5.9 TB/s) at 185.5 VALU
 // instructions per option and 5 waves per SIMD, where Ref64's general
-// primitives (248 instructions) took 94; with 3 waves per SIMD 82.9, not
-// pipelined 86.8, one option per work-item (8-byte stores) 84-87, the waves
-// capped by 8 KB of LDS each 84.
+// primitives (248 instructions) took 94.  At 180 instructions, 81.2 us, it took
+// 82.9 with 3 waves per SIMD, 86.8 not pipelined, 84-87 with one option per
+// work-item (8-byte stores), 84 with the waves capped by 8 KB of LDS each.
 template <int VW, bool AL = true>
 struct PriceF64 {
     static constexpr int kVW = 2;

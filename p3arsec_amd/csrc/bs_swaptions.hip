@@ -992,7 +992,7 @@ bool draws_zero(int64_t c, int64_t count) {
 // into which the last kernel writes the results, and device memory for the
 // parameters and partial sums.  Stream-ordered allocation (22 us with its
 // free), a pageable upload (14 us) and a pageable download (20 us) cost more
-// than the kernels of a small call: 64 swaptions x 20,000 trials take 49 us
+// than the kernels of a small call: 64 swaptions x 20,000 trials take 42 us
 // and took 91.
 constexpr int kSwDevices = 64;
 constexpr int kSwSpaces = 4;
@@ -1000,10 +1000,10 @@ constexpr size_t kSpaceHost = size_t(1) << 20, kSpaceDev = size_t(16) << 20;
 constexpr size_t kSpaceFlag = 64;   // the end of the pinned memory
 
 // Launches that end by themselves (SwDone) save k_sw_final and the stream's
-// synchronisation, 4 us a call (1 x 1000 trials 22.9 and 18.5 us, 32 x 50,000
-// 117.6 and 113.5, 6272 blocks 394.6 and 392.5), but every block then waits for
-// its partial's acknowledgement, which over many rounds costs as much (128 x 1M,
-// 31,360 blocks, 763 and 767 us).
+// synchronisation, 4 to 6 us a call (1 x 1000 trials 23.3 and 17.7 us, 32 x 50,000
+// 125 and 119, 128 x 300,000, 4736 blocks, 272 and 268), but every block then
+// waits for its partials' acknowledgement, which over many rounds costs as much
+// (128 x 550,000, 8704 blocks, 453 and 448 us, 128 x 1M, 15,744 blocks, 775 both).
 constexpr size_t kSwSelfMax = 512;
 constexpr int64_t kSwSelfBlocks = 8192;
 
