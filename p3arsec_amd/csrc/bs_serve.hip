@@ -206,7 +206,7 @@ using ServeGreeks = GreeksF32<kVW>;
 // are, a batch's wait is what the dispatcher's next round can be filled with: with
 // every small batch in this form, rounds came more often and smaller, and the bulk
 // lane's tail grew.  Every small batch / by this rule / only with nothing else in
-// flight / none, at a Poisson rate, the middle of four runs in turn on one box:
+// flight / none, at a Poisson rate, the middle of four runs in turn:
 //   20,000/s     p50 20.0, 21.4, 22.4, 25.0 us
 //   200,000/s    p50 21-37, 29-42, 35-43, 33-44 us over the four
 //   800,000/s    p99 205, 152, 161, 158 us (of books up to 64K options 139, 129, 135, 128)
