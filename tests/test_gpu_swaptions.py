@@ -285,8 +285,8 @@ def desk(count):
 
 
 @pytest.mark.parametrize("sws,trials", [
-    # work-items of 2, 4, 8 and 32 rows in the whole call (8 to 125,056 blocks of
-    # 1024 paths), fewer in its parts; units of 2, 4 and 8 rows
+    # work-items of 2 to 32 rows in the whole call (8 to 125,056 blocks of 1024
+    # paths), fewer in its parts; units of 2 and 8 rows
     (lambda: W.parsec_portfolio(600)[0], 600), (lambda: W.parsec_portfolio(70)[0], 16_385),
     (lambda: W.parsec_portfolio(65)[0], 262_145), (lambda: W.parsec_portfolio(128)[0], 524_288),
     (lambda: W.parsec_portfolio(128)[0], 1_000_000), (lambda: desk(40), 30_001),
